@@ -18,6 +18,11 @@
  * owned by the library.  Calls that overlap on one device -- on two streams,
  * or from two host threads -- share it and race: serialise them.
  *
+ * Large query batches are partitioned through workspaces of the library's own
+ * (at most two per device, each at most 16 bytes a query of 2^27 and tables);
+ * queries may overlap with other queries on any stream or host thread.  A
+ * query enqueued on a stream that is being captured uses none.
+ *
  * Query answers are always uint64: the slot of the query key in the layout,
  * or n when the key is absent (the reference's own miss value,
  * cpu/src/query-bst.h:42, cpu/src/query-btree.h:53).

@@ -56,6 +56,24 @@ uint64_t emu_ballot(bool p) {
     const int w = t_lane / 64;
     return g_wave[w].arrive(p ? (1ull << (t_lane % 64)) : 0ull);
 }
+// every lane of a wave posts its value, then reads the lane d below it
+static int g_shfl[1024];
+int emu_shfl_up(int v, unsigned d) {
+    const unsigned l = (unsigned)t_lane % 64;
+    g_shfl[t_lane] = v;
+    emu_ballot(true);
+    const int r = l >= d ? g_shfl[t_lane - d] : v;
+    emu_ballot(true);
+    return r;
+}
+// every lane of the wave calls it
+int emu_readlane(int v, int lane) {
+    g_shfl[t_lane] = v;
+    emu_ballot(true);
+    const int r = g_shfl[t_lane / 64 * 64 + lane];
+    emu_ballot(true);
+    return r;
+}
 void emu_sleep() { std::this_thread::yield(); }
 uint64_t emu_clock() {
     return (uint64_t)std::chrono::duration_cast<std::chrono::nanoseconds>(

@@ -39,6 +39,8 @@ tl_status check_err_flag(Ctx *c, hipStream_t) {
     if (*c->err_flag) { *c->err_flag = 0; return TL_ETIMEOUT; }
     return TL_OK;
 }
+Lease *lease_take(Ctx *, size_t, hipStream_t) { return nullptr; }
+void lease_give(Lease *, hipStream_t) {}
 tl_status Timer::start(hipStream_t, float *m) { ms = m; return TL_OK; }
 tl_status Timer::stop() { if (ms) *ms = 0; return TL_OK; }
 Timer::~Timer() {}
@@ -72,7 +74,18 @@ tl_status tl_permute_mveb(void *, uint64_t, tl_dtype, void *, float *) NOTEXP(tl
 }
 
 #include "src/tl_queue.hpp"
+#include "src/tl_tile.hpp"
 namespace tl {
+#ifndef EMU_WITH_TILE   // the emulated tl_tile.hip defines these itself
+bool part_wanted(const TileArray &, uint32_t, const void *, uint64_t, const uint64_t *, double) {
+    return false;
+}
+uint64_t part_bytes(const TileArray &, uint32_t, uint64_t) { return 0; }
+Workspace &query_workspace() {
+    static Workspace w;
+    return w;
+}
+#endif
 // the emulated persistent launch never uses the query queues
 bool queue_takes(const tl_batch_item &) { return false; }
 QueueItem queue_item(const tl_batch_item &, uint64_t, uint64_t, uint64_t, uint32_t, uint32_t,

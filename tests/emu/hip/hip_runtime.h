@@ -37,6 +37,10 @@ unsigned char *emu_smem();
 #define __syncthreads() emu_syncthreads()
 #define __ballot(p) emu_ballot((p))
 #define __any(p) (emu_ballot((p)) != 0)
+int emu_shfl_up(int v, unsigned d);
+int emu_readlane(int v, int lane);
+#define __builtin_amdgcn_readlane(v, l) emu_readlane((v), (l))
+#define __shfl_up(v, d) emu_shfl_up((v), (d))
 #define __builtin_amdgcn_s_sleep(n) emu_sleep()
 #define __builtin_amdgcn_fence(o, s) __atomic_thread_fence(__ATOMIC_SEQ_CST)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)

@@ -27,6 +27,7 @@
 #include "tl_kernels.hpp"
 #include "tl_plan.hpp"
 #include "tl_queue.hpp"
+#include "tl_tile.hpp"
 
 namespace tl {
 
@@ -556,6 +557,9 @@ struct Batch {
     size_t q_ticket_at = 0;
     uint64_t q_chunk = 4096;       // queries per queue ticket
     void *d_queue = nullptr;
+    // workspaces of the partitioned lookups, one per branch
+    void *d_qws = nullptr;
+    uint64_t qws_stride = 0;
     tl_batch_config cfg{};
     std::vector<BOp> ops;
     std::vector<BTask> tasks;
@@ -578,7 +582,7 @@ struct Batch {
         if (graph) (void)hipGraphDestroy(graph);
         for (void *p : {(void *)d_ops, (void *)d_tasks, (void *)d_blob, (void *)d_done,
                         (void *)d_ticket, (void *)d_flags, (void *)d_err, d_stash, d_pdata,
-                        d_pstash, (void *)d_pflags, d_wdata, d_wstash, (void *)d_wctr, d_queue})
+                        d_pstash, (void *)d_pflags, d_wdata, d_wstash, (void *)d_wctr, d_queue, d_qws})
             if (p) (void)hipFree(p);
         for (int k = 0; k < NSUB; k++)
             if (sub[k]) (void)hipStreamDestroy(sub[k]);
@@ -858,6 +862,24 @@ static tl_status build_queues(Batch &B) {
     return TL_OK;
 }
 
+// item a as its lookups see it (its table set is uploaded)
+static TileArray tile_array(const Batch &B, uint32_t a) {
+    const tl_batch_item &it = B.items[a];
+    TileArray t{it.A, it.n, TILE_BST, it.b, nullptr, nullptr, nullptr, 0, 0, false};
+    if (it.layout == 1) t.layout = TILE_BTREE;
+    if (it.layout == 2) {
+        const unsigned char *base = (const unsigned char *)B.d_pdata;
+        const QTables &q = B.qt[a];
+        t.layout = TILE_VEB;
+        t.tables = (const tl_veb_table *)(base + q.tables_at);
+        t.idx = (const uint64_t *)(base + q.idx_at);
+        t.tidx = (const uint32_t *)(base + q.tidx_at);
+        t.table_size = q.tsize;
+        t.ntables = q.nt;
+    }
+    return t;
+}
+
 static tl_status build_planned(Batch &B, Ctx *c) {
     Tuning tu = tuning_for(c);
 
@@ -943,6 +965,19 @@ static tl_status build_planned(Batch &B, Ctx *c) {
     TL_HIP(hipMalloc(&B.d_pstash, B.stash_stride * Batch::NSUB));
     TL_HIP(hipMalloc((void **)&B.d_pflags, flag_bytes));
     TL_TRY(build_queues(B));
+    // workspaces for the arrays whose lookups are worth partitioning; short of
+    // memory, the batch does without
+    for (uint32_t a = 0; a < B.items.size(); a++) {
+        const tl_batch_item &it = B.items[a];
+        const TileArray ta = tile_array(B, a);
+        if (it.nq && part_wanted(ta, it.dtype, it.Q, it.nq, it.ans, 1.0))
+            B.qws_stride = std::max(B.qws_stride, part_bytes(ta, it.dtype, it.nq));
+    }
+    B.qws_stride = (B.qws_stride + 255) & ~255ull;
+    if (B.qws_stride && hipMalloc(&B.d_qws, B.qws_stride * Batch::NSUB) != hipSuccess) {
+        (void)hipGetLastError();
+        B.d_qws = nullptr;
+    }
     for (int k = 0; k < Batch::NSUB; k++)
         TL_HIP(hipStreamCreateWithFlags(&B.sub[k], hipStreamNonBlocking));
     for (int f = 0; f < 2; f++) {
@@ -1314,6 +1349,19 @@ struct QueryShape {
     }
 };
 
+// the lookups enqueued on branch k use its workspace
+struct BranchWorkspace {
+    Workspace before;
+    BranchWorkspace(const Batch &B, int k) : before(query_workspace()) {
+        static char none;   // too small for any batch: no workspace of the library's
+        Workspace w;
+        w.mem = B.d_qws ? (char *)B.d_qws + k * B.qws_stride : (void *)&none;
+        w.bytes = B.d_qws ? B.qws_stride : 0;
+        query_workspace() = w;
+    }
+    ~BranchWorkspace() { query_workspace() = before; }
+};
+
 static tl_status run_queries(Batch &B, const unsigned char *base, hipStream_t s) {
     QueryShape shape(B.cfg);
     TL_TRY(fork_branches(B, 1, s));
@@ -1336,6 +1384,7 @@ static tl_status run_queries(Batch &B, const unsigned char *base, hipStream_t s)
         const tl_batch_item &it = B.items[a];
         if (!it.nq || (queues && B.queued[a])) continue;
         hipStream_t q_s = B.sub[B.query_branch[a]];
+        const BranchWorkspace ws(B, B.query_branch[a]);
         if (it.layout == 0) {
             TL_TRY(tl_query_bst(it.A, it.n, it.dtype, it.Q, it.nq, it.ans, q_s, nullptr));
         } else if (it.layout == 1) {

@@ -46,6 +46,8 @@ void set_error(const std::string &msg);
 // ---------------------------------------------------------------------------
 // per-device context
 
+struct Lease;
+
 struct Ctx {
     int device = -1;
     int num_cus = 256;
@@ -75,6 +77,24 @@ tl_status scratch(Ctx *c, int slot, size_t bytes, void **out);
 tl_status copy_to_device(Ctx *c, int slot, const void *host, size_t bytes, hipStream_t s,
                          void **dev_out);
 tl_status check_err_flag(Ctx *c, hipStream_t s);
+
+// Workspaces of the partitioned lookups, LEASES per device.  A lease is one
+// call's from lease_take() to lease_give(); work enqueued after lease_take()
+// on its stream runs after the workspace's earlier users on any stream, so
+// calls on several streams and host threads are safe.  Null when every
+// workspace is another thread's at the moment, when the stream is being
+// captured (a graph may not keep library memory) or when memory is short: the
+// caller then does without.
+constexpr int LEASES = 2;
+struct Lease {
+    void *mem = nullptr;
+    size_t bytes = 0;
+    hipEvent_t done = nullptr;   // the last user's work
+    hipStream_t last = nullptr;
+    bool taken = false;
+};
+Lease *lease_take(Ctx *c, size_t bytes, hipStream_t s);
+void lease_give(Lease *l, hipStream_t s);
 
 struct Timer {
     hipEvent_t a = nullptr, b = nullptr;

@@ -11,6 +11,7 @@
 #include "tl_internal.hpp"
 #include "tl_descent.hpp"
 #include "tl_queue.hpp"
+#include "tl_tile.hpp"
 
 namespace tl {
 
@@ -897,6 +898,10 @@ extern "C" tl_status tl_query_bst(const void *dev_A, uint64_t n, tl_dtype dtype,
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
+    const TileArray ta{dev_A, n, TILE_BST, 1, nullptr, nullptr, nullptr, 0, 0, false};
+    bool taken;
+    TL_TRY(large_query(c, ta, dtype, dev_q, nq, dev_ans, s, &taken));
+    if (taken) return tm.stop();
     TL_DISPATCH(dtype, launch_bst, c, dev_A, n, dev_q, nq, dev_ans, s);
     TL_LAUNCH_CHECK();
     return tm.stop();
@@ -912,6 +917,10 @@ extern "C" tl_status tl_query_binary(const void *dev_A, uint64_t n, tl_dtype dty
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
+    const TileArray ta{dev_A, n, TILE_SORTED, 1, nullptr, nullptr, nullptr, 0, 0, false};
+    bool taken;
+    TL_TRY(large_query(c, ta, dtype, dev_q, nq, dev_ans, s, &taken));
+    if (taken) return tm.stop();
     TL_DISPATCH(dtype, launch_binary, c, dev_A, n, dev_q, nq, dev_ans, s);
     TL_LAUNCH_CHECK();
     return tm.stop();
@@ -931,14 +940,18 @@ extern "C" tl_status tl_query_btree(const void *dev_A, uint64_t n, uint64_t b, t
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
+    const TileArray ta{dev_A, n, TILE_BTREE, b, nullptr, nullptr, nullptr, 0, 0, false};
+    bool taken;
+    TL_TRY(large_query(c, ta, dtype, dev_q, nq, dev_ans, s, &taken));
+    if (taken) return tm.stop();
     TL_DISPATCH(dtype, launch_btree, c, dev_A, n, b, dev_q, nq, dev_ans, s);
     TL_LAUNCH_CHECK();
     return tm.stop();
 }
 
-extern "C" tl_status tl_query_mveb(const void *dev_A, const tl_veb_table *dev_table, uint64_t n,
-                                   uint32_t d, tl_dtype dtype, const void *dev_q, uint64_t nq,
-                                   uint64_t *dev_ans, void *stream, float *ms) {
+static tl_status query_perfect(const void *dev_A, const tl_veb_table *dev_table, uint64_t n,
+                               uint32_t d, tl_dtype dtype, const void *dev_q, uint64_t nq,
+                               uint64_t *dev_ans, void *stream, float *ms, bool classic) {
     TL_TRY(qcheck(dev_A, n, dev_q, nq, dev_ans));
     if (nq == 0) return TL_OK;
     if (n == 0 || d == 0 || d > 63 || !dev_table || n > (1ull << d) - 1) {
@@ -950,10 +963,20 @@ extern "C" tl_status tl_query_mveb(const void *dev_A, const tl_veb_table *dev_ta
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
+    const TileArray ta{dev_A, n, TILE_VEB, 1, dev_table, nullptr, nullptr, d, 1, classic};
+    bool taken;
+    TL_TRY(large_query(c, ta, dtype, dev_q, nq, dev_ans, s, &taken));
+    if (taken) return tm.stop();
     TL_DISPATCH(dtype, launch_mveb, c, dev_A, n, dev_table, d, (const uint64_t *)nullptr,
                 (const uint32_t *)nullptr, 1u, dev_q, nq, dev_ans, s);
     TL_LAUNCH_CHECK();
     return tm.stop();
+}
+
+extern "C" tl_status tl_query_mveb(const void *dev_A, const tl_veb_table *dev_table, uint64_t n,
+                                   uint32_t d, tl_dtype dtype, const void *dev_q, uint64_t nq,
+                                   uint64_t *dev_ans, void *stream, float *ms) {
+    return query_perfect(dev_A, dev_table, n, d, dtype, dev_q, nq, dev_ans, stream, ms, false);
 }
 
 static tl_status query_nonperfect(const void *dev_A, const tl_veb_table *dev_tables,
@@ -976,6 +999,11 @@ static tl_status query_nonperfect(const void *dev_A, const tl_veb_table *dev_tab
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
+    const TileArray ta{dev_A,         n,          TILE_VEB,   1,      dev_tables, dev_idx,
+                       dev_table_idx, table_size, num_tables, classic};
+    bool taken;
+    TL_TRY(large_query(c, ta, dtype, dev_q, nq, dev_ans, s, &taken));
+    if (taken) return tm.stop();
     TL_DISPATCH(dtype, launch_mveb, c, dev_A, n, dev_tables, table_size, dev_idx, dev_table_idx,
                 num_tables, dev_q, nq, dev_ans, s);
     TL_LAUNCH_CHECK();
@@ -996,7 +1024,7 @@ extern "C" tl_status tl_query_veb(const void *dev_A, const tl_veb_table *dev_tab
                                   uint32_t d, tl_dtype dtype, const void *dev_q, uint64_t nq,
                                   uint64_t *dev_ans, void *stream, float *ms) {
     // the search of a perfect tree depends only on its table (classic rule)
-    return tl_query_mveb(dev_A, dev_table, n, d, dtype, dev_q, nq, dev_ans, stream, ms);
+    return query_perfect(dev_A, dev_table, n, d, dtype, dev_q, nq, dev_ans, stream, ms, true);
 }
 
 extern "C" tl_status tl_query_veb_nonperfect(const void *dev_A, const tl_veb_table *dev_tables,

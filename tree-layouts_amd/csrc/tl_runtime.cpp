@@ -107,6 +107,58 @@ tl_status check_err_flag(Ctx *c, hipStream_t s) {
     return TL_OK;
 }
 
+static std::mutex g_lease_mu;
+static Lease g_lease[64][LEASES];
+
+Lease *lease_take(Ctx *c, size_t bytes, hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    // another thread's capture must not see the calls below
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    std::lock_guard<std::mutex> lk(g_lease_mu);
+    Lease *best = nullptr;
+    for (Lease &l : g_lease[c->device])   // this stream's own first, then a large one
+        if (!l.taken && (!best || (l.mem && l.last == s && best->last != s) ||
+                         (best->last != s && l.bytes > best->bytes)))
+            best = &l;
+    bool ok = best != nullptr;
+    if (ok && !best->done)
+        ok = hipEventCreateWithFlags(&best->done, hipEventDisableTiming) == hipSuccess;
+    if (ok && best->bytes < bytes) {
+        if (best->mem) {
+            ok = hipEventSynchronize(best->done) == hipSuccess && hipFree(best->mem) == hipSuccess;
+            best->mem = nullptr;
+            best->bytes = 0;
+        }
+        if (ok && hipMalloc(&best->mem, bytes) != hipSuccess) {
+            best->mem = nullptr;
+            ok = false;
+        }
+        if (ok) best->bytes = bytes;
+    } else if (ok) {
+        ok = hipStreamWaitEvent(s, best->done, 0) == hipSuccess;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    best->taken = true;
+    best->last = s;
+    return best;
+}
+
+void lease_give(Lease *l, hipStream_t s) {
+    const bool ok = hipEventRecord(l->done, s) == hipSuccess;
+    if (!ok) (void)hipStreamSynchronize(s);   // nothing pending then
+    std::lock_guard<std::mutex> lk(g_lease_mu);
+    l->taken = false;
+}
+
 tl_status Timer::start(hipStream_t s_, float *ms_) {
     s = s_;
     ms = ms_;

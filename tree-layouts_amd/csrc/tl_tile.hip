@@ -1,0 +1,1480 @@
+// tl_tile.hip -- lookups of large query batches, for gfx950.
+//
+// One lane per query, a tile of queries per workgroup.  What bounds such a
+// descent is not the bytes: every load of an unsorted wave touches 64
+// different cache lines, which the vector cache takes one a clock, and every
+// step costs its vector instructions.  So a workgroup first puts its tile in
+// approximate key order (1024 buckets split at equal ranks of the array, one
+// counting sort in LDS), after which the lanes of a wave walk neighbouring
+// paths: their loads fall into few lines on all but the last levels.  The
+// descents then run level by level in lock step, with 32-bit positions and
+// nothing per lane but the compare, the step and the hit.
+//
+// The path taken through the layout, and so the answer, is the one of the
+// one-array kernels in tl_query.hip for every query: the first key equal to q
+// on the descent, also where keys repeat.
+//
+// Arrays well past the caches are served by the partitioned form below: there
+// every unsorted descent waits for lines from memory, however its tile is
+// ordered.  Measured (queries of keys that are there, before -> now):
+//   BST 2^20 4-byte keys, 2^20 queries          41 -> 28 us (tile)
+//   B-tree b=16, 2^30 8-byte keys, 2^27         10.5 -> 5.35 ms (partition)
+//   BST, the same                               28.5 -> 5.3 ms (partition)
+//   mvEB 3*10^8 8-byte keys, 2^26, Zipf(1.1)    5.58 -> 3.30 ms (partition)
+#include <math.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "tl_descent.hpp"
+#include "tl_internal.hpp"
+#include "tl_tile.hpp"
+
+namespace tl {
+
+constexpr uint32_t TILE_BINS = 1024;
+constexpr uint32_t TILE_TABLES = 256;   // vEB table entries kept in LDS
+
+constexpr uint32_t RANGE_KEYS = 4096;   // keys of a range, at most (partitioned lookups)
+
+// an incomplete vEB tree: top and bottom levels, full bottom trees, keys of the
+// incomplete one
+constexpr uint32_t VEB_CHAIN = 8;
+struct VebLevel {
+    uint32_t rd, ld, nf, inc;
+};
+
+struct TileShape {
+    uint32_t n;
+    uint32_t b, nodes;      // TILE_BTREE
+    uint32_t levels;        // full levels: of the binary tree, or of nodes
+    uint32_t table_size, ntables;
+    const tl_veb_table *tables;
+    const uint64_t *idx;
+    const uint32_t *tidx;
+    uint32_t classic;
+    // rank -> slot of a BST or B-tree (BtreeShape's); 2^64 / (b + 1) rounded up
+    uint32_t nint, span, rem, nsep, depth;
+    uint64_t recip;
+    uint32_t small_mul, small_shift;   // x / (b + 1) = x * mul >> shift, x < 2 RANGE_KEYS
+    // rank -> slot of a vEB: the incomplete trees from the whole one down (the
+    // incomplete bottom tree of one is the next), then a perfect tree of
+    // chain_d levels (0: none); split[d]: top levels of a perfect tree of d
+    VebLevel chain[VEB_CHAIN];
+    uint32_t nchain, chain_d;
+    uint8_t split[36];
+};
+
+struct VebEntry {
+    uint32_t L, R, D;
+};
+
+// What tile_slot() looks up in LDS.  TILE_BTREE: level[z].  TILE_VEB: the
+// slots of the perfect trees of at most 8 levels, tree d's rank x at
+// small[2^d + x]: a rank of a tree of 2^16 keys takes one split and one
+// look-up instead of up to four splits.
+constexpr uint32_t SMALL_LEVELS = 8;
+template <int LAYOUT>
+struct SlotMap {
+    uint32_t level[32];
+};
+template <>
+struct SlotMap<TILE_VEB> {
+    uint8_t small[2u << SMALL_LEVELS];
+};
+
+// slot of rank x in the vEB (mveb_pos32 with the tables)
+__device__ inline uint32_t veb_slot(uint32_t x, const TileShape &s, const SlotMap<TILE_VEB> &m) {
+    uint32_t base = 0, d = s.chain_d;
+    for (uint32_t j = 0; j < s.nchain; j++) {
+        const VebLevel e = s.chain[j];
+        const uint32_t r = (1u << e.rd) - 1, l = (1u << e.ld) - 1, span = e.nf << e.ld;
+        if (x < span) {
+            const uint32_t k = x >> e.ld, c = x & l;
+            d = c == l ? e.rd : e.ld;
+            base += c == l ? 0u : r + k * l;
+            x = c == l ? k : c;
+            break;
+        }
+        if (x >= span + e.inc) {
+            x = e.nf + (x - span - e.inc);
+            d = e.rd;
+            break;
+        }
+        base += r + e.nf * l;
+        x -= span;
+    }
+    while (d > SMALL_LEVELS) {
+        const uint32_t rd = s.split[d], ld = d - rd, l = (1u << ld) - 1;
+        const uint32_t k = x >> ld, c = x & l;
+        base += c == l ? 0u : (1u << rd) - 1 + k * l;
+        d = c == l ? rd : ld;
+        x = c == l ? k : c;
+    }
+    return base + m.small[(1u << d) + x];
+}
+
+// slot of rank x in the layout; m.level[z]: first slot of the level whose keys'
+// internal ranks + 1 are divisible by (b + 1)^z and no more (TILE_BTREE)
+template <int LAYOUT>
+__device__ inline uint32_t tile_slot(uint32_t x, const TileShape &s, const SlotMap<LAYOUT> &m) {
+    if constexpr (LAYOUT == TILE_SORTED) {
+        return x;
+    } else if constexpr (LAYOUT == TILE_VEB) {
+        return veb_slot(x, s, m);
+    } else if constexpr (LAYOUT == TILE_BST) {
+        if (x < s.span) {
+            if (!(x & 1)) return s.nint + (x >> 1);
+            x >>= 1;
+        } else {
+            x -= s.nsep;
+        }
+        const uint32_t y = x + 1, z = (uint32_t)__clz((int)__brev(y));
+        return ((y | (1u << s.depth)) >> (z + 1)) - 1;
+    } else {
+        auto div = [&](uint32_t v) { return (uint32_t)__umul64hi(v, s.recip); };
+        const uint32_t k1 = s.b + 1;
+        if (x < s.span) {
+            const uint32_t row = div(x);
+            if (x - row * k1 < s.b) return s.nint + x - row;
+            x = row;
+        } else if (x < s.span + s.rem) {
+            return s.nint + x - s.nsep;
+        } else {
+            x -= s.span + s.rem - s.nsep;
+        }
+        uint32_t r = x + 1, z = 0, q = div(r);
+        while (r == q * k1) {
+            r = q;
+            q = div(r);
+            z++;
+        }
+        return m.level[z] + r - q - 1;
+    }
+}
+
+// fills the map (a workgroup of at least 64 lanes), ends with a barrier
+template <int LAYOUT>
+__device__ inline void slot_map(const TileShape &s, SlotMap<LAYOUT> &m) {
+    const uint32_t tid = threadIdx.x;
+    if constexpr (LAYOUT == TILE_BTREE) {
+        if (tid < s.depth) m.level[tid] = (uint32_t)(ipow64(s.b + 1, s.depth - 1 - tid) - 1);
+    }
+    if constexpr (LAYOUT == TILE_VEB) {
+        for (uint32_t i = tid + 2; i < (2u << SMALL_LEVELS); i += blockDim.x) {
+            const uint32_t d = 31u - (uint32_t)__clz((int)i), x = i - (1u << d);
+            m.small[i] = x < (1u << d) - 1
+                             ? (uint8_t)mveb_pos32(x, (1u << d) - 1, s.classic != 0)
+                             : (uint8_t)0;
+        }
+    }
+    __syncthreads();
+}
+
+// first rank of range j of 2^lg
+__device__ inline uint32_t range_first(uint32_t j, uint32_t n, uint32_t lg) {
+    return (uint32_t)(((uint64_t)j * n) >> lg);
+}
+
+// in-order place (1 .. 2^lg - 1) of node i of a complete tree of lg levels
+__device__ inline uint32_t heap_order(uint32_t i, uint32_t lg) {
+    const uint32_t t = 31u - (uint32_t)__clz((int)i);
+    return (2 * (i - (1u << t)) + 1) << (lg - 1 - t);
+}
+
+// its inverse: the node at place y of a complete tree of lg levels
+__device__ inline uint32_t heap_node(uint32_t y, uint32_t lg) {
+    return (y | (1u << lg)) >> ((uint32_t)__clz((int)__brev(y)) + 1);
+}
+
+// where place y of a range's keys lies (range_fill)
+__device__ inline uint32_t heap_at(uint32_t y, uint32_t lg) {
+    return y ? heap_node(y, lg) : 0u;
+}
+
+// ---- the descents of QN queries of a lane.  res[k]: the slot, or n.
+
+// level-order BST, 1-based node m at A[m - 1]
+template <typename K, int QN>
+__device__ inline void tile_bst(const K *__restrict__ A, const TileShape &s, const K (&q)[QN],
+                                uint32_t (&res)[QN]) {
+    uint32_t m[QN], hit[QN];
+#pragma unroll
+    for (int k = 0; k < QN; k++) {
+        m[k] = 1;
+        hit[k] = ~0u;
+    }
+    for (uint32_t t = 0; t < s.levels; t++) {
+        K v[QN];
+#pragma unroll
+        for (int k = 0; k < QN; k++) v[k] = A[m[k] - 1];
+#pragma unroll
+        for (int k = 0; k < QN; k++) {
+            // node numbers grow along the path: the smallest equal one is the first
+            if (v[k] == q[k]) hit[k] = min(hit[k], m[k]);
+            m[k] = 2 * m[k] + (q[k] > v[k] ? 1u : 0u);
+        }
+    }
+    K v[QN];
+#pragma unroll
+    for (int k = 0; k < QN; k++)
+        if (m[k] <= s.n) v[k] = A[m[k] - 1];
+#pragma unroll
+    for (int k = 0; k < QN; k++) {
+        if (m[k] <= s.n && v[k] == q[k]) hit[k] = min(hit[k], m[k]);
+        res[k] = hit[k] == ~0u ? s.n : hit[k] - 1;
+    }
+}
+
+// level-order B-tree: a branch-free lower bound in every node.  The key at
+// the lower bound is the last one compared that was not smaller, so its
+// equality needs no load of its own.
+template <typename K, int QN>
+__device__ inline void tile_btree(const K *__restrict__ A, const TileShape &s, const K (&q)[QN],
+                                  uint32_t (&res)[QN]) {
+    const uint32_t b = s.b, n = s.n;
+    uint32_t node[QN];
+#pragma unroll
+    for (int k = 0; k < QN; k++) {
+        node[k] = 0;
+        res[k] = n;
+    }
+    // the nodes of the full levels are whole; of the last level a node may
+    // be short (slots at or past n count as larger than every key) or absent
+    for (uint32_t t = 0; t <= s.levels; t++) {
+        const bool last = t == s.levels;
+        uint32_t at[QN];
+        bool eq[QN], in[QN];
+#pragma unroll
+        for (int k = 0; k < QN; k++) {
+            in[k] = !last || node[k] < s.nodes;
+            at[k] = in[k] ? node[k] * b : 0u;
+            eq[k] = false;
+        }
+        for (uint32_t len = b; len > 0;) {
+            const uint32_t half = (len + 1) >> 1;
+            K v[QN];
+#pragma unroll
+            for (int k = 0; k < QN; k++) v[k] = A[min(at[k] + half, n) - 1];
+#pragma unroll
+            for (int k = 0; k < QN; k++) {
+                const bool less = v[k] < q[k] && (!last || at[k] + half <= n);
+                const bool same = v[k] == q[k] && (!last || at[k] + half <= n);
+                eq[k] = less ? eq[k] : same;
+                at[k] += less ? half : 0u;
+            }
+            len -= half;
+        }
+#pragma unroll
+        for (int k = 0; k < QN; k++) {
+            const uint32_t js = at[k] - node[k] * b;
+            if (in[k] && eq[k] && res[k] == n) res[k] = at[k];
+            node[k] = node[k] * (b + 1) + 1 + js;
+        }
+    }
+}
+
+// vEB (tables of either split): structure after structure, every lane at the
+// same depth, so the table entries are the wave's.  The position at depth t
+// is 1 + the sum of R + (bfs & R) * L over t, D[t], D[D[t]], .. (bfs shifted
+// to that depth): no per-lane position stack.
+template <typename K, int QN>
+__device__ inline void tile_veb(const K *__restrict__ A, const TileShape &s, const VebEntry *tb,
+                                const uint32_t *s_end, const uint32_t *s_tidx, const K (&q)[QN],
+                                uint32_t (&res)[QN]) {
+    const uint32_t n = s.n;
+    bool pend[QN];
+#pragma unroll
+    for (int k = 0; k < QN; k++) {
+        pend[k] = true;
+        res[k] = n;
+    }
+    uint32_t off = 0;
+    for (uint32_t j = 0; j < s.ntables; j++) {
+        const uint32_t end = s_end[j];
+        if (off >= end) continue;
+        const uint32_t d = 32u - (uint32_t)__clz((int)(n - off));
+        const VebEntry *e = tb + s_tidx[j];
+        bool act[QN], any = false;
+        uint32_t bfs[QN], at[QN];
+#pragma unroll
+        for (int k = 0; k < QN; k++) {
+            act[k] = pend[k];
+            pend[k] = false;
+            any |= act[k];
+            bfs[k] = 1;
+            at[k] = off;
+        }
+        if (!__any(any)) break;
+        for (uint32_t t = 1;; t++) {
+            K v[QN];
+#pragma unroll
+            for (int k = 0; k < QN; k++)
+                if (act[k]) v[k] = A[at[k]];
+#pragma unroll
+            for (int k = 0; k < QN; k++) {
+                if (act[k] && v[k] == q[k]) {
+                    res[k] = at[k];
+                    act[k] = false;
+                }
+                bfs[k] = 2 * bfs[k] + (act[k] && q[k] > v[k] ? 1u : 0u);
+                at[k] = off;
+            }
+            if (t >= d) break;
+            for (uint32_t x = t; x != 0;) {
+                const uint32_t L = e[x].L, R = e[x].R, D = e[x].D;
+#pragma unroll
+                for (int k = 0; k < QN; k++) at[k] += R + ((bfs[k] >> (t - x)) & R) * L;
+                x = D < x ? D : 0u;
+            }
+            any = false;
+#pragma unroll
+            for (int k = 0; k < QN; k++) {
+                if (act[k] && at[k] >= end) {   // in a later structure
+                    act[k] = false;
+                    pend[k] = true;
+                }
+                any |= act[k];
+            }
+            if (!__any(any)) break;
+        }
+        off = end;
+    }
+}
+
+// binary search of the sorted array: the last key <= q (tl_query.hip's
+// window steps), or n where every key is larger
+template <typename K, int QN>
+__device__ inline void tile_sorted(const K *__restrict__ A, const TileShape &s, const K (&q)[QN],
+                                   uint32_t (&res)[QN]) {
+    const K first = A[0];
+#pragma unroll
+    for (int k = 0; k < QN; k++) res[k] = 0;
+    for (uint32_t len = s.n; len > 1;) {
+        const uint32_t half = len >> 1;
+        K v[QN];
+#pragma unroll
+        for (int k = 0; k < QN; k++) v[k] = A[res[k] + half];
+#pragma unroll
+        for (int k = 0; k < QN; k++) res[k] += v[k] <= q[k] ? half : 0u;
+        len -= half;
+    }
+#pragma unroll
+    for (int k = 0; k < QN; k++)
+        if (res[k] == 0 && !(first <= q[k])) res[k] = s.n;
+}
+
+// ---- the kernel
+
+template <typename K, int LAYOUT, int QN>
+__device__ inline void tile_descend(const K *__restrict__ A, const TileShape &s,
+                                    const VebEntry *tb, const uint32_t *s_end,
+                                    const uint32_t *s_tidx, const K (&q)[QN],
+                                    uint32_t (&res)[QN]) {
+    if constexpr (LAYOUT == TILE_BST)
+        tile_bst<K, QN>(A, s, q, res);
+    else if constexpr (LAYOUT == TILE_BTREE)
+        tile_btree<K, QN>(A, s, q, res);
+    else if constexpr (LAYOUT == TILE_VEB)
+        tile_veb<K, QN>(A, s, tb, s_end, s_tidx, q, res);
+    else
+        tile_sorted<K, QN>(A, s, q, res);
+}
+
+constexpr int TILE_NT = 512;   // lanes per workgroup
+constexpr int TILE_QN = 4;     // descents of a lane in flight
+
+// IT queries per lane, tiles of NT * IT.  Workgroups go round robin to the 8
+// XCDs; each XCD takes one run of consecutive tiles (neighbouring tiles of a
+// batch in key order share their cache lines in one L2).
+template <typename K, int LAYOUT, int IT, typename AT>
+__global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A, TileShape s,
+                                                        const K *__restrict__ Q, uint64_t nq,
+                                                        AT *__restrict__ ans, uint32_t tiles) {
+    constexpr uint32_t T = TILE_NT * IT;
+    __shared__ K spl[TILE_BINS];               // heap order, node 1 the root
+    __shared__ uint32_t bins[TILE_BINS];
+    __shared__ uint32_t wsum[TILE_NT / 64];
+    __shared__ K keys[T];                      // the tile in bucket order; then its answers
+    __shared__ uint16_t from[T];               // place in the tile of each sorted query
+    __shared__ VebEntry tb[LAYOUT == TILE_VEB ? TILE_TABLES : 1];
+    __shared__ uint32_t s_end[64], s_tidx[64];
+    uint32_t *answers = reinterpret_cast<uint32_t *>(keys);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ SlotMap<LAYOUT> map;
+    slot_map<LAYOUT>(s, map);
+    {
+        for (uint32_t i = tid; i < TILE_BINS; i += TILE_NT) {
+            if (i == 0) continue;
+            spl[i] = A[tile_slot<LAYOUT>(range_first(heap_order(i, 10), s.n, 10), s, map)];
+        }
+        if constexpr (LAYOUT == TILE_VEB) {
+            for (uint32_t i = tid; i < s.table_size; i += TILE_NT)
+                tb[i] = {(uint32_t)s.tables[i].L, (uint32_t)s.tables[i].R, s.tables[i].D};
+            if (tid < s.ntables) {
+                s_end[tid] = s.idx ? (uint32_t)s.idx[tid] : s.n;
+                s_tidx[tid] = s.tidx ? s.tidx[tid] : 0u;
+            }
+        }
+    }
+    const uint32_t per = (tiles + 7) >> 3, step = gridDim.x >> 3;
+    for (uint32_t loc = blockIdx.x >> 3; loc < per; loc += step) {
+        const uint32_t tile = (blockIdx.x & 7) * per + loc;
+        if (tile >= tiles) break;
+        const uint64_t base = (uint64_t)tile * T;
+        const uint32_t cnt = (uint32_t)min((uint64_t)T, nq - base);
+        for (uint32_t i = tid; i < TILE_BINS; i += TILE_NT) bins[i] = 0;
+        __syncthreads();
+        K qv[IT];
+        uint32_t place[IT];   // bucket, then rank within it above bit 10
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const uint32_t i = k * TILE_NT + tid;
+            qv[k] = i < cnt ? Q[base + i] : K{};
+        }
+#pragma unroll
+        for (int k = 0; k < IT; k++) place[k] = 1;
+        for (int t = 0; t < 10; t++) {
+#pragma unroll
+            for (int k = 0; k < IT; k++)
+                place[k] = 2 * place[k] + (qv[k] >= spl[place[k]] ? 1u : 0u);
+        }
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const uint32_t bin = place[k] - TILE_BINS;
+            const uint32_t i = k * TILE_NT + tid;
+            if (i < cnt) place[k] = bin | (atomicAdd(&bins[bin], 1u) << 10);
+        }
+        __syncthreads();
+        {   // exclusive scan of the bucket counts, two a lane
+            const uint32_t a = bins[2 * tid], c = bins[2 * tid + 1];
+            uint32_t x = a + c;
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)x, (unsigned)o);
+                if (lane >= (uint32_t)o) x += y;
+            }
+            if (lane == 63) wsum[wave] = x;
+            __syncthreads();
+            uint32_t before = x - a - c;
+            for (uint32_t w = 0; w < wave; w++) before += wsum[w];
+            bins[2 * tid] = before;
+            bins[2 * tid + 1] = before + a;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const uint32_t i = k * TILE_NT + tid;
+            if (i < cnt) {
+                const uint32_t p = bins[place[k] & (TILE_BINS - 1)] + (place[k] >> 10);
+                keys[p] = qv[k];
+                from[p] = (uint16_t)i;
+            }
+        }
+        __syncthreads();
+        // a wave takes 64 * IT consecutive queries of the order
+        uint32_t src[IT];
+#pragma unroll
+        for (int k = 0; k < IT; k++) {
+            const uint32_t p = min((wave * IT + k) * 64 + lane, cnt - 1);
+            qv[k] = keys[p];
+            src[k] = from[p];
+        }
+        __syncthreads();   // keys[] becomes the answers
+#pragma unroll
+        for (int k0 = 0; k0 < IT; k0 += TILE_QN) {
+            K q[TILE_QN];
+            uint32_t res[TILE_QN];
+#pragma unroll
+            for (int k = 0; k < TILE_QN; k++) q[k] = qv[k0 + k];
+            tile_descend<K, LAYOUT, TILE_QN>(A, s, tb, s_end, s_tidx, q, res);
+#pragma unroll
+            for (int k = 0; k < TILE_QN; k++)
+                if ((wave * IT + k0 + k) * 64 + lane < cnt) answers[src[k0 + k]] = res[k];
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < cnt; i += TILE_NT) ans[base + i] = (AT)answers[i];
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
+// partitioned lookups: batches of at least a few queries per array line.
+//
+// (2^27 queries of 2^30 8-byte keys move 10 GB in the answering kernel, 2.3 ms,
+// and 24 bytes a query and pass through four kernels: count 0.45 ms, scatter
+// 0.6 ms, return 0.45 ms.)
+//
+// The array is cut into 2^lg ranges of equal rank count, each small enough
+// for LDS; the queries are put in range order (one counting pass, or two when
+// there are more ranges than a pass has counters), each workgroup then reads a
+// range's keys once, coalesced, and answers the range's queries from LDS, and
+// the answers go back to the order of the queries.  So the array is read once
+// where the descents of unsorted queries miss the caches on every level past
+// the top ones.
+
+constexpr uint32_t PART_LG = 10;        // log2 of the ranges of one pass, at most
+constexpr uint32_t PART_BINS = 1u << PART_LG;
+constexpr uint32_t PART_NT = 1024;
+constexpr uint32_t PART_GROUP = 32;     // tiles of one column sum
+constexpr uint32_t RANGE_NT = 512;
+constexpr uint32_t RANGE_CHUNK = 4096;  // queries of one workgroup's turn
+
+// bound[j]: the smallest key of range j
+template <typename W, int LAYOUT>
+__global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, TileShape s,
+                                                     uint32_t lg, W *__restrict__ bound) {
+    __shared__ SlotMap<LAYOUT> map;
+    slot_map<LAYOUT>(s, map);
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < (1u << lg)) bound[j] = A[tile_slot<LAYOUT>(range_first(j, s.n, lg), s, map)];
+}
+
+// workgroup b's place in a grid of per * 8: XCD b % 8 takes one run of tiles
+__device__ inline uint32_t xcd_tile(uint32_t tiles) {
+    const uint32_t per = (tiles + 7) >> 3;
+    return (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+}
+
+// what a tile of a pass is: queries [lo, hi) of the input, to be split at the
+// bounds first + step, first + 2 * step, ..
+struct PartTile {
+    uint64_t lo, hi;
+    uint32_t first;
+};
+
+// the tile's bucket tables: tile t of the first pass is queries t * T ..; of
+// the second pass, a piece of one first-pass bucket (tstart: tiles before each
+// bucket, bstart: queries before each bucket)
+template <bool SECOND>
+__device__ inline PartTile part_tile(uint32_t t, uint64_t nq, uint32_t T, uint32_t lg1,
+                                     uint32_t lg2, const uint32_t *__restrict__ bstart,
+                                     const uint32_t *__restrict__ tstart) {
+    PartTile p;
+    if constexpr (SECOND) {
+        uint32_t lo = 0, hi = 1u << lg1;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (tstart[mid] <= t) lo = mid;
+            else hi = mid;
+        }
+        p.lo = bstart[lo] + (uint64_t)(t - tstart[lo]) * T;
+        p.hi = min((uint64_t)bstart[lo + 1], p.lo + T);
+        p.first = lo << lg2;
+    } else {
+        p.lo = (uint64_t)t * T;
+        p.hi = min(nq, p.lo + T);
+        p.first = 0;
+    }
+    return p;
+}
+
+// Counts of a tile's queries per bucket (counts[t][bucket]); every query's
+// bucket and rank among the tile's queries of it go to pack[].
+template <typename K, bool SECOND, int IT>
+__global__ __launch_bounds__(PART_NT) void k_part_count(
+    const K *__restrict__ Q, uint64_t nq, const K *__restrict__ bound, uint32_t lg1, uint32_t lg2,
+    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    uint32_t *__restrict__ pack, uint32_t *__restrict__ counts) {
+    __shared__ K spl[PART_BINS];
+    __shared__ uint32_t cnt[PART_BINS];
+    const uint32_t lg = SECOND ? lg2 : lg1, B = 1u << lg, step = SECOND ? 1u : 1u << lg2;
+    const uint32_t t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    K q[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + threadIdx.x;
+        q[k] = i < p.hi ? Q[i] : K{};
+    }
+    if (threadIdx.x < B) {
+        cnt[threadIdx.x] = 0;
+        if (threadIdx.x)
+            spl[threadIdx.x] = bound[p.first + (uint64_t)heap_order(threadIdx.x, lg) * step];
+    }
+    __syncthreads();
+    uint32_t node[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) node[k] = 1;
+    for (uint32_t l = 0; l < lg; l++) {
+#pragma unroll
+        for (int k = 0; k < IT; k++) node[k] = 2 * node[k] + (q[k] >= spl[node[k]] ? 1u : 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + threadIdx.x;
+        if (i < p.hi) {
+            const uint32_t bin = node[k] - B;
+            pack[i] = bin | (atomicAdd(&cnt[bin], 1u) << PART_LG);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < B) counts[(uint64_t)t * B + threadIdx.x] = cnt[threadIdx.x];
+}
+
+// first pass: sums of each bucket over groups of PART_GROUP tiles
+__global__ __launch_bounds__(PART_NT) void k_part_sums(const uint32_t *__restrict__ counts,
+                                                       uint32_t B, uint32_t tiles,
+                                                       uint32_t *__restrict__ gsum) {
+    const uint32_t t0 = blockIdx.x * PART_GROUP, t1 = min(tiles, t0 + PART_GROUP);
+    if (threadIdx.x >= B) return;
+    uint32_t x = 0;
+#pragma unroll 8
+    for (uint32_t t = t0; t < t1; t++) x += counts[(uint64_t)t * B + threadIdx.x];
+    gsum[(uint64_t)blockIdx.x * B + threadIdx.x] = x;
+}
+
+// exclusive scan of one value a lane over the whole workgroup; the total in
+// *total
+__device__ inline uint32_t block_scan(uint32_t v, uint32_t *wsum, uint32_t *total) {
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, (unsigned)o);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (uint32_t w = 0; w < blockDim.x / 64; w++) {
+        if (w < wave) before += wsum[w];
+        all += wsum[w];
+    }
+    __syncthreads();
+    *total = all;
+    return before + x - v;
+}
+
+// first pass, one workgroup: the groups' sums become the queries of the
+// bucket in earlier groups; bstart[] the queries of earlier buckets; tstart[]
+// the second pass's tiles of T queries of earlier buckets
+__global__ __launch_bounds__(PART_NT) void k_part_starts(uint32_t *__restrict__ gsum, uint32_t B,
+                                                         uint32_t groups, uint32_t T,
+                                                         uint32_t *__restrict__ bstart,
+                                                         uint32_t *__restrict__ tstart) {
+    __shared__ uint32_t wsum[PART_NT / 64];
+    const uint32_t bin = threadIdx.x;
+    uint32_t run = 0;
+    if (bin < B) {
+#pragma unroll 8
+        for (uint32_t g = 0; g < groups; g++) {
+            const uint32_t v = gsum[(uint64_t)g * B + bin];
+            gsum[(uint64_t)g * B + bin] = run;
+            run += v;
+        }
+    }
+    uint32_t total, tiles;
+    const uint32_t at = block_scan(run, wsum, &total);
+    const uint32_t tl = block_scan((run + T - 1) / T, wsum, &tiles);
+    if (bin < B) {
+        bstart[bin] = at;
+        tstart[bin] = tl;
+    }
+    if (bin == 0) {
+        bstart[B] = total;
+        tstart[B] = tiles;
+    }
+}
+
+// first pass: places[t][bucket], the place of the tile's first query of the
+// bucket
+__global__ __launch_bounds__(PART_NT) void k_part_places(const uint32_t *__restrict__ counts,
+                                                         uint32_t B, uint32_t tiles,
+                                                         const uint32_t *__restrict__ gsum,
+                                                         const uint32_t *__restrict__ bstart,
+                                                         uint32_t *__restrict__ places) {
+    const uint32_t t0 = blockIdx.x * PART_GROUP, t1 = min(tiles, t0 + PART_GROUP);
+    const uint32_t bin = threadIdx.x;
+    if (bin >= B) return;
+    uint32_t run = bstart[bin] + gsum[(uint64_t)blockIdx.x * B + bin];
+#pragma unroll 8
+    for (uint32_t t = t0; t < t1; t++) {
+        places[(uint64_t)t * B + bin] = run;
+        run += counts[(uint64_t)t * B + bin];
+    }
+}
+
+// second pass, a workgroup per first-pass bucket: the same for its tiles, and
+// the start of each of its ranges (rstart)
+__global__ __launch_bounds__(PART_NT) void k_part_places2(const uint32_t *__restrict__ counts,
+                                                          uint32_t lg1, uint32_t lg2,
+                                                          const uint32_t *__restrict__ bstart,
+                                                          const uint32_t *__restrict__ tstart,
+                                                          uint32_t *__restrict__ places,
+                                                          uint32_t *__restrict__ rstart) {
+    __shared__ uint32_t wsum[PART_NT / 64];
+    const uint32_t B = 1u << lg2, bin = threadIdx.x, k = blockIdx.x;
+    const uint32_t t0 = tstart[k], t1 = tstart[k + 1];
+    uint32_t sum = 0;
+    if (bin < B) {
+#pragma unroll 8
+        for (uint32_t t = t0; t < t1; t++) sum += counts[(uint64_t)t * B + bin];
+    }
+    uint32_t total;
+    uint32_t run = bstart[k] + block_scan(sum, wsum, &total);
+    if (bin < B) {
+        rstart[((uint64_t)k << lg2) + bin] = run;
+#pragma unroll 8
+        for (uint32_t t = t0; t < t1; t++) {
+            places[(uint64_t)t * B + bin] = run;
+            run += counts[(uint64_t)t * B + bin];
+        }
+    }
+    if (k + 1 == gridDim.x && bin == 0) rstart[(uint64_t)gridDim.x << lg2] = bstart[k + 1];
+}
+
+// Every query to its place.  The tile is put in bucket order in LDS first (the places, then the queries, through one
+// buffer), so that a bucket's queries leave as one run: written from where
+// they were read, single queries filled cache lines so slowly that most were
+// written back several times (5.8 GB for 2^27 8-byte queries, where 1.6 GB
+// are written now).
+template <typename K, bool SECOND, int IT>
+__global__ __launch_bounds__(PART_NT) void k_part_scatter(
+    const K *__restrict__ Q, uint64_t nq, uint32_t lg1, uint32_t lg2,
+    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
+    const uint32_t *__restrict__ pack, K *__restrict__ out) {
+    __shared__ K stage[PART_NT * IT];
+    __shared__ uint32_t at[PART_BINS], local[PART_BINS];
+    __shared__ uint32_t wsum[PART_NT / 64];
+    uint32_t *stage_to = reinterpret_cast<uint32_t *>(stage);
+    const uint32_t B = 1u << (SECOND ? lg2 : lg1), tid = threadIdx.x;
+    const uint32_t t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    const uint32_t cnt = (uint32_t)(p.hi - p.lo);
+    K q[IT];
+    uint32_t pk[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        q[k] = i < p.hi ? Q[i] : K{};
+        pk[k] = i < p.hi ? pack[i] : 0u;
+    }
+    const uint32_t mine = tid < B ? counts[(uint64_t)t * B + tid] : 0u;
+    uint32_t total;
+    const uint32_t before = block_scan(mine, wsum, &total);
+    if (tid < B) {
+        local[tid] = before;
+        at[tid] = places[(uint64_t)t * B + tid] - before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        if (i < p.hi) {
+            const uint32_t bin = pk[k] & (PART_BINS - 1);
+            const uint32_t x = local[bin] + (pk[k] >> PART_LG);   // place in the tile
+            pk[k] = x;
+            stage_to[x] = at[bin] + x;
+        }
+    }
+    __syncthreads();
+    uint32_t to[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        to[k] = x < cnt ? stage_to[x] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++)
+        if (p.lo + k * PART_NT + tid < p.hi) stage[pk[k]] = q[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        if (x < cnt) out[to[k]] = stage[x];
+    }
+}
+
+// The way back: dst[i] = src[place of query i], tile by tile as they were
+// scattered, the runs read into LDS whole (read one by one from there, 2^27
+// answers took 0.72 ms; the vector cache passes on one line a lane).
+// dst may be pack itself.
+template <bool SECOND, int IT, typename AT>
+__global__ __launch_bounds__(PART_NT) void k_part_return(
+    const uint32_t *__restrict__ src, uint64_t nq, uint32_t lg1, uint32_t lg2,
+    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
+    const uint32_t *pack, AT *dst) {
+    __shared__ uint32_t stage[PART_NT * IT];
+    __shared__ uint32_t at[PART_BINS], local[PART_BINS];
+    __shared__ uint32_t wsum[PART_NT / 64];
+    const uint32_t B = 1u << (SECOND ? lg2 : lg1), tid = threadIdx.x;
+    const uint32_t t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    const uint32_t cnt = (uint32_t)(p.hi - p.lo);
+    uint32_t pk[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        pk[k] = i < p.hi ? pack[i] : 0u;
+    }
+    const uint32_t mine = tid < B ? counts[(uint64_t)t * B + tid] : 0u;
+    uint32_t total;
+    const uint32_t before = block_scan(mine, wsum, &total);
+    if (tid < B) {
+        local[tid] = before;
+        at[tid] = places[(uint64_t)t * B + tid] - before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t bin = pk[k] & (PART_BINS - 1);
+        const uint32_t x = local[bin] + (pk[k] >> PART_LG);
+        if (p.lo + k * PART_NT + tid < p.hi) stage[x] = at[bin] + x;
+        pk[k] = x;
+    }
+    __syncthreads();
+    uint32_t v[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        v[k] = x < cnt ? src[stage[x]] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++) {   // a lane's own places
+        const uint32_t x = k * PART_NT + tid;
+        if (x < cnt) stage[x] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        if (i < p.hi) dst[i] = (AT)stage[pk[k]];
+    }
+}
+
+template <typename K>
+__device__ inline K key_max() {
+    return (K)-1 > (K)0 ? (K)-1 : (K)(((K)1 << (8 * sizeof(K) - 2)) - 1 + ((K)1 << (8 * sizeof(K) - 2)));
+}
+
+// slots of a range on one level of a B-tree, where `level`: place y is at
+// first + y - row, row the places' c0 + y in rows of b + 1, or, for a row's
+// last, at sep_slot[row] (tabled for the first SEP_SLOTS)
+constexpr uint32_t SEP_SLOTS = 1024;
+struct RangeSlots {
+    bool level;
+    uint32_t first, c0;
+};
+
+// The m keys of ranks r0 .. : the first in heap[0], rank r0 + y at place y of
+// the heap of 2^depth - 1 nodes, the places past them the largest key.  All of
+// a lane's loads are issued before the first is stored.  The ranks' slots are
+// what this costs (with tile_slot() for every key the vector unit was busy for
+// three quarters of the time of a B-tree's ranges and all of a vEB's), so they
+// are found by what neighbours share:
+//   B-tree: all keys of a range on the leaf level (or the one above it) lie at
+//     rank - row + a constant, and rows follow from the place in the range by
+//     a 24-bit product; the separators between them take tile_slot().
+//   vEB: 64 consecutive ranks share a bottom tree of 64 or more, which one
+//     lane finds for them; the root behind it takes tile_slot().
+template <typename K, int LAYOUT>
+__device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape &s,
+                                        const SlotMap<LAYOUT> &map, uint32_t r0, uint32_t m,
+                                        uint32_t depth, K *heap, uint32_t *sep_slot) {
+    constexpr uint32_t PER = RANGE_KEYS / RANGE_NT;
+    const uint32_t tid = threadIdx.x;
+    // heap_at(k * RANGE_NT + tid): the trailing zeros are the lane's, but lane 0's
+    const uint32_t up = tid ? (uint32_t)__clz((int)__brev(tid)) + 1 : 0u;
+    auto lane_node = [&](uint32_t k, uint32_t lg) {
+        const uint32_t y = k * RANGE_NT + tid;
+        return tid ? (y | (1u << lg)) >> up : heap_at(y, lg);
+    };
+    if constexpr (LAYOUT == TILE_BTREE) {
+        const uint32_t k1 = s.b + 1, past = s.span + s.rem;
+        const bool leaf = r0 + m <= s.span;
+        if (leaf || r0 >= past) {
+            const uint32_t x0 = leaf ? r0 : r0 - past + s.nsep;   // rank on its level
+            const uint32_t row0 = (uint32_t)__umul64hi(x0, s.recip), c0 = x0 - row0 * k1;
+            const uint32_t first = (leaf ? s.nint : map.level[0]) + (x0 - row0);
+            const K *at = A + first;
+            // separators: the ends of rows row0 ..
+            const uint32_t seps = ((c0 + m) * s.small_mul) >> s.small_shift;
+            const uint32_t per = (seps + RANGE_NT - 1) / RANGE_NT;
+            constexpr uint32_t SEP = 2;   // kept in registers, more where b < 3
+            K v[PER], w[SEP];
+            auto sep_at = [&](uint32_t i) { return (i + 1) * k1 - 1 - c0; };   // its place
+#pragma unroll
+            for (uint32_t k = 0; k < PER; k++) {
+                const uint32_t y = k * RANGE_NT + tid;
+                const uint32_t t = c0 + y, q = (t * s.small_mul) >> s.small_shift;
+                v[k] = y < m && t - q * k1 != s.b ? at[y - q] : key_max<K>();
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < SEP; k++) {
+                const uint32_t i = k * RANGE_NT + tid;
+                if (i < seps) {
+                    const uint32_t slot = tile_slot<LAYOUT>(r0 + sep_at(i), s, map);
+                    w[k] = A[slot];
+                    if (i < SEP_SLOTS) sep_slot[i] = slot;
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < PER; k++) {
+                const uint32_t y = k * RANGE_NT + tid;
+                const uint32_t t = c0 + y, q = (t * s.small_mul) >> s.small_shift;
+                if (y < (1u << depth) && (t - q * k1 != s.b || y >= m))
+                    heap[lane_node(k, depth)] = v[k];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < SEP; k++) {
+                const uint32_t i = k * RANGE_NT + tid;
+                if (i < seps) heap[heap_at(sep_at(i), depth)] = w[k];
+            }
+            for (uint32_t k = SEP; k < per; k++) {
+                const uint32_t i = k * RANGE_NT + tid;
+                if (i < seps)
+                    heap[heap_at(sep_at(i), depth)] =
+                        A[tile_slot<LAYOUT>(r0 + sep_at(i), s, map)];
+            }
+            return {true, first, c0};
+        }
+    }
+    if constexpr (LAYOUT == TILE_VEB) {
+        // groups of 64 ranks starting at multiples of 64, PER + 1 a wave: lane k
+        // finds the bottom tree of group k (d levels, first slot base, the
+        // group's first rank u in it) and whether its last rank is a root
+        const uint32_t lane = tid & 63, g0 = (r0 & ~63u) + (tid & ~63u);
+        uint32_t base = 0, mine;
+        bool root_here = false;
+        {
+            uint32_t u = g0 + lane * RANGE_NT, d = s.chain_d;
+            bool whole = lane <= PER, tail = false;
+            for (uint32_t j = 0; j < s.nchain; j++) {
+                const VebLevel e = s.chain[j];
+                const uint32_t span = e.nf << e.ld, l = (1u << e.ld) - 1;
+                if (u < span) {
+                    whole = whole && e.ld >= 6;
+                    base += (1u << e.rd) - 1 + (u >> e.ld) * l;
+                    u &= l;
+                    tail = u + 63 == l;
+                    d = e.ld;
+                    break;
+                }
+                if (e.ld < 6 || u + 64 > span + e.inc) {
+                    whole = false;
+                    break;
+                }
+                base += (1u << e.rd) - 1 + e.nf * l;
+                u -= span;
+            }
+            while (whole && d > SMALL_LEVELS) {
+                const uint32_t rd = s.split[d], ld = d - rd, l = (1u << ld) - 1;
+                whole = ld >= 6 && u + 64 <= (1u << d) - (tail ? 0u : 1u);
+                base += (1u << rd) - 1 + (u >> ld) * l;
+                u &= l;
+                tail = u + 63 == l;
+                d = ld;
+            }
+            whole = whole && d >= 6 && u + 64 <= (1u << d) - (tail ? 0u : 1u);
+            root_here = whole && tail;
+            // u < 2^d <= 2^SMALL_LEVELS where whole
+            mine = whole ? ((1u << d) + u) | (tail ? 1u << 30 : 0u) | 1u << 31 : 0u;
+        }
+        K v[PER + 1], root{};
+#pragma unroll
+        for (uint32_t k = 0; k <= PER; k++) {
+            const uint32_t x = g0 + k * RANGE_NT + lane;
+            const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)k);
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)k);
+            if (x >= r0 && x < r0 + m && !(lane == 63 && (at >> 30) == 3))
+                v[k] = A[at ? first + map.small[(at & 0xFFFF) + lane] : veb_slot(x, s, map)];
+        }
+        const uint32_t my_root = g0 + lane * RANGE_NT + 63;
+        root_here = root_here && my_root >= r0 && my_root < r0 + m;
+        if (root_here) root = A[veb_slot(my_root, s, map)];
+#pragma unroll
+        for (uint32_t k = 0; k <= PER; k++) {
+            const uint32_t x = g0 + k * RANGE_NT + lane;
+            const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)k);
+            if (x >= r0 && x < r0 + m && !(lane == 63 && (at >> 30) == 3))
+                heap[heap_at(x - r0, depth)] = v[k];
+        }
+        if (root_here) heap[heap_at(my_root - r0, depth)] = root;
+        for (uint32_t y = m + tid; y < (1u << depth); y += RANGE_NT)
+            heap[heap_at(y, depth)] = key_max<K>();
+        return {false, 0, 0};
+    }
+    K v[PER];
+#pragma unroll
+    for (uint32_t k = 0; k < PER; k++) {
+        const uint32_t y = k * RANGE_NT + tid;
+        v[k] = y < m ? A[tile_slot<LAYOUT>(r0 + y, s, map)] : key_max<K>();
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < PER; k++) {
+        const uint32_t y = k * RANGE_NT + tid;
+        if (y < (1u << depth)) heap[lane_node(k, depth)] = v[k];
+    }
+    return {false, 0, 0};
+}
+
+// The queries of a range from its keys in LDS.  S holds the queries in range
+// order, range j's at rstart[j] .. rstart[j + 1].  A key that occurs more than
+// once is answered by the descent itself, whose first equal key it has to be.
+template <typename K, int LAYOUT>
+__global__ __launch_bounds__(RANGE_NT) void k_part_answer(
+    const K *__restrict__ A, TileShape s, uint32_t lg, const K *__restrict__ S, uint32_t nq,
+    const uint32_t *__restrict__ rstart, uint32_t chunks, uint32_t *__restrict__ out) {
+    constexpr uint32_t WIN = 64;   // range starts at hand
+    __shared__ K heap[RANGE_KEYS];
+    __shared__ uint32_t sep_slot[LAYOUT == TILE_BTREE ? SEP_SLOTS : 1];
+    __shared__ uint32_t win[WIN + 1];
+    __shared__ VebEntry tb[LAYOUT == TILE_VEB ? TILE_TABLES : 1];
+    __shared__ uint32_t s_end[64], s_tidx[64];
+    __shared__ SlotMap<LAYOUT> map;
+    const uint32_t tid = threadIdx.x, n = s.n, ranges = 1u << lg;
+    if constexpr (LAYOUT == TILE_VEB) {
+        for (uint32_t i = tid; i < s.table_size; i += RANGE_NT)
+            tb[i] = {(uint32_t)s.tables[i].L, (uint32_t)s.tables[i].R, s.tables[i].D};
+        if (tid < s.ntables) {
+            s_end[tid] = s.idx ? (uint32_t)s.idx[tid] : n;
+            s_tidx[tid] = s.tidx ? s.tidx[tid] : 0u;
+        }
+    }
+    const uint32_t chunk = xcd_tile(chunks);
+    if (chunk >= chunks) return;
+    slot_map<LAYOUT>(s, map);
+    uint32_t p = chunk * RANGE_CHUNK;
+    const uint32_t p1 = min(nq, p + RANGE_CHUNK);
+    while (p < p1) {
+        // the range of query p, and the starts of the ranges after it
+        uint32_t lo = 0, hi = ranges;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (rstart[mid] <= p) lo = mid;
+            else hi = mid;
+        }
+        const uint32_t j0 = lo;
+        __syncthreads();
+        if (tid <= WIN) win[tid] = rstart[min(j0 + tid, ranges)];
+        __syncthreads();
+        for (uint32_t w = 0; w < WIN && p < p1; w++) {
+            const uint32_t qhi = min(p1, win[w + 1]);
+            if (qhi <= p) continue;
+            const uint32_t j = j0 + w;
+            const uint32_t r0 = range_first(j, n, lg), m = range_first(j + 1, n, lg) - r0;
+            const uint32_t depth = 32u - (uint32_t)__clz((int)(m - 1));   // 2^depth >= m
+            K q = p + tid < qhi ? S[p + tid] : K{};
+            __syncthreads();   // the last range's queries are answered
+            const RangeSlots rs = range_fill<K, LAYOUT>(A, s, map, r0, m, depth, heap, sep_slot);
+            __syncthreads();
+            for (uint32_t q0 = p; q0 < qhi; q0 += RANGE_NT) {
+                const uint32_t i = q0 + tid;
+                if (q0 != p) q = i < qhi ? S[i] : K{};
+                // the keys after the first that are smaller than q
+                // (TILE_SORTED: not larger)
+                uint32_t node = 1;
+                for (uint32_t l = 0; l < depth; l++) {
+                    const K key = heap[node];
+                    const bool right = LAYOUT == TILE_SORTED ? key <= q : key < q;
+                    node = 2 * node + (right ? 1u : 0u);
+                }
+                const uint32_t below = min(node - (1u << depth), m - 1);
+                uint32_t ans = n;
+                if constexpr (LAYOUT == TILE_SORTED) {
+                    if (heap[0] <= q) ans = r0 + below;
+                } else {
+                    bool again = false;
+                    const uint32_t x = q <= heap[0] ? 0u : below + 1;
+                    if (x < m && heap[heap_at(x, depth)] == q) {
+                        const uint32_t t = rs.c0 + x, row = (t * s.small_mul) >> s.small_shift;
+                        if (LAYOUT == TILE_BTREE && rs.level && row < SEP_SLOTS)
+                            ans = t - row * (s.b + 1) != s.b ? rs.first + x - row : sep_slot[row];
+                        else
+                            ans = tile_slot<LAYOUT>(r0 + x, s, map);
+                        if (x == 0 && r0 > 0) again = A[tile_slot<LAYOUT>(r0 - 1, s, map)] == q;
+                        if (x + 1 < m) again |= heap[heap_at(x + 1, depth)] == q;
+                    }
+                    if (__any(again)) {
+                        const K qq[1] = {q};
+                        uint32_t res[1];
+                        tile_descend<K, LAYOUT, 1>(A, s, tb, s_end, s_tidx, qq, res);
+                        if (again) ans = res[0];
+                    }
+                }
+                if (i < qhi) out[i] = ans;
+            }
+            p = qhi;
+        }
+    }
+}
+
+// ---- host side
+
+static TileShape tile_shape(const TileArray &a) {
+    TileShape s{};
+    s.n = (uint32_t)a.n;
+    s.b = (uint32_t)a.b;
+    if (a.layout == TILE_BST || a.layout == TILE_BTREE) {
+        const uint32_t b = a.layout == TILE_BST ? 1u : s.b;
+        s.nodes = (uint32_t)((a.n + b - 1) / b);
+        s.levels = ilog_base(a.n + 1, b + 1);   // levels whose every node is whole
+        const BtreeShape bs = btree_shape(s.n, b);
+        s.nint = bs.nint;
+        s.span = bs.span;
+        s.rem = bs.rem;
+        s.nsep = bs.nsep;
+        s.depth = ilog_base((uint64_t)bs.nint + 1, b + 1);
+        s.recip = ~0ull / (b + 1) + 1;
+        // exact below 2 RANGE_KEYS: 2^shift > 2 RANGE_KEYS (b + 1)
+        s.small_shift = floor_log2_64(2ull * RANGE_KEYS * (b + 1)) + 1;
+        s.small_mul = (uint32_t)(((1ull << s.small_shift) + b) / (b + 1));
+    }
+    if (a.layout == TILE_VEB) {
+        uint64_t n = a.n;
+        for (uint32_t d = 2; d <= 32; d++) {
+            uint32_t rd, ld;
+            veb_split(d, rd, ld, a.classic);
+            s.split[d] = (uint8_t)rd;
+        }
+        while (n & (n + 1)) {
+            VebLevel &e = s.chain[s.nchain++];
+            veb_split(floor_log2_64(n) + 1, e.rd, e.ld, a.classic);
+            const uint64_t r = (1ull << e.rd) - 1, l = (1ull << e.ld) - 1;
+            e.nf = (uint32_t)((n - r) / l);
+            e.inc = (uint32_t)(n - r - e.nf * l);
+            n = e.inc;
+        }
+        s.chain_d = n ? floor_log2_64(n) + 1 : 0;
+    }
+    s.table_size = a.table_size;
+    s.ntables = a.ntables;
+    s.tables = a.tables;
+    s.idx = a.idx;
+    s.tidx = a.tidx;
+    s.classic = a.classic;
+    return s;
+}
+
+template <typename K, int LAYOUT, int IT, typename AT>
+static void tile_launch(Ctx *c, const TileArray &a, const void *q, uint64_t nq, AT *ans,
+                        hipStream_t s) {
+    constexpr uint32_t T = TILE_NT * IT;
+    const uint32_t tiles = (uint32_t)((nq + T - 1) / T);
+    const uint32_t per_cu = 4;
+    const uint32_t grid = std::min<uint32_t>((tiles + 7) / 8, c->num_cus * per_cu / 8) * 8;
+    hipLaunchKernelGGL((k_query_tile<K, LAYOUT, IT, AT>), dim3(grid), dim3(TILE_NT), 0, s,
+                       (const K *)a.A, tile_shape(a), (const K *)q, nq, ans, tiles);
+}
+
+template <typename K, int IT, typename AT>
+static void tile_layout(Ctx *c, const TileArray &a, const void *q, uint64_t nq, AT *ans,
+                        hipStream_t s) {
+    switch (a.layout) {
+    case TILE_BST: tile_launch<K, TILE_BST, IT, AT>(c, a, q, nq, ans, s); break;
+    case TILE_BTREE: tile_launch<K, TILE_BTREE, IT, AT>(c, a, q, nq, ans, s); break;
+    case TILE_VEB: tile_launch<K, TILE_VEB, IT, AT>(c, a, q, nq, ans, s); break;
+    default: tile_launch<K, TILE_SORTED, IT, AT>(c, a, q, nq, ans, s); break;
+    }
+}
+
+tl_status tile_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
+                     uint64_t *ans, hipStream_t s) {
+    switch (dtype) {
+    case TL_U32: tile_layout<uint32_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
+    case TL_U64: tile_layout<uint64_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
+    case TL_I32: tile_layout<int32_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
+    default: tile_layout<int64_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
+    }
+    TL_LAUNCH_CHECK();
+    return TL_OK;
+}
+
+// ---- partitioned lookups
+
+// where everything of one partitioned batch lies in its workspace
+struct PartPlan {
+    uint32_t lg1, lg2, it, tiles1, tiles2, groups;
+    uint64_t bound, bstart, tstart, rstart, gsum, counts, places, counts2, places2, pack, pack2;
+    uint64_t second, bytes;
+};
+
+static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
+    PartPlan p{};
+    uint32_t lg = 1;
+    while (((n + (1ull << lg) - 1) >> lg) > RANGE_KEYS) lg++;
+    p.lg1 = std::min(lg, PART_LG);
+    p.lg2 = lg - p.lg1;
+    p.it = nq >= (1u << 22) ? 16 : 4;
+    const uint64_t T = (uint64_t)PART_NT * p.it;
+    p.tiles1 = (uint32_t)((nq + T - 1) / T);
+    p.tiles2 = p.lg2 ? p.tiles1 + (1u << p.lg1) : 0;
+    p.groups = (p.tiles1 + PART_GROUP - 1) / PART_GROUP;
+    uint64_t at = 0;
+    auto take = [&](uint64_t bytes) {
+        const uint64_t o = at;
+        at += (bytes + 255) & ~255ull;
+        return o;
+    };
+    p.bound = take((uint64_t)w << lg);
+    p.bstart = take(((1ull << p.lg1) + 1) * 4);
+    p.tstart = take(((1ull << p.lg1) + 1) * 4);
+    p.rstart = p.lg2 ? take(((1ull << lg) + 1) * 4) : p.bstart;
+    p.gsum = take(((uint64_t)p.groups << p.lg1) * 4);
+    p.counts = take(((uint64_t)p.tiles1 << p.lg1) * 4);
+    p.places = take(((uint64_t)p.tiles1 << p.lg1) * 4);
+    if (p.lg2) {
+        p.counts2 = take(((uint64_t)p.tiles2 << p.lg2) * 4);
+        p.places2 = take(((uint64_t)p.tiles2 << p.lg2) * 4);
+    }
+    p.pack = take(nq * 4);
+    p.pack2 = take(nq * 4);   // then the answers in the first pass's order
+    // the queries after the second pass: behind those after the first in the
+    // answer array, which has room for both when keys have 4 bytes
+    p.second = p.lg2 && w == 8 ? take(nq * 8) : 0;
+    p.bytes = at;
+    return p;
+}
+
+constexpr uint64_t PART_MAX_QUERIES = 1ull << 27;   // of one segment of a batch
+
+uint64_t part_bytes(const TileArray &a, uint32_t dtype, uint64_t nq) {
+    const uint32_t w = (dtype == TL_U32 || dtype == TL_I32) ? 4 : 8;
+    return part_plan(a.n, w, std::min(nq, PART_MAX_QUERIES)).bytes;
+}
+
+template <typename K, bool SECOND, int IT>
+static void part_pass(const PartPlan &p, const K *q, uint64_t nq, char *ws, K *out,
+                      hipStream_t s) {
+    uint32_t *bstart = (uint32_t *)(ws + p.bstart), *tstart = (uint32_t *)(ws + p.tstart);
+    uint32_t *counts = (uint32_t *)(ws + (SECOND ? p.counts2 : p.counts));
+    uint32_t *places = (uint32_t *)(ws + (SECOND ? p.places2 : p.places));
+    uint32_t *pack = (uint32_t *)(ws + (SECOND ? p.pack2 : p.pack));
+    uint32_t *gsum = (uint32_t *)(ws + p.gsum);
+    const uint32_t tiles = SECOND ? p.tiles2 : p.tiles1, B1 = 1u << p.lg1;
+    const dim3 grid((tiles + 7) / 8 * 8), block(PART_NT);
+    hipLaunchKernelGGL((k_part_count<K, SECOND, IT>), grid, block, 0, s, q, nq,
+                       (const K *)(ws + p.bound), p.lg1, p.lg2, (const uint32_t *)bstart,
+                       (const uint32_t *)tstart, tiles, pack, counts);
+    if (SECOND) {
+        hipLaunchKernelGGL(k_part_places2, dim3(B1), block, 0, s, (const uint32_t *)counts, p.lg1,
+                           p.lg2, (const uint32_t *)bstart, (const uint32_t *)tstart, places,
+                           (uint32_t *)(ws + p.rstart));
+    } else {
+        hipLaunchKernelGGL(k_part_sums, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
+                           tiles, gsum);
+        hipLaunchKernelGGL(k_part_starts, dim3(1), block, 0, s, gsum, B1, p.groups,
+                           (uint32_t)(PART_NT * IT), bstart, tstart);
+        hipLaunchKernelGGL(k_part_places, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
+                           tiles, (const uint32_t *)gsum, (const uint32_t *)bstart, places);
+    }
+    hipLaunchKernelGGL((k_part_scatter<K, SECOND, IT>), grid, block, 0, s, q, nq, p.lg1, p.lg2,
+                       (const uint32_t *)bstart, (const uint32_t *)tstart, tiles,
+                       (const uint32_t *)places, (const uint32_t *)counts, (const uint32_t *)pack,
+                       out);
+}
+
+// the answers of a pass's output order to its input order
+template <bool SECOND, int IT, typename AT>
+static void part_return(const PartPlan &p, const uint32_t *found, uint64_t nq, char *ws, AT *dst,
+                        hipStream_t s) {
+    const uint32_t tiles = SECOND ? p.tiles2 : p.tiles1;
+    hipLaunchKernelGGL((k_part_return<SECOND, IT, AT>), dim3((tiles + 7) / 8 * 8), dim3(PART_NT), 0,
+                       s, found, nq, p.lg1, p.lg2, (const uint32_t *)(ws + p.bstart),
+                       (const uint32_t *)(ws + p.tstart), tiles,
+                       (const uint32_t *)(ws + (SECOND ? p.places2 : p.places)),
+                       (const uint32_t *)(ws + (SECOND ? p.counts2 : p.counts)),
+                       (const uint32_t *)(ws + (SECOND ? p.pack2 : p.pack)), dst);
+}
+
+template <typename K, int LAYOUT, int IT>
+static void part_segment(const PartPlan &p, const TileArray &a, const K *q, uint64_t nq,
+                         uint64_t *ans, char *ws, hipStream_t s) {
+    using W = typename std::conditional<sizeof(K) == 4, uint32_t, uint64_t>::type;
+    const TileShape sh = tile_shape(a);
+    const uint32_t lg = p.lg1 + p.lg2;
+    const uint32_t chunks = (uint32_t)((nq + RANGE_CHUNK - 1) / RANGE_CHUNK);
+    hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256), dim3(256), 0, s,
+                       (const W *)a.A, sh, lg, (W *)(ws + p.bound));
+    K *first = (K *)ans, *sorted = first;
+    uint32_t *found = (uint32_t *)(ws + p.pack2);
+    part_pass<K, false, IT>(p, q, nq, ws, first, s);
+    if (p.lg2) {
+        sorted = sizeof(K) == 4 ? first + nq : (K *)(ws + p.second);
+        part_pass<K, true, IT>(p, first, nq, ws, sorted, s);
+        found = (uint32_t *)ans;
+    }
+    hipLaunchKernelGGL((k_part_answer<K, LAYOUT>), dim3((chunks + 7) / 8 * 8), dim3(RANGE_NT), 0,
+                       s, (const K *)a.A, sh, lg, (const K *)sorted, (uint32_t)nq,
+                       (const uint32_t *)(ws + p.rstart), chunks, found);
+    if (p.lg2) {
+        part_return<true, IT>(p, found, nq, ws, (uint32_t *)(ws + p.pack2), s);
+        found = (uint32_t *)(ws + p.pack2);
+    }
+    part_return<false, IT>(p, found, nq, ws, ans, s);
+}
+
+template <typename K, int LAYOUT>
+static void part_segment(const TileArray &a, const K *q, uint64_t nq, uint64_t *ans, char *ws,
+                         hipStream_t s) {
+    const PartPlan p = part_plan(a.n, sizeof(K), nq);
+    if (p.it == 16)
+        part_segment<K, LAYOUT, 16>(p, a, q, nq, ans, ws, s);
+    else
+        part_segment<K, LAYOUT, 4>(p, a, q, nq, ans, ws, s);
+}
+
+template <typename K>
+static void part_layout(const TileArray &a, const K *q, uint64_t nq, uint64_t *ans, char *ws,
+                        hipStream_t s) {
+    for (uint64_t at = 0; at < nq; at += PART_MAX_QUERIES) {
+        const uint64_t m = std::min(PART_MAX_QUERIES, nq - at);
+        switch (a.layout) {
+        case TILE_BST: part_segment<K, TILE_BST>(a, q + at, m, ans + at, ws, s); break;
+        case TILE_BTREE: part_segment<K, TILE_BTREE>(a, q + at, m, ans + at, ws, s); break;
+        case TILE_VEB: part_segment<K, TILE_VEB>(a, q + at, m, ans + at, ws, s); break;
+        default: part_segment<K, TILE_SORTED>(a, q + at, m, ans + at, ws, s); break;
+        }
+    }
+}
+
+tl_status part_query(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq, uint64_t *ans,
+                     void *ws, hipStream_t s) {
+    switch (dtype) {
+    case TL_U32: part_layout<uint32_t>(a, (const uint32_t *)q, nq, ans, (char *)ws, s); break;
+    case TL_U64: part_layout<uint64_t>(a, (const uint64_t *)q, nq, ans, (char *)ws, s); break;
+    case TL_I32: part_layout<int32_t>(a, (const int32_t *)q, nq, ans, (char *)ws, s); break;
+    default: part_layout<int64_t>(a, (const int64_t *)q, nq, ans, (char *)ws, s); break;
+    }
+    TL_LAUNCH_CHECK();
+    return TL_OK;
+}
+
+// ---- which of them answers a batch
+
+static uint32_t key_width(uint32_t dtype) { return (dtype == TL_U32 || dtype == TL_I32) ? 4 : 8; }
+
+bool tile_can(const TileArray &a, uint32_t dtype, uint64_t nq) {
+    if (dtype > TL_I64 || a.n < 4096 || a.n >= (1ull << 32) - 1 || nq < (1u << 16) ||
+        nq >= (1ull << 40))
+        return false;
+    // every node number of a descent fits 32 bits
+    if (a.layout == TILE_BTREE &&
+        (a.b < 1 || a.b > 1024 || (a.n + a.b - 1) / a.b >= (1ull << 32) / (a.b + 1) - 1))
+        return false;
+    // conceptual positions (below twice the structure's keys) fit 32 bits
+    if (a.layout == TILE_VEB &&
+        (a.table_size > TILE_TABLES || a.ntables > 64 || a.n >= (1ull << 31)))
+        return false;
+    return true;
+}
+
+bool part_can(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
+              const uint64_t *ans) {
+    if (!tile_can(a, dtype, nq)) return false;
+    // the answer array holds the queries in range order meanwhile
+    const char *q0 = (const char *)q, *a0 = (const char *)ans;
+    if (q0 < a0 + nq * 8 && a0 < q0 + nq * key_width(dtype)) return false;
+    // ranges are of the whole layout: its tables have to be those of all of it
+    if (a.layout == TILE_VEB) {
+        const TileShape s = tile_shape(a);
+        uint32_t structures = 1;
+        for (uint32_t j = 0; j < s.nchain; j++) structures += s.chain[j].inc != 0;
+        if (structures != a.ntables) return false;
+    }
+    return true;
+}
+
+// Time of a batch in picoseconds by each path, from lookups of uniform keys
+// measured on arrays of 2^14 .. 2^28 keys of both widths: a start-up, and per
+// query a figure that grows with the array's bytes (2^16, 2^18 .. 2^32).
+struct PathCost {
+    double start;
+    uint16_t query[9];
+};
+static double path_ps(const PathCost &c, uint64_t n, uint32_t w, uint64_t nq, double more = 0) {
+    const double l = std::min(16.0, std::max(0.0, log2((double)n * w) - 16)) / 2;
+    const int i = std::min(7, (int)l);
+    const double q = c.query[i] + (c.query[i + 1] - c.query[i]) * (l - i);
+    return c.start + (double)nq * std::max(1.0, q + more);
+}
+
+// the kernels of tl_query.hip, and the tile-sorted descents.  The wide B-tree
+// descent's cost is its lanes': 5 ps more a query for each lane of a node
+// past two.  A partitioned batch reads every range (2.3 ps a key, slots and
+// all) and moves every query 18 ps worth a pass, whatever the layout.
+static const PathCost COST_OLD[] = {{8e6, {13, 15, 20, 28, 45, 75, 112, 152, 190}},
+                                    {5e6, {18, 22, 22, 26, 27, 32, 44, 57, 70}},
+                                    {8e6, {27, 33, 39, 45, 58, 71, 90, 129, 160}},
+                                    {12e6, {13, 22, 31, 40, 122, 197, 248, 290, 330}}};
+static const PathCost COST_GROUP = {5e6, {38, 44, 48, 53, 63, 64, 75, 90, 105}};
+static const PathCost COST_TILE[] = {{12e6, {7, 8, 11, 17, 33, 73, 110, 148, 185}},
+                                     {22e6, {15, 18, 22, 32, 45, 76, 124, 180, 240}},
+                                     {38e6, {21, 27, 31, 37, 50, 76, 103, 144, 180}},
+                                     {12e6, {8, 15, 26, 37, 89, 162, 211, 259, 300}}};
+
+static double old_ps(const TileArray &a, uint32_t w, uint64_t nq) {
+    if (a.layout != TILE_BTREE) return path_ps(COST_OLD[a.layout], a.n, w, nq);
+    if (a.b > 64) return 5e6 + (double)nq * 4.0 * a.b;   // one lane scans the nodes
+    if (a.b == 1) return path_ps(COST_OLD[TILE_BST], a.n, w, nq);
+    if (wide_ok(a.A, a.b, w))
+        return path_ps(COST_OLD[TILE_BTREE], a.n, w, nq, 5.0 * wide_group(a.b, w) - 10.0);
+    return path_ps(COST_GROUP, a.n, w, nq);
+}
+
+static double part_ps(const TileArray &a, uint32_t w, uint64_t nq) {
+    const uint32_t passes = part_plan(a.n, w, std::min(nq, PART_MAX_QUERIES)).lg2 ? 2 : 1;
+    const uint64_t segments = (nq + PART_MAX_QUERIES - 1) / PART_MAX_QUERIES;
+    return segments * (50e6 * passes + 2.3 * a.n) + (double)nq * 18 * passes;
+}
+
+Workspace &query_workspace() {
+    static thread_local Workspace w;
+    return w;
+}
+
+// $TL_QUERY_PATH: plain, tile or part picks that path wherever it can run
+static int forced_path() {
+    const char *e = getenv("TL_QUERY_PATH");
+    if (!e) return -1;
+    return !strcmp(e, "plain") ? 0 : !strcmp(e, "tile") ? 1 : !strcmp(e, "part") ? 2 : -1;
+}
+
+bool part_wanted(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
+                 const uint64_t *ans, double other) {
+    if (!part_can(a, dtype, q, nq, ans)) return false;
+    const int f = forced_path();
+    if (f >= 0) return f == 2;
+    const uint32_t w = key_width(dtype);
+    return part_ps(a, w, nq) < other * std::min(old_ps(a, w, nq), path_ps(COST_TILE[a.layout], a.n, w, nq));
+}
+
+tl_status part_try(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
+                   uint64_t *ans, hipStream_t s, double other, bool *taken) {
+    *taken = false;
+    if (!part_wanted(a, dtype, q, nq, ans, other)) return TL_OK;
+    const uint64_t need = part_bytes(a, dtype, nq);
+    const Workspace &w = query_workspace();
+    if (w.mem) {
+        if (w.bytes < need) return TL_OK;
+        *taken = true;
+        return part_query(a, dtype, q, nq, ans, w.mem, s);
+    }
+    Lease *l = lease_take(c, need, s);
+    if (!l) return TL_OK;
+    *taken = true;
+    const tl_status st = part_query(a, dtype, q, nq, ans, l->mem, s);
+    lease_give(l, s);
+    return st;
+}
+
+tl_status large_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
+                      uint64_t *ans, hipStream_t s, bool *taken) {
+    TL_TRY(part_try(c, a, dtype, q, nq, ans, s, 1.0, taken));
+    if (*taken || !tile_can(a, dtype, nq)) return TL_OK;
+    const int f = forced_path();
+    const uint32_t w = key_width(dtype);
+    if (f == 0 || (f < 0 && path_ps(COST_TILE[a.layout], a.n, w, nq) >= old_ps(a, w, nq)))
+        return TL_OK;
+    *taken = true;
+    return tile_query(c, a, dtype, q, nq, ans, s);
+}
+
+}   // namespace tl
