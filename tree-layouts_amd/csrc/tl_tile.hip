@@ -30,6 +30,7 @@
 
 #include "tl_descent.hpp"
 #include "tl_internal.hpp"
+#include "tl_slots.hpp"
 #include "tl_tile.hpp"
 
 namespace tl {
@@ -39,139 +40,19 @@ constexpr uint32_t TILE_TABLES = 256;   // vEB table entries kept in LDS
 
 constexpr uint32_t RANGE_KEYS = 4096;   // keys of a range, at most (partitioned lookups)
 
-// an incomplete vEB tree: top and bottom levels, full bottom trees, keys of the
-// incomplete one
-constexpr uint32_t VEB_CHAIN = 8;
-struct VebLevel {
-    uint32_t rd, ld, nf, inc;
-};
-
-struct TileShape {
-    uint32_t n;
-    uint32_t b, nodes;      // TILE_BTREE
+struct TileShape : SlotShape {
+    uint32_t nodes;         // TILE_BTREE
     uint32_t levels;        // full levels: of the binary tree, or of nodes
     uint32_t table_size, ntables;
     const tl_veb_table *tables;
     const uint64_t *idx;
     const uint32_t *tidx;
-    uint32_t classic;
-    // rank -> slot of a BST or B-tree (BtreeShape's); 2^64 / (b + 1) rounded up
-    uint32_t nint, span, rem, nsep, depth;
-    uint64_t recip;
     uint32_t small_mul, small_shift;   // x / (b + 1) = x * mul >> shift, x < 2 RANGE_KEYS
-    // rank -> slot of a vEB: the incomplete trees from the whole one down (the
-    // incomplete bottom tree of one is the next), then a perfect tree of
-    // chain_d levels (0: none); split[d]: top levels of a perfect tree of d
-    VebLevel chain[VEB_CHAIN];
-    uint32_t nchain, chain_d;
-    uint8_t split[36];
 };
 
 struct VebEntry {
     uint32_t L, R, D;
 };
-
-// What tile_slot() looks up in LDS.  TILE_BTREE: level[z].  TILE_VEB: the
-// slots of the perfect trees of at most 8 levels, tree d's rank x at
-// small[2^d + x]: a rank of a tree of 2^16 keys takes one split and one
-// look-up instead of up to four splits.
-constexpr uint32_t SMALL_LEVELS = 8;
-template <int LAYOUT>
-struct SlotMap {
-    uint32_t level[32];
-};
-template <>
-struct SlotMap<TILE_VEB> {
-    uint8_t small[2u << SMALL_LEVELS];
-};
-
-// slot of rank x in the vEB (mveb_pos32 with the tables)
-__device__ inline uint32_t veb_slot(uint32_t x, const TileShape &s, const SlotMap<TILE_VEB> &m) {
-    uint32_t base = 0, d = s.chain_d;
-    for (uint32_t j = 0; j < s.nchain; j++) {
-        const VebLevel e = s.chain[j];
-        const uint32_t r = (1u << e.rd) - 1, l = (1u << e.ld) - 1, span = e.nf << e.ld;
-        if (x < span) {
-            const uint32_t k = x >> e.ld, c = x & l;
-            d = c == l ? e.rd : e.ld;
-            base += c == l ? 0u : r + k * l;
-            x = c == l ? k : c;
-            break;
-        }
-        if (x >= span + e.inc) {
-            x = e.nf + (x - span - e.inc);
-            d = e.rd;
-            break;
-        }
-        base += r + e.nf * l;
-        x -= span;
-    }
-    while (d > SMALL_LEVELS) {
-        const uint32_t rd = s.split[d], ld = d - rd, l = (1u << ld) - 1;
-        const uint32_t k = x >> ld, c = x & l;
-        base += c == l ? 0u : (1u << rd) - 1 + k * l;
-        d = c == l ? rd : ld;
-        x = c == l ? k : c;
-    }
-    return base + m.small[(1u << d) + x];
-}
-
-// slot of rank x in the layout; m.level[z]: first slot of the level whose keys'
-// internal ranks + 1 are divisible by (b + 1)^z and no more (TILE_BTREE)
-template <int LAYOUT>
-__device__ inline uint32_t tile_slot(uint32_t x, const TileShape &s, const SlotMap<LAYOUT> &m) {
-    if constexpr (LAYOUT == TILE_SORTED) {
-        return x;
-    } else if constexpr (LAYOUT == TILE_VEB) {
-        return veb_slot(x, s, m);
-    } else if constexpr (LAYOUT == TILE_BST) {
-        if (x < s.span) {
-            if (!(x & 1)) return s.nint + (x >> 1);
-            x >>= 1;
-        } else {
-            x -= s.nsep;
-        }
-        const uint32_t y = x + 1, z = (uint32_t)__clz((int)__brev(y));
-        return ((y | (1u << s.depth)) >> (z + 1)) - 1;
-    } else {
-        auto div = [&](uint32_t v) { return (uint32_t)__umul64hi(v, s.recip); };
-        const uint32_t k1 = s.b + 1;
-        if (x < s.span) {
-            const uint32_t row = div(x);
-            if (x - row * k1 < s.b) return s.nint + x - row;
-            x = row;
-        } else if (x < s.span + s.rem) {
-            return s.nint + x - s.nsep;
-        } else {
-            x -= s.span + s.rem - s.nsep;
-        }
-        uint32_t r = x + 1, z = 0, q = div(r);
-        while (r == q * k1) {
-            r = q;
-            q = div(r);
-            z++;
-        }
-        return m.level[z] + r - q - 1;
-    }
-}
-
-// fills the map (a workgroup of at least 64 lanes), ends with a barrier
-template <int LAYOUT>
-__device__ inline void slot_map(const TileShape &s, SlotMap<LAYOUT> &m) {
-    const uint32_t tid = threadIdx.x;
-    if constexpr (LAYOUT == TILE_BTREE) {
-        if (tid < s.depth) m.level[tid] = (uint32_t)(ipow64(s.b + 1, s.depth - 1 - tid) - 1);
-    }
-    if constexpr (LAYOUT == TILE_VEB) {
-        for (uint32_t i = tid + 2; i < (2u << SMALL_LEVELS); i += blockDim.x) {
-            const uint32_t d = 31u - (uint32_t)__clz((int)i), x = i - (1u << d);
-            m.small[i] = x < (1u << d) - 1
-                             ? (uint8_t)mveb_pos32(x, (1u << d) - 1, s.classic != 0)
-                             : (uint8_t)0;
-        }
-    }
-    __syncthreads();
-}
 
 // first rank of range j of 2^lg
 __device__ inline uint32_t range_first(uint32_t j, uint32_t n, uint32_t lg) {
@@ -408,7 +289,7 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
     {
         for (uint32_t i = tid; i < TILE_BINS; i += TILE_NT) {
             if (i == 0) continue;
-            spl[i] = A[tile_slot<LAYOUT>(range_first(heap_order(i, 10), s.n, 10), s, map)];
+            spl[i] = A[slot_of<LAYOUT>(range_first(heap_order(i, 10), s.n, 10), s, map)];
         }
         if constexpr (LAYOUT == TILE_VEB) {
             for (uint32_t i = tid; i < s.table_size; i += TILE_NT)
@@ -528,13 +409,7 @@ __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, Ti
     __shared__ SlotMap<LAYOUT> map;
     slot_map<LAYOUT>(s, map);
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < (1u << lg)) bound[j] = A[tile_slot<LAYOUT>(range_first(j, s.n, lg), s, map)];
-}
-
-// workgroup b's place in a grid of per * 8: XCD b % 8 takes one run of tiles
-__device__ inline uint32_t xcd_tile(uint32_t tiles) {
-    const uint32_t per = (tiles + 7) >> 3;
-    return (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (j < (1u << lg)) bound[j] = A[slot_of<LAYOUT>(range_first(j, s.n, lg), s, map)];
 }
 
 // what a tile of a pass is: queries [lo, hi) of the input, to be split at the
@@ -866,14 +741,14 @@ struct RangeSlots {
 // The m keys of ranks r0 .. : the first in heap[0], rank r0 + y at place y of
 // the heap of 2^depth - 1 nodes, the places past them the largest key.  All of
 // a lane's loads are issued before the first is stored.  The ranks' slots are
-// what this costs (with tile_slot() for every key the vector unit was busy for
+// what this costs (with slot_of() for every key the vector unit was busy for
 // three quarters of the time of a B-tree's ranges and all of a vEB's), so they
 // are found by what neighbours share:
 //   B-tree: all keys of a range on the leaf level (or the one above it) lie at
 //     rank - row + a constant, and rows follow from the place in the range by
-//     a 24-bit product; the separators between them take tile_slot().
+//     a 24-bit product; the separators between them take slot_of().
 //   vEB: 64 consecutive ranks share a bottom tree of 64 or more, which one
-//     lane finds for them; the root behind it takes tile_slot().
+//     lane finds for them; the root behind it takes slot_of().
 template <typename K, int LAYOUT>
 __device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape &s,
                                         const SlotMap<LAYOUT> &map, uint32_t r0, uint32_t m,
@@ -910,7 +785,7 @@ __device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape
             for (uint32_t k = 0; k < SEP; k++) {
                 const uint32_t i = k * RANGE_NT + tid;
                 if (i < seps) {
-                    const uint32_t slot = tile_slot<LAYOUT>(r0 + sep_at(i), s, map);
+                    const uint32_t slot = slot_of<LAYOUT>(r0 + sep_at(i), s, map);
                     w[k] = A[slot];
                     if (i < SEP_SLOTS) sep_slot[i] = slot;
                 }
@@ -931,7 +806,7 @@ __device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape
                 const uint32_t i = k * RANGE_NT + tid;
                 if (i < seps)
                     heap[heap_at(sep_at(i), depth)] =
-                        A[tile_slot<LAYOUT>(r0 + sep_at(i), s, map)];
+                        A[slot_of<LAYOUT>(r0 + sep_at(i), s, map)];
             }
             return {true, first, c0};
         }
@@ -1005,7 +880,7 @@ __device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape
 #pragma unroll
     for (uint32_t k = 0; k < PER; k++) {
         const uint32_t y = k * RANGE_NT + tid;
-        v[k] = y < m ? A[tile_slot<LAYOUT>(r0 + y, s, map)] : key_max<K>();
+        v[k] = y < m ? A[slot_of<LAYOUT>(r0 + y, s, map)] : key_max<K>();
     }
 #pragma unroll
     for (uint32_t k = 0; k < PER; k++) {
@@ -1088,8 +963,8 @@ __global__ __launch_bounds__(RANGE_NT) void k_part_answer(
                         if (LAYOUT == TILE_BTREE && rs.level && row < SEP_SLOTS)
                             ans = t - row * (s.b + 1) != s.b ? rs.first + x - row : sep_slot[row];
                         else
-                            ans = tile_slot<LAYOUT>(r0 + x, s, map);
-                        if (x == 0 && r0 > 0) again = A[tile_slot<LAYOUT>(r0 - 1, s, map)] == q;
+                            ans = slot_of<LAYOUT>(r0 + x, s, map);
+                        if (x == 0 && r0 > 0) again = A[slot_of<LAYOUT>(r0 - 1, s, map)] == q;
                         if (x + 1 < m) again |= heap[heap_at(x + 1, depth)] == q;
                     }
                     if (__any(again)) {
@@ -1110,46 +985,19 @@ __global__ __launch_bounds__(RANGE_NT) void k_part_answer(
 
 static TileShape tile_shape(const TileArray &a) {
     TileShape s{};
-    s.n = (uint32_t)a.n;
-    s.b = (uint32_t)a.b;
+    static_cast<SlotShape &>(s) = slot_shape(a.layout, a.n, a.b, a.classic);
     if (a.layout == TILE_BST || a.layout == TILE_BTREE) {
-        const uint32_t b = a.layout == TILE_BST ? 1u : s.b;
-        s.nodes = (uint32_t)((a.n + b - 1) / b);
-        s.levels = ilog_base(a.n + 1, b + 1);   // levels whose every node is whole
-        const BtreeShape bs = btree_shape(s.n, b);
-        s.nint = bs.nint;
-        s.span = bs.span;
-        s.rem = bs.rem;
-        s.nsep = bs.nsep;
-        s.depth = ilog_base((uint64_t)bs.nint + 1, b + 1);
-        s.recip = ~0ull / (b + 1) + 1;
+        s.nodes = (uint32_t)((a.n + s.b - 1) / s.b);
+        s.levels = ilog_base(a.n + 1, s.b + 1ull);   // levels whose every node is whole
         // exact below 2 RANGE_KEYS: 2^shift > 2 RANGE_KEYS (b + 1)
-        s.small_shift = floor_log2_64(2ull * RANGE_KEYS * (b + 1)) + 1;
-        s.small_mul = (uint32_t)(((1ull << s.small_shift) + b) / (b + 1));
-    }
-    if (a.layout == TILE_VEB) {
-        uint64_t n = a.n;
-        for (uint32_t d = 2; d <= 32; d++) {
-            uint32_t rd, ld;
-            veb_split(d, rd, ld, a.classic);
-            s.split[d] = (uint8_t)rd;
-        }
-        while (n & (n + 1)) {
-            VebLevel &e = s.chain[s.nchain++];
-            veb_split(floor_log2_64(n) + 1, e.rd, e.ld, a.classic);
-            const uint64_t r = (1ull << e.rd) - 1, l = (1ull << e.ld) - 1;
-            e.nf = (uint32_t)((n - r) / l);
-            e.inc = (uint32_t)(n - r - e.nf * l);
-            n = e.inc;
-        }
-        s.chain_d = n ? floor_log2_64(n) + 1 : 0;
+        s.small_shift = floor_log2_64(2ull * RANGE_KEYS * (s.b + 1)) + 1;
+        s.small_mul = (uint32_t)(((1ull << s.small_shift) + s.b) / (s.b + 1));
     }
     s.table_size = a.table_size;
     s.ntables = a.ntables;
     s.tables = a.tables;
     s.idx = a.idx;
     s.tidx = a.tidx;
-    s.classic = a.classic;
     return s;
 }
 

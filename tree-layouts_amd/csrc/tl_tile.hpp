@@ -3,10 +3,9 @@
 #pragma once
 
 #include "tl_internal.hpp"
+#include "tl_slots.hpp"
 
 namespace tl {
-
-enum TileLayout : uint32_t { TILE_BST, TILE_BTREE, TILE_VEB, TILE_SORTED };
 
 // one array as a lookup sees it.  tables / idx / tidx: the vEB query table
 // set (idx and tidx null for a perfect tree of one table)
