@@ -66,6 +66,13 @@ int emu_shfl_up(int v, unsigned d) {
     emu_ballot(true);
     return r;
 }
+int emu_shfl_xor(int v, int m) {
+    g_shfl[t_lane] = v;
+    emu_ballot(true);
+    const int r = g_shfl[t_lane / 64 * 64 + ((t_lane % 64) ^ m)];
+    emu_ballot(true);
+    return r;
+}
 // every lane of the wave calls it
 int emu_readlane(int v, int lane) {
     g_shfl[t_lane] = v;

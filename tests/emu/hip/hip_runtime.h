@@ -38,13 +38,15 @@ unsigned char *emu_smem();
 #define __ballot(p) emu_ballot((p))
 #define __any(p) (emu_ballot((p)) != 0)
 int emu_shfl_up(int v, unsigned d);
+int emu_shfl_xor(int v, int m);
+#define __shfl_xor(v, m) emu_shfl_xor((v), (m))
 int emu_readlane(int v, int lane);
 #define __builtin_amdgcn_readlane(v, l) emu_readlane((v), (l))
 #define __shfl_up(v, d) emu_shfl_up((v), (d))
 #define __builtin_amdgcn_s_sleep(n) emu_sleep()
 #define __builtin_amdgcn_fence(o, s) __atomic_thread_fence(__ATOMIC_SEQ_CST)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
-#define __builtin_amdgcn_wave_barrier() ((void)0)
+#define __builtin_amdgcn_wave_barrier() ((void)emu_ballot(true))
 inline uint64_t wall_clock64() { return emu_clock(); }
 
 #define __HIP_MEMORY_SCOPE_WAVEFRONT 1

@@ -3,6 +3,20 @@
 // the sorted, distinct input every layout assumes (the reference's drivers
 // build such input themselves, cpu/src/common.h:33-40).
 //
+// Splitter sort.  The keys are partitioned into buckets of about 1000 by
+// splitters from samples, in one pass (1024 buckets) or two, each a count and
+// a scatter whose tile leaves LDS in bucket order; a bucket is then sorted in
+// LDS by one workgroup and its repeats dropped, and one pass closes the gaps.
+// Whatever the key width and range, every key moves four times (the digits of
+// a radix sort move it once per 8 bits that vary: 100 million 40-bit keys took
+// five passes at 1.0 ms and 6.2 ms in all; now 3.1 ms, as many of 62 bits).  A key equal to a splitter is not partitioned but
+// noted with it, so a key that repeats often costs nothing, however often.
+//
+// Bucket sizes are the samples' luck.  Where one does not fit (it never has,
+// by the samples' numbers), nothing has been lost: the partitioned keys and
+// the noted splitters are the input's distinct keys and some repeats, and the
+// radix sort below takes over from them.  It also serves the largest arrays.
+//
 // LSD radix sort, 8-bit digits, stable, ping-ponging between the caller's
 // array and one library-owned buffer of n keys.  Signed keys sort by their
 // bits with the sign bit flipped.  A pass whose digit is the same for every
@@ -20,10 +34,14 @@
 // memory, so equal digits keep their order (the sort is stable).
 // Duplicates: every sorted key that differs from its predecessor is kept;
 // a count per tile, a scan, and a compaction into the other buffer.
+#include <stdlib.h>
+
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "tl_internal.hpp"
+#include "tl_partition.hpp"
 #include "tl_plan.hpp"
 
 namespace tl {
@@ -273,6 +291,635 @@ static tl_status scan_u32(uint32_t *v, uint64_t len, uint32_t *sums, hipStream_t
     return TL_OK;
 }
 
+// ---------------------------------------------------------------------------
+// the splitter sort
+
+constexpr uint32_t RANGE_NT = 512, RANGE_IT = 8;
+constexpr uint32_t RANGE_CAP = RANGE_NT * RANGE_IT;   // keys of a bucket, at most
+constexpr uint32_t RANGE_GOAL = 1536;                 // ... on average
+constexpr uint32_t RANGE_BINS = 2048;
+constexpr uint32_t SORT_LG1 = 8;   // log2 of the first of two passes' buckets
+constexpr uint64_t SPLIT_MAX_KEYS = 1ull << 29;       // 2^10 and 2^9 buckets
+
+template <typename K>
+using Bits = typename std::conditional<sizeof(K) == 4, uint32_t, uint64_t>::type;
+// the key's bits in its own order, and back
+template <typename K>
+__device__ inline Bits<K> to_bits(K k) {
+    const Bits<K> top = (K)-1 < (K)0 ? (Bits<K>)1 << (8 * sizeof(K) - 1) : 0;
+    return (Bits<K>)k ^ top;
+}
+template <typename K>
+__device__ inline K from_bits(Bits<K> u) {
+    const Bits<K> top = (K)-1 < (K)0 ? (Bits<K>)1 << (8 * sizeof(K) - 1) : 0;
+    return (K)(u ^ top);
+}
+
+// sorts buf[0 .. cnt) in LDS, cnt <= NT * IT: LSD radix over the 8-bit digits
+// that vary.  hist: NT / 64 * 256 words
+template <typename U, uint32_t NT, uint32_t IT>
+__device__ inline void lds_sort(U *buf, uint32_t cnt, uint32_t *hist, uint32_t *wsum) {
+    __shared__ uint32_t vary_lo, vary_hi;
+    constexpr uint32_t NW = NT / 64;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint64_t lt = (1ull << lane) - 1;
+    if (tid == 0) vary_lo = vary_hi = 0;
+    __syncthreads();
+    uint64_t vary = 0;
+    for (uint32_t i = tid; i < cnt; i += NT) vary |= (uint64_t)(buf[i] ^ buf[0]);
+    if ((uint32_t)vary) atomicOr(&vary_lo, (uint32_t)vary);
+    if (vary >> 32) atomicOr(&vary_hi, (uint32_t)(vary >> 32));
+    __syncthreads();
+    vary = (uint64_t)vary_hi << 32 | vary_lo;
+    const uint32_t items = (cnt + NT - 1) / NT;   // slots of a lane, in memory order
+    for (uint32_t shift = 0; shift < 8 * sizeof(U); shift += 8) {
+        if (((vary >> shift) & 0xFF) == 0) continue;
+        for (uint32_t i = tid; i < NW * 256; i += NT) hist[i] = 0;
+        __syncthreads();
+        U x[IT];
+        uint32_t rank[IT];
+#pragma unroll
+        for (uint32_t k = 0; k < IT; k++) {
+            if (k >= items) continue;
+            const uint32_t i = (w * items + k) * 64 + lane;
+            const bool valid = i < cnt;
+            x[k] = valid ? buf[i] : (U)0;
+            const uint32_t d = (uint32_t)(x[k] >> shift) & 0xFF;
+            uint64_t peers = __ballot(valid);
+#pragma unroll
+            for (uint32_t bit = 0; bit < 8; bit++) {
+                const bool on = (d >> bit) & 1u;
+                const uint64_t m = __ballot(on);
+                peers &= on ? m : ~m;
+            }
+            rank[k] = valid ? hist[w * 256 + d] + (uint32_t)__popcll(peers & lt) : 0u;
+            __builtin_amdgcn_wave_barrier();
+            if (valid && (peers & lt) == 0) hist[w * 256 + d] += (uint32_t)__popcll(peers);
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        // starts of (digit, wave) in digit order, then wave order
+        uint32_t sum = 0;
+        if (tid < 256)
+            for (uint32_t ww = 0; ww < NW; ww++) sum += hist[ww * 256 + tid];
+        uint32_t total;
+        uint32_t run = block_scan(sum, wsum, &total);
+        if (tid < 256)
+            for (uint32_t ww = 0; ww < NW; ww++) {
+                const uint32_t c = hist[ww * 256 + tid];
+                hist[ww * 256 + tid] = run;
+                run += c;
+            }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < IT; k++) {
+            const uint32_t i = (w * items + k) * 64 + lane;
+            if (k < items && i < cnt)
+                buf[hist[w * 256 + ((uint32_t)(x[k] >> shift) & 0xFF)] + rank[k]] = x[k];
+        }
+        __syncthreads();
+    }
+}
+
+// place of sample i of `samples` among count items: one of each equal share, at
+// a place that does not follow a stride of the data
+__device__ inline uint64_t sample_at(uint32_t i, uint32_t samples, uint64_t count) {
+    const uint64_t lo = (uint64_t)i * count / samples, hi = (uint64_t)(i + 1) * count / samples;
+    return hi > lo ? lo + (uint64_t)(i * 2654435761u) % (hi - lo) : lo;
+}
+
+// bound[j << lg2], j < 2^lg1: the first pass's splitters (one workgroup), or
+// with SECOND bound[k << lg2 | o], 0 < o < 2^lg2: those of bucket k, a
+// workgroup each
+template <typename K, bool SECOND, uint32_t IT>
+__global__ __launch_bounds__(1024) void k_sort_sample(const K *__restrict__ keys, uint64_t n,
+                                                      uint32_t lg1, uint32_t lg2,
+                                                      const uint32_t *__restrict__ bstart,
+                                                      K *__restrict__ bound) {
+    constexpr uint32_t SAMPLES = 1024 * IT;
+    __shared__ Bits<K> buf[SAMPLES];
+    __shared__ uint32_t hist[16 * 256], wsum[16];
+    const uint64_t lo = SECOND ? bstart[blockIdx.x] : 0;
+    const uint64_t count = SECOND ? bstart[blockIdx.x + 1] - lo : n;
+    if (SECOND && count == 0) {   // no key meets these
+        for (uint32_t o = threadIdx.x + 1; o < (1u << lg2); o += 1024)
+            bound[((uint64_t)blockIdx.x << lg2) + o] = bound[(uint64_t)blockIdx.x << lg2];
+        return;
+    }
+    for (uint32_t i = threadIdx.x; i < SAMPLES; i += 1024)
+        buf[i] = to_bits<K>(keys[lo + sample_at(i, SAMPLES, count)]);
+    __syncthreads();
+    lds_sort<Bits<K>, 1024, IT>(buf, SAMPLES, hist, wsum);
+    if (SECOND) {
+        for (uint32_t o = threadIdx.x + 1; o < (1u << lg2); o += 1024)
+            bound[((uint64_t)blockIdx.x << lg2) + o] =
+                from_bits<K>(buf[(uint64_t)o * SAMPLES >> lg2]);
+    } else {
+        for (uint32_t j = threadIdx.x; j < (1u << lg1); j += 1024)
+            bound[(uint64_t)j << lg2] = from_bits<K>(buf[(uint64_t)j * SAMPLES >> lg1]);
+    }
+}
+
+// the tile's splitters in heap order (node 0 unused), and bucket by bucket
+template <typename K, bool SECOND>
+__device__ inline void sort_splitters(const K *__restrict__ bound, const PartTile &p, uint32_t lg1,
+                                      uint32_t lg2, K *spl, K *low) {
+    const uint32_t lg = SECOND ? lg2 : lg1, step = SECOND ? 1u : 1u << lg2;
+    if (threadIdx.x < (1u << lg)) {
+        low[threadIdx.x] = bound[p.first + (uint64_t)threadIdx.x * step];
+        if (threadIdx.x)
+            spl[threadIdx.x] = bound[p.first + (uint64_t)heap_order(threadIdx.x, lg) * step];
+    }
+}
+
+// bucket of each key, and whether the key equals the bucket's splitter (the
+// first bucket of all has none)
+template <typename K, int IT>
+__device__ inline void sort_buckets(const K (&q)[IT], const K *spl, const K *low, uint32_t first,
+                                    uint32_t lg, uint32_t (&bin)[IT], bool (&eq)[IT]) {
+#pragma unroll
+    for (int k = 0; k < IT; k++) bin[k] = 1;
+    for (uint32_t l = 0; l < lg; l++) {
+#pragma unroll
+        for (int k = 0; k < IT; k++) bin[k] = 2 * bin[k] + (q[k] >= spl[bin[k]] ? 1u : 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        bin[k] -= 1u << lg;
+        eq[k] = q[k] == low[bin[k]] && (first + bin[k]) != 0;
+    }
+}
+
+template <typename K, bool SECOND, int IT>
+__global__ __launch_bounds__(PART_NT) void k_sort_count(
+    const K *__restrict__ keys, uint64_t n, const K *__restrict__ bound, uint32_t lg1,
+    uint32_t lg2, const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart,
+    uint32_t tiles, uint32_t *__restrict__ counts, uint32_t *__restrict__ present) {
+    __shared__ K spl[PART_BINS], low[PART_BINS];
+    __shared__ uint32_t cnt[PART_BINS];
+    const uint32_t lg = SECOND ? lg2 : lg1, B = 1u << lg, t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, n, PART_NT * IT, lg1, lg2, bstart, tstart);
+    K q[IT];
+    uint32_t bin[IT];
+    bool eq[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + threadIdx.x;
+        q[k] = i < p.hi ? keys[i] : K{};
+    }
+    if (threadIdx.x < B) cnt[threadIdx.x] = 0;
+    sort_splitters<K, SECOND>(bound, p, lg1, lg2, spl, low);
+    __syncthreads();
+    sort_buckets<K, IT>(q, spl, low, p.first, lg, bin, eq);
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        if (p.lo + k * PART_NT + threadIdx.x < p.hi) {
+            if (eq[k])
+                present[SECOND ? p.first + bin[k] : bin[k] << lg2] = 1;
+            else
+                atomicAdd(&cnt[bin[k]], 1u);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < B) counts[(uint64_t)t * B + threadIdx.x] = cnt[threadIdx.x];
+}
+
+// every key that equals no splitter to its bucket, the tile in bucket order in
+// LDS first (the places, then the keys), so that it is written in runs
+template <typename K, bool SECOND, int IT>
+__global__ __launch_bounds__(PART_NT) void k_sort_scatter(
+    const K *__restrict__ keys, uint64_t n, const K *__restrict__ bound, uint32_t lg1,
+    uint32_t lg2, const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart,
+    uint32_t tiles, const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
+    K *__restrict__ out) {
+    __shared__ K stage[PART_NT * IT];
+    __shared__ uint32_t at[PART_BINS], local[PART_BINS];
+    __shared__ uint32_t wsum[PART_NT / 64];
+    K *spl = stage, *low = stage + PART_BINS;   // read before the stage is written
+    uint32_t *stage_to = reinterpret_cast<uint32_t *>(stage);
+    const uint32_t lg = SECOND ? lg2 : lg1, B = 1u << lg, tid = threadIdx.x, t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, n, PART_NT * IT, lg1, lg2, bstart, tstart);
+    K q[IT];
+    uint32_t bin[IT], to[IT];
+    bool eq[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        q[k] = i < p.hi ? keys[i] : K{};
+    }
+    sort_splitters<K, SECOND>(bound, p, lg1, lg2, spl, low);
+    const uint32_t mine = tid < B ? counts[(uint64_t)t * B + tid] : 0u;
+    uint32_t total;
+    const uint32_t before = block_scan(mine, wsum, &total);
+    if (tid < B) {
+        local[tid] = before;
+        at[tid] = places[(uint64_t)t * B + tid] - before;
+    }
+    __syncthreads();
+    sort_buckets<K, IT>(q, spl, low, p.first, lg, bin, eq);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        eq[k] |= p.lo + k * PART_NT + tid >= p.hi;   // not moved
+        if (!eq[k]) {
+            const uint32_t x = atomicAdd(&local[bin[k]], 1u);
+            stage_to[x] = at[bin[k]] + x;
+            bin[k] = x;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        to[k] = x < total ? stage_to[x] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++)
+        if (!eq[k]) stage[bin[k]] = q[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        if (x < total) out[to[k]] = stage[x];
+    }
+}
+
+// smallest / largest value of a wave, in every lane
+template <typename U, bool LARGEST>
+__device__ inline U wave_extreme(U v) {
+    for (int o = 1; o < 64; o <<= 1) {
+        U other = (U)(uint32_t)__shfl_xor((int)(uint32_t)v, o);
+        if constexpr (sizeof(U) == 8)
+            other |= (U)(uint32_t)__shfl_xor((int)(uint32_t)((uint64_t)v >> 32), o) << 32;
+        v = LARGEST ? max(v, other) : min(v, other);
+    }
+    return v;
+}
+
+// Bucket j (rcount[j] keys at S[rstart[j]]) sorted in LDS, its distinct keys to
+// the same place of out (which may be S), their number plus the splitter's
+// presence to kept[j].  One counting pass over 2048 equal parts of the bucket's
+// span leaves a key or two in each, which find their order by comparing.
+// Buckets whose keys crowd are left (kept[j] = CROWDED) to a second launch,
+// which sorts all their digits (and needs the registers for it).
+constexpr uint32_t CROWDED = ~0u;
+template <typename K, bool CROWD_PASS>
+__global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
+                                                         const uint32_t *__restrict__ rstart,
+                                                         const uint32_t *__restrict__ rcount,
+                                                         const uint32_t *__restrict__ present,
+                                                         K *out, uint32_t *__restrict__ kept,
+                                                         uint32_t *__restrict__ overflow) {
+    using U = Bits<K>;
+    constexpr uint32_t CROWD = 32, NW = RANGE_NT / 64;
+    __shared__ U buf[RANGE_CAP];
+    __shared__ uint32_t bins[RANGE_BINS + 1], wsum[NW], wcount[RANGE_IT * NW];
+    __shared__ U span[2 * NW];
+    __shared__ uint32_t crowded;
+    if (CROWD_PASS && kept[blockIdx.x] != CROWDED) return;
+    const uint32_t j = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint32_t lo = rstart[j], cnt = rcount[j];
+    if (cnt == 0 || cnt > RANGE_CAP) {
+        if (tid == 0) {
+            kept[j] = present[j];
+            if (cnt) *overflow = 1;
+        }
+        return;
+    }
+    U x[RANGE_IT];
+    uint32_t place[RANGE_IT];
+    if (tid == 0) crowded = 0;
+    for (uint32_t i = tid; i <= RANGE_BINS; i += RANGE_NT) bins[i] = 0;
+    U least = ~(U)0, most = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < RANGE_IT; k++) {
+        if (k * RANGE_NT >= cnt) continue;   // the whole workgroup's, here and below
+        const uint32_t i = k * RANGE_NT + tid;
+        if (i < cnt) {
+            x[k] = to_bits<K>(S[lo + i]);
+            least = min(least, x[k]);
+            most = max(most, x[k]);
+        }
+    }
+    least = wave_extreme<U, false>(least);
+    most = wave_extreme<U, true>(most);
+    if (lane == 0) {
+        span[w] = least;
+        span[NW + w] = most;
+    }
+    __syncthreads();
+    for (uint32_t ww = 0; ww < NW; ww++) {
+        least = min(least, span[ww]);
+        most = max(most, span[NW + ww]);
+    }
+    const U first = least;
+    const uint64_t width = most - least;
+    const uint32_t bits = width ? 64u - (uint32_t)__clzll((long long)width) : 0u;
+    const uint32_t shift = bits > 11 ? bits - 11 : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < RANGE_IT; k++) {
+        if (k * RANGE_NT >= cnt) continue;
+        if (k * RANGE_NT + tid < cnt)
+            place[k] = atomicAdd(&bins[(uint32_t)((U)(x[k] - first) >> shift)], 1u);
+    }
+    __syncthreads();
+    {
+        constexpr uint32_t PER = RANGE_BINS / RANGE_NT;
+        uint32_t c[PER], sum = 0, top = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < PER; k++) {
+            c[k] = bins[tid * PER + k];
+            sum += c[k];
+            top = max(top, c[k]);
+        }
+        if (top > CROWD && shift) crowded = 1;
+        uint32_t total;
+        uint32_t run = block_scan(sum, wsum, &total);
+#pragma unroll
+        for (uint32_t k = 0; k < PER; k++) {
+            bins[tid * PER + k] = run;
+            run += c[k];
+        }
+        if (tid == 0) bins[RANGE_BINS] = cnt;
+    }
+    __syncthreads();
+    if (!CROWD_PASS && crowded) {
+        if (tid == 0) kept[j] = CROWDED;
+        return;
+    }
+    if constexpr (CROWD_PASS) {
+#pragma unroll
+        for (uint32_t k = 0; k < RANGE_IT; k++) {
+            const uint32_t i = k * RANGE_NT + tid;
+            if (i < cnt) buf[i] = x[k];
+        }
+        __syncthreads();
+        lds_sort<U, RANGE_NT, RANGE_IT>(buf, cnt, bins, wsum);
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < RANGE_IT; k++) {
+            if (k * RANGE_NT >= cnt) continue;
+            if (k * RANGE_NT + tid < cnt) {
+                place[k] += bins[(uint32_t)((U)(x[k] - first) >> shift)];
+                buf[place[k]] = x[k];
+            }
+        }
+        __syncthreads();
+    }
+    if (!CROWD_PASS && shift) {   // a part holds keys that differ
+#pragma unroll
+        for (uint32_t k = 0; k < RANGE_IT; k++) {
+            if (k * RANGE_NT >= cnt) continue;
+            if (k * RANGE_NT + tid < cnt) {
+                const uint32_t b = (uint32_t)((U)(x[k] - first) >> shift);
+                const uint32_t s0 = bins[b], s1 = bins[b + 1];
+                uint32_t at = s0;
+                for (uint32_t i = s0; i < s1; i++) {
+                    const U y = buf[i];
+                    at += y < x[k] || (y == x[k] && i < place[k]) ? 1u : 0u;
+                }
+                place[k] = at;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < RANGE_IT; k++) {
+            if (k * RANGE_NT >= cnt) continue;
+            if (k * RANGE_NT + tid < cnt) buf[place[k]] = x[k];
+        }
+        __syncthreads();
+    }
+    // distinct keys in order: 64 at a time, (k, wave) after (k, wave)
+    bool keep[RANGE_IT];
+#pragma unroll
+    for (uint32_t k = 0; k < RANGE_IT; k++) {
+        keep[k] = false;
+        if (k * RANGE_NT >= cnt) {
+            if (lane == 0) wcount[k * NW + w] = 0;
+            continue;
+        }
+        const uint32_t i = k * RANGE_NT + tid;
+        keep[k] = i < cnt;
+        if (keep[k]) {
+            x[k] = buf[i];
+            keep[k] = i == 0 || x[k] != buf[i - 1];
+        }
+        const uint64_t m = __ballot(keep[k]);
+        place[k] = (uint32_t)__popcll(m & ((1ull << lane) - 1));
+        if (lane == 0) wcount[k * NW + w] = (uint32_t)__popcll(m);
+    }
+    __syncthreads();
+    static_assert(RANGE_IT * NW <= 64, "one count a lane of a wave");
+    uint32_t total;
+    const uint32_t mine = tid < RANGE_IT * NW ? wcount[tid] : 0u;
+    const uint32_t before = block_scan(mine, wsum, &total);
+    if (tid < RANGE_IT * NW) wcount[tid] = before;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < RANGE_IT; k++) {
+        if (k * RANGE_NT >= cnt) continue;
+        if (keep[k]) out[lo + wcount[k * NW + w] + place[k]] = from_bits<K>(x[k]);
+    }
+    if (tid == 0) kept[j] = total + present[j];
+}
+
+// the distinct keys of bucket j, behind its splitter where present, to
+// off[j] .. of the result
+template <typename K>
+__global__ __launch_bounds__(256) void k_sort_close(const K *__restrict__ T,
+                                                    const uint32_t *__restrict__ rstart,
+                                                    const uint32_t *__restrict__ present,
+                                                    const K *__restrict__ bound,
+                                                    const uint32_t *__restrict__ off,
+                                                    uint32_t ranges, const uint32_t *sum,
+                                                    const uint32_t *__restrict__ overflow,
+                                                    K *__restrict__ keys) {
+    if (*overflow) return;
+    const uint32_t j = blockIdx.x, o = off[j], lo = rstart[j], pre = present[j];
+    const uint32_t c = (j + 1 < ranges ? off[j + 1] : *sum) - o - pre;
+    if (pre && threadIdx.x == 0) keys[o] = bound[j];
+    for (uint32_t i = threadIdx.x; i < c; i += 256) keys[o + pre + i] = T[lo + i];
+}
+
+// After an overflow: the splitters present back among the keys.  The first
+// pass's go behind the *count partitioned keys; the second pass's into the gap
+// that their keys left at the end of their bucket (what else the gap holds is
+// still keys of the input).
+template <typename K>
+__global__ __launch_bounds__(1024) void k_sort_append(const uint32_t *__restrict__ present,
+                                                      const K *__restrict__ bound, uint32_t lg1,
+                                                      uint32_t lg2,
+                                                      const uint32_t *__restrict__ rstart,
+                                                      const uint32_t *__restrict__ rcount, K *dst,
+                                                      uint32_t *count) {
+    const uint32_t k = threadIdx.x, B2 = 1u << lg2;
+    if (k >= (1u << lg1)) return;
+    const uint32_t j0 = k << lg2, last = j0 + B2 - 1;
+    if (present[j0]) dst[atomicAdd(count, 1u)] = bound[j0];
+    uint32_t at = rstart[last] + rcount[last];
+    for (uint32_t j = j0 + 1; j <= last; j++)
+        if (present[j]) dst[at++] = bound[j];
+}
+
+__global__ void k_sort_range_of(uint32_t *rstart, uint32_t n, uint32_t *rcount,
+                                uint32_t *present) {
+    *rstart = 0;
+    *rcount = n;
+    *present = 0;
+}
+
+template <typename K, bool SECOND, int IT>
+static void sort_pass(const K *in, K *out, uint64_t n, uint32_t lg1, uint32_t lg2, uint32_t tiles,
+                      uint32_t groups, const K *bound, uint32_t *bstart, uint32_t *tstart,
+                      uint32_t *rstart, uint32_t *rcount, uint32_t *gsum, uint32_t *counts,
+                      uint32_t *places, uint32_t *present, hipStream_t s) {
+    const dim3 grid((tiles + 7) / 8 * 8), block(PART_NT);
+    hipLaunchKernelGGL((k_sort_count<K, SECOND, IT>), grid, block, 0, s, in, n, bound, lg1, lg2,
+                       (const uint32_t *)bstart, (const uint32_t *)tstart, tiles, counts, present);
+    if (SECOND) {
+        hipLaunchKernelGGL(k_part_places2, dim3(1u << lg1), block, 0, s, (const uint32_t *)counts,
+                           lg1, lg2, (const uint32_t *)bstart, (const uint32_t *)tstart, places,
+                           rstart, rcount);
+    } else {
+        hipLaunchKernelGGL(k_part_sums, dim3(groups), block, 0, s, (const uint32_t *)counts,
+                           1u << lg1, tiles, gsum);
+        hipLaunchKernelGGL(k_part_starts, dim3(1), block, 0, s, gsum, 1u << lg1, groups,
+                           (uint32_t)(PART_NT * IT), bstart, tstart, lg2 ? (uint32_t *)nullptr : rcount);
+        hipLaunchKernelGGL(k_part_places, dim3(groups), block, 0, s, (const uint32_t *)counts,
+                           1u << lg1, tiles, (const uint32_t *)gsum, (const uint32_t *)bstart,
+                           places);
+    }
+    hipLaunchKernelGGL((k_sort_scatter<K, SECOND, IT>), grid, block, 0, s, in, n, bound, lg1, lg2,
+                       (const uint32_t *)bstart, (const uint32_t *)tstart, tiles,
+                       (const uint32_t *)places, (const uint32_t *)counts, out);
+}
+
+template <typename K>
+static void sort_ranges(const K *S, const uint32_t *rstart, const uint32_t *rcount,
+                        const uint32_t *present, K *out, uint32_t *kept, uint32_t *overflow,
+                        uint32_t ranges, hipStream_t s) {
+    hipLaunchKernelGGL((k_sort_range<K, false>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
+                       rcount, present, out, kept, overflow);
+    hipLaunchKernelGGL((k_sort_range<K, true>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
+                       rcount, present, out, kept, overflow);
+}
+
+template <typename U>
+static tl_status sort_dedupe_t(Ctx *c, U *keys, uint64_t n, U flip, uint64_t *n_out, hipStream_t s);
+
+// sorts and drops repeats; n <= SPLIT_MAX_KEYS
+template <typename K>
+static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStream_t s) {
+    if (n <= 1) {
+        *n_out = n;
+        return TL_OK;
+    }
+    uint32_t lg = 1;
+    while ((n >> lg) >= RANGE_GOAL) lg++;
+    // few enough splitters a pass for their samples (32 and 64 each): a
+    // bucket's size is then the goal's within a factor of 2.4
+    const uint32_t lg1 = lg <= PART_LG ? lg : lg > SORT_LG1 + 9 ? lg - 9 : SORT_LG1;
+    const uint32_t lg2 = lg - lg1, ranges = 1u << lg;
+    const bool wide = n >= (1u << 22);   // queries per lane of a tile: 16, else 4
+    const uint64_t T = (uint64_t)PART_NT * (wide ? 16 : 4);
+    const uint32_t tiles1 = (uint32_t)((n + T - 1) / T), tiles2 = lg2 ? tiles1 + (1u << lg1) : 0;
+    const uint32_t groups = (tiles1 + PART_GROUP - 1) / PART_GROUP;
+    const uint64_t cells = std::max((uint64_t)tiles1 << lg1, (uint64_t)tiles2 << lg2);
+    // words of scratch slot 5: overflow and a count, bstart, tstart, rstart,
+    // rcount, present, kept and the sums of its scan, gsum, counts, places; then
+    // the splitters
+    const uint64_t B1 = (1ull << lg1) + 1, sums = ranges / SCAN_CHUNK + 3;
+    uint64_t words = 2 + 2 * B1 + (ranges + 1ull) + 3ull * ranges + sums +
+                     ((uint64_t)groups << lg1) + 2 * cells;
+    words = (words + 1) & ~1ull;
+    uint32_t *m = nullptr;
+    TL_TRY(scratch(c, 5, words * 4 + (size_t)ranges * sizeof(K), (void **)&m));
+    uint32_t *overflow = m, *count = m + 1, *bstart = m + 2, *tstart = bstart + B1;
+    uint32_t *rstart = lg2 ? tstart + B1 : bstart, *rcount = tstart + B1 + ranges + 1;
+    uint32_t *present = rcount + ranges;
+    uint32_t *kept = present + ranges, *ksum = kept + ranges, *gsum = ksum + sums;
+    uint32_t *counts = gsum + ((uint64_t)groups << lg1), *places = counts + cells;
+    K *bound = (K *)(m + words);
+    if (n <= RANGE_CAP) {   // one bucket, sorted where it is
+        hipLaunchKernelGGL(k_sort_range_of, dim3(1), dim3(1), 0, s, bstart, (uint32_t)n, rcount,
+                           present);
+        sort_ranges<K>(keys, bstart, rcount, present, keys, kept, overflow, 1, s);
+        TL_LAUNCH_CHECK();
+        uint32_t u = 0;
+        TL_HIP(hipMemcpyAsync(&u, kept, 4, hipMemcpyDeviceToHost, s));
+        TL_HIP(hipStreamSynchronize(s));
+        *n_out = u;
+        return TL_OK;
+    }
+    K *tmp = nullptr;
+    TL_TRY(scratch(c, 4, n * sizeof(K), (void **)&tmp));
+    TL_TRY(fill_u32_launch(m, 2, 0, s));
+    TL_TRY(fill_u32_launch(present, ranges, 0, s));
+    if (lg1 <= 8)
+        hipLaunchKernelGGL((k_sort_sample<K, false, 8>), dim3(1), dim3(1024), 0, s,
+                           (const K *)keys, n, lg1, lg2, (const uint32_t *)nullptr, bound);
+    else
+        hipLaunchKernelGGL((k_sort_sample<K, false, 16>), dim3(1), dim3(1024), 0, s,
+                           (const K *)keys, n, lg1, lg2, (const uint32_t *)nullptr, bound);
+    TL_LAUNCH_CHECK();
+    K *sorted = tmp, *other = keys;   // the partitioned keys, and the other buffer
+#define TL_SORT_PASS(SECOND, IT, in, out, tiles)                                                   \
+    sort_pass<K, SECOND, IT>(in, out, n, lg1, lg2, tiles, groups, bound, bstart, tstart, rstart,   \
+                             rcount, gsum, counts, places, present, s)
+    if (wide) TL_SORT_PASS(false, 16, keys, tmp, tiles1);
+    else TL_SORT_PASS(false, 4, keys, tmp, tiles1);
+    TL_LAUNCH_CHECK();
+    if (lg2) {
+        if (lg2 <= 6)
+            hipLaunchKernelGGL((k_sort_sample<K, true, 4>), dim3(1u << lg1), dim3(1024), 0, s,
+                               (const K *)tmp, n, lg1, lg2, (const uint32_t *)bstart, bound);
+        else
+            hipLaunchKernelGGL((k_sort_sample<K, true, 16>), dim3(1u << lg1), dim3(1024), 0, s,
+                               (const K *)tmp, n, lg1, lg2, (const uint32_t *)bstart, bound);
+        if (wide) TL_SORT_PASS(true, 16, tmp, keys, tiles2);
+        else TL_SORT_PASS(true, 4, tmp, keys, tiles2);
+        TL_LAUNCH_CHECK();
+        std::swap(sorted, other);
+    }
+#undef TL_SORT_PASS
+    sort_ranges<K>(sorted, rstart, rcount, present, other, kept, overflow, ranges, s);
+    TL_LAUNCH_CHECK();
+    TL_TRY(scan_u32(kept, ranges, ksum, s));
+    const uint32_t *sum = ksum + (ranges + SCAN_CHUNK - 1) / SCAN_CHUNK;
+    // close the gaps into the buffer that held the partitioned keys
+    hipLaunchKernelGGL(k_sort_close<K>, dim3(ranges), dim3(256), 0, s, (const K *)other,
+                       (const uint32_t *)rstart, (const uint32_t *)present, (const K *)bound,
+                       (const uint32_t *)kept, ranges, sum, (const uint32_t *)overflow, sorted);
+    TL_LAUNCH_CHECK();
+    uint32_t h[3];   // overflow; keys partitioned (and the second pass's gaps); distinct keys
+    TL_HIP(hipMemcpyAsync(&h[0], overflow, 4, hipMemcpyDeviceToHost, s));
+    TL_HIP(hipMemcpyAsync(&h[1], bstart + (1u << lg1), 4, hipMemcpyDeviceToHost, s));
+    TL_HIP(hipMemcpyAsync(&h[2], sum, 4, hipMemcpyDeviceToHost, s));
+    TL_HIP(hipStreamSynchronize(s));
+    const uint64_t have = h[0] ? h[1] : h[2];
+    if (sorted != keys && have)
+        TL_HIP(hipMemcpyAsync(keys, sorted, have * sizeof(K), hipMemcpyDeviceToDevice, s));
+    if (!h[0]) {
+        *n_out = h[2];
+        return TL_OK;
+    }
+    // a bucket was too large: the partitioned keys and the splitters present
+    // hold every distinct key
+    TL_TRY(fill_u32_launch(count, 1, h[1], s));
+    hipLaunchKernelGGL(k_sort_append<K>, dim3(1), dim3(1024), 0, s, (const uint32_t *)present,
+                       (const K *)bound, lg1, lg2, (const uint32_t *)rstart,
+                       (const uint32_t *)rcount, keys, count);
+    TL_LAUNCH_CHECK();
+    uint32_t left = 0;
+    TL_HIP(hipMemcpyAsync(&left, count, 4, hipMemcpyDeviceToHost, s));
+    TL_HIP(hipStreamSynchronize(s));
+    const Bits<K> flip = (K)-1 < (K)0 ? (Bits<K>)1 << (8 * sizeof(K) - 1) : 0;
+    return sort_dedupe_t<Bits<K>>(c, (Bits<K> *)keys, left, flip, n_out, s);
+}
+
 template <typename U>
 static tl_status sort_dedupe_t(Ctx *c, U *keys, uint64_t n, U flip, uint64_t *n_out,
                                hipStream_t s) {
@@ -356,7 +1003,14 @@ extern "C" tl_status tl_sort_dedupe(void *dev_keys, uint64_t n, tl_dtype dtype, 
     Timer tm;
     TL_TRY(tm.start(s, ms));
     tl_status st;
-    if (W == 4) {
+    if (n <= SPLIT_MAX_KEYS && !(getenv("TL_SORT_RADIX") && atoi(getenv("TL_SORT_RADIX")) == 1)) {
+        switch (dtype) {
+        case TL_U32: st = split_sort<uint32_t>(c, (uint32_t *)dev_keys, n, n_out, s); break;
+        case TL_U64: st = split_sort<uint64_t>(c, (uint64_t *)dev_keys, n, n_out, s); break;
+        case TL_I32: st = split_sort<int32_t>(c, (int32_t *)dev_keys, n, n_out, s); break;
+        default: st = split_sort<int64_t>(c, (int64_t *)dev_keys, n, n_out, s); break;
+        }
+    } else if (W == 4) {
         const uint32_t flip = dtype == TL_I32 ? 0x80000000u : 0u;
         st = sort_dedupe_t<uint32_t>(c, (uint32_t *)dev_keys, n, flip, n_out, s);
     } else {
