@@ -16,7 +16,11 @@
  *
  * Scratch (stash, move flags, plan tables, error word) is per device and
  * owned by the library.  Calls that overlap on one device -- on two streams,
- * or from two host threads -- share it and race: serialise them.
+ * or from two host threads -- share it and race: serialise them.  The stash of
+ * a BST or B-tree permutation grows to its internal keys, 6.25 GiB at most; when
+ * that is more, or is not to be had, the permutation makes do with
+ * max(2^24, n/16) keys and takes longer.  Arrays of at most 128 MiB of any
+ * layout take a stash of their size.
  *
  * Large query batches are partitioned through workspaces of the library's own
  * (at most two per device, each at most 16 bytes a query of 2^27 and tables);

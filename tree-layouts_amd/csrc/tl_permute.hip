@@ -678,16 +678,18 @@ static tl_status launch_plan(Ctx *c, const Plan &pl, T *A, hipStream_t s, const 
 }
 
 // ---------------------------------------------------------------------------
-// arrays of at most DIRECT_KEYS keys (the stash every plan may use) fit the
-// stash whole: one copy there and one pass back, every key straight to its
-// slot (inverse: from it), instead of a plan's uploaded tables and up to a
-// dozen dependent launches.  Reads (inverse: writes) are contiguous; the writes
-// of a tile fall into one run per level of the tree, whose partial lines meet
-// in the tile's L2, and both buffers fit the 256 MB cache.  Faster than the
-// plan at every size up to the limit; B-tree b=16 of 8-byte keys, plan -> now:
-// 1000 keys 20 -> 12 us, 10^5 74 -> 12, 10^6 86 -> 16, 2^24 213 -> 86 us
-// (6.2 TB/s); BST 131 -> 87, mvEB 194 -> 100 us at 2^24.
-constexpr uint64_t DIRECT_KEYS = 1ull << 24;
+// arrays of at most DIRECT_BYTES fit a stash whole: one copy there and one pass
+// back, every key straight to its slot (inverse: from it), instead of a plan's
+// uploaded tables and up to a dozen dependent launches.  Reads (inverse: writes)
+// are contiguous; the writes of a tile fall into one run per level of the tree,
+// whose partial lines meet in the tile's L2, and both buffers fit the 256 MB
+// cache: past it the slides below are as fast, which move fewer bytes (4-byte
+// BSTs and B-trees at 128 MiB: 97-108 us against 137-159, at 152 MiB 150-168
+// against 152-168).  Faster than the plan at every size up to the limit; B-tree
+// b=16 of 8-byte keys, plan -> now: 1000 keys 20 -> 12 us, 10^5 74 -> 12, 10^6
+// 86 -> 16, 2^24 213 -> 86 us (6.2 TB/s); BST 131 -> 87, mvEB 194 -> 100 us at
+// 2^24; of 4-byte keys at 2^25 - 1: mvEB 189 -> 119 us.
+constexpr uint64_t DIRECT_BYTES = 1ull << 27;
 constexpr int DIRECT_IT = 8;
 
 template <typename W, int LAYOUT, bool INV>
@@ -739,6 +741,416 @@ static tl_status run_direct(Ctx *c, Layout lay, W *A, uint64_t n, uint64_t b, bo
     if (tl == TILE_BST) return direct_launch<W, TILE_BST>(c, A, sh, inverse, s);
     if (tl == TILE_BTREE) return direct_launch<W, TILE_BTREE>(c, A, sh, inverse, s);
     return direct_launch<W, TILE_VEB>(c, A, sh, inverse, s);
+}
+
+// ---------------------------------------------------------------------------
+// larger BSTs and B-trees: one pass over the keys.  Every leaf's slot lies at
+// or right of its rank, in rank order, so the sorted keys are swept from the
+// right: a tile's leaves go straight to their slots, its internal keys to the
+// stash in slot order, which a copy then puts in front.  Where the leaves are
+// few, the keys of the level above them lie right of their ranks too, up to a
+// row that follows from the sizes, and go straight to their slots as well.  A
+// tile stores once the tiles it overwrites, all right of it, have been read,
+// as in chained moves.  The inverse copies the stash's slots there first and
+// sweeps from the left.
+// Bound by memory: 2 n keys are moved, and 2 more for each that is stashed (a
+// BST's n/4 to n/2, few of most B-trees); gathering level by level moved 4 to 9
+// for each key.  Plan -> now, forward: BST of 5*10^8 4-byte keys 6.18 -> 1.23 ms
+// (5 TB/s), of 2^30 8-byte keys 7.25 -> 4.87 ms; B-tree b=16 of 2^30 8-byte keys
+// 7.22 -> 4.18 ms (5.5 TB/s); b=8 of 2*10^8 4-byte keys 2.06 -> 0.39 ms, its
+// inverse 2.10 -> 0.41.
+// Faster than the plan at every size and b measured past DIRECT_BYTES.
+// Tiles of 64 KB: tickets come from one counter at about 66 a us, which bounds
+// 4-byte keys in tiles half the size (5*10^8 in a BST: 1.28 -> 1.21 ms).  The
+// inverse, whose loads are the scattered ones, has no registers for 64 keys a
+// lane (1.41 -> 1.71 ms).
+constexpr uint32_t SLIDE_NT = 256, SLIDE_LANE = 256;   // bytes of a lane
+template <typename W, bool INV>
+constexpr uint32_t SLIDE_IT = SLIDE_LANE / (INV ? 8 : sizeof(W));
+template <typename W, bool INV>
+constexpr uint32_t SLIDE_KEYS = SLIDE_NT * SLIDE_IT<W, INV>;
+constexpr uint64_t SLIDE_STASH = 5ull << 30;   // bytes, at most
+
+struct SlideShape : SlotShape {
+    uint32_t tiles, k1, mul;   // t / k1 = t * mul >> 32 for t < 2^16, k1 < 2^13
+    uint32_t tail;             // internal keys alone from this rank on
+    uint32_t up, up_end;       // slots of the level above the leaves that
+                               // never see the stash
+    uint32_t gap;              // of them, those without a place in the stash
+};
+
+static SlideShape slide_shape(uint32_t layout, uint64_t n, uint64_t b, uint32_t keys) {
+    SlideShape s{};
+    static_cast<SlotShape &>(s) = slot_shape(layout, n, b, false);
+    s.k1 = s.b + 1;
+    s.tail = s.span + s.rem;
+    s.tiles = (uint32_t)((n + keys - 1) / keys);
+    s.mul = (uint32_t)((0xFFFFFFFFull + s.k1) / s.k1);
+    // the key of internal rank i, row r = i / k1 of that level, goes to
+    // up + i - r from rank i + (leaves before it)
+    const uint64_t leaves = s.n - s.nint;
+    s.up = (uint32_t)(ipow64(s.k1, s.depth - 1) - 1);
+    s.up_end = s.up + (uint32_t)(leaves < s.up ? (s.up - leaves) * s.b : 0);
+    // (slots keep their place in a 16-byte line)
+    s.gap = (s.up_end - s.up) & ~15u;
+    return s;
+}
+
+// row of place t < 2^16 counted from the start of a tile's first row
+// (b <= 4096)
+template <int LAYOUT>
+__device__ inline uint32_t slide_row(uint32_t t, const SlideShape &s) {
+    if constexpr (LAYOUT == TILE_BST) return t >> 1;
+    return __umulhi(t, s.mul);
+}
+
+// leaves / internal keys of smaller rank
+__device__ inline uint32_t slide_leaves(uint32_t x, const SlideShape &s) {
+    if (x < s.span) return x - (uint32_t)__umul64hi(x, s.recip);
+    return min(x, s.tail) - s.nsep;
+}
+
+// rank of leaf j; of internal key i
+__device__ inline uint32_t slide_rank(uint32_t j, const SlideShape &s) {
+    return j + min(j / s.b, s.nsep);
+}
+__device__ inline uint32_t slide_internal(uint32_t i, const SlideShape &s) {
+    return i < s.nsep ? i * s.k1 + s.b : i + (s.tail - s.nsep);
+}
+
+// where an internal slot is in the stash
+__device__ inline uint32_t slide_stash(uint32_t slot, const SlideShape &s) {
+    return slot < s.up ? slot : slot - s.gap;
+}
+
+// waits for the tiles of the keys [lo, hi)
+template <typename W, bool INV>
+__device__ inline bool slide_wait(uint32_t lo, uint32_t hi, uint32_t tile, const SlideShape &s,
+                                  uint32_t *flags, uint32_t *err, uint64_t limit) {
+    if (lo >= hi) return true;
+    for (uint32_t g = lo / SLIDE_KEYS<W, INV>; g <= (hi - 1) / SLIDE_KEYS<W, INV>; g++) {
+        const bool before = INV ? g < tile : g > tile;
+        if (before && !wait_flag(&flags[INV ? g : s.tiles - 1 - g], err, limit)) return false;
+    }
+    return true;
+}
+
+// tile (of keys [x0, x0 + m), ticket t) has been read: publishes that, and waits
+// until the keys that it overwrites have been
+template <typename W, bool INV>
+__device__ inline bool slide_turn(uint32_t t, uint32_t tile, uint32_t x0, uint32_t m,
+                                  const SlideShape &s, uint32_t *flags, uint32_t *err,
+                                  uint64_t limit) {
+    __hip_atomic_store(&flags[t], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t x1 = x0 + m;
+    if constexpr (INV) {
+        uint32_t lo = max(x0, s.nint), hi = x1;
+        if (lo < hi) {
+            lo = slide_rank(lo - s.nint, s);
+            hi = slide_rank(hi - 1 - s.nint, s) + 1;
+        }
+        if (!slide_wait<W, INV>(lo, hi, tile, s, flags, err, limit)) return false;
+        lo = max(x0, s.up);
+        hi = min(x1, s.up_end);
+        if (lo < hi) {
+            const uint32_t j0 = lo - s.up, j1 = hi - 1 - s.up;
+            lo = slide_internal(j0 + j0 / s.b, s);
+            hi = slide_internal(j1 + j1 / s.b, s) + 1;
+        }
+        return slide_wait<W, INV>(lo, hi, tile, s, flags, err, limit);
+    } else {
+        const uint32_t l0 = slide_leaves(x0, s), l1 = slide_leaves(x1, s);
+        if (!slide_wait<W, INV>(s.nint + l0, s.nint + l1, tile, s, flags, err, limit)) return false;
+        const uint32_t i0 = x0 - l0, i1 = x1 - l1;
+        return slide_wait<W, INV>(s.up + i0 - (uint32_t)__umul64hi(i0, s.recip),
+                               min(s.up_end, s.up + i1 - (uint32_t)__umul64hi(i1, s.recip)), tile,
+                               s, flags, err, limit);
+    }
+}
+
+template <typename W, int LAYOUT, bool INV>
+__global__ __launch_bounds__(SLIDE_NT) void k_level_slide(W *__restrict__ A, W *__restrict__ stash,
+                                                          SlideShape s, uint32_t *flags,
+                                                          uint32_t *err, uint64_t limit) {
+    __shared__ SlotMap<LAYOUT> map;
+    __shared__ W sep[SLIDE_KEYS<W, INV> / 2 + 1];   // the tile's separators, row by row
+    __shared__ uint32_t s_t, s_ok;
+    const uint32_t tid = threadIdx.x;
+    uint32_t *ticket = flags + s.tiles;
+    slot_map<LAYOUT>(s, map);
+    for (;;) {
+        if (tid == 0) s_t = atomicAdd(ticket, 1u);
+        __syncthreads();
+        const uint32_t t = s_t;
+        if (t >= s.tiles) return;
+        const uint32_t tile = INV ? t : s.tiles - 1 - t;
+        const uint32_t x0 = tile * SLIDE_KEYS<W, INV>, m = min(SLIDE_KEYS<W, INV>, s.n - x0);
+        const uint32_t row0 = x0 < s.span ? (uint32_t)__umul64hi(x0, s.recip) : s.nsep;
+        const uint32_t c0 = x0 - row0 * s.k1;
+        const uint32_t in_rows = x0 < s.span ? min(m, s.span - x0) : 0u;
+        const uint32_t seps = in_rows ? slide_row<LAYOUT>(c0 + in_rows, s) : 0u;
+        const uint32_t tail_i = s.tail - s.nsep;   // internal rank of rank x >= tail: x - tail_i
+        auto direct = [&](uint32_t slot) { return slot - s.up < s.up_end - s.up; };
+        W v[SLIDE_IT<W, INV>];
+        // Tiles of whole-row keys alone, almost all: leaves and separators, or
+        // internal keys of the last level and those above it, which go to the
+        // stash or stay clear of it.  What is not a separator goes to side + i -
+        // its row, and rows follow by steps from key to key, where finding each
+        // key's slot took three times the vector instructions that the memory
+        // leaves time for with 4-byte keys.
+        const uint32_t up0 = x0 - tail_i, up_row0 = (uint32_t)__umul64hi(up0, s.recip);
+        const bool leaves = in_rows == SLIDE_KEYS<W, INV>, ups = x0 >= s.tail && m == SLIDE_KEYS<W, INV>;
+        const uint32_t up_slot = s.up + up0 - up_row0;   // the first key's, and the last's at most
+        const bool up_in = up_slot + SLIDE_KEYS<W, INV> <= s.up_end, up_out = up_slot >= s.up_end;
+        if (leaves || (ups && (up_in || up_out))) {
+            const uint32_t c_0 = leaves ? c0 : up0 - up_row0 * s.k1;
+            const bool in_stash = ups && up_out;
+            char *side = leaves     ? (char *)(A + s.nint + x0 - row0)
+                         : in_stash ? (char *)(stash + up_slot - s.gap)
+                                    : (char *)(A + up_slot);
+            const uint32_t nseps = slide_row<LAYOUT>(c_0 + SLIDE_KEYS<W, INV>, s);
+            const uint32_t dq = SLIDE_NT / s.k1, dc = SLIDE_NT - dq * s.k1;
+            const uint32_t q0 = slide_row<LAYOUT>(c_0 + tid, s), c_tid = c_0 + tid - q0 * s.k1;
+            // fn(k, row, whether it is that row's separator) for each key
+            auto each = [&](auto fn) {
+                uint32_t q = q0, c = c_tid;
+#pragma unroll
+                for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) {
+                    fn(k, q, c == s.b);
+                    q += dq;
+                    if constexpr (LAYOUT != TILE_BST) {
+                        c += dc;
+                        const bool wrap = c >= s.k1;
+                        c -= wrap ? s.k1 : 0u;
+                        q += wrap ? 1u : 0u;
+                    }
+                }
+            };
+            auto at = [&](uint32_t k, uint32_t q) -> W & {
+                return *(W *)(side + (uint32_t)((k * SLIDE_NT + tid - q) * sizeof(W)));
+            };
+            // slot of the separator of row q
+            auto sep_slot = [&](uint32_t q) {
+                return internal_slot<LAYOUT>(leaves ? row0 + q : (up_row0 + q) * s.k1 + s.b, s, map);
+            };
+            W *mine = A + x0 + tid;
+            if constexpr (INV) {
+                each([&](uint32_t k, uint32_t q, bool is_sep) {
+                    if (!is_sep) v[k] = at(k, q);
+                });
+                for (uint32_t i = tid; i < nseps; i += SLIDE_NT) {
+                    const uint32_t slot = sep_slot(i);
+                    sep[i] = direct(slot) ? A[slot] : stash[slide_stash(slot, s)];
+                }
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) v[k] = mine[k * SLIDE_NT];
+            }
+            loads_done();
+            __syncthreads();
+            if (tid == 0) s_ok = slide_turn<W, INV>(t, tile, x0, m, s, flags, err, limit);
+            __syncthreads();
+            const bool ok = s_ok;
+            if constexpr (INV) {
+                // the separators join the other keys before the barrier, so that
+                // every lane stores at once (in two halves, alternate keys each,
+                // 2^28 8-byte keys took 2.4 ms)
+                each([&](uint32_t k, uint32_t q, bool is_sep) {
+                    const W y = sep[q];
+                    v[k] = is_sep ? y : v[k];
+                });
+                __syncthreads();
+                if (ok) {
+#pragma unroll
+                    for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) mine[k * SLIDE_NT] = v[k];
+                }
+                continue;
+            }
+            each([&](uint32_t k, uint32_t q, bool is_sep) {
+                if (is_sep) sep[q] = v[k];
+                else if (ok || in_stash) at(k, q) = v[k];
+            });
+            __syncthreads();
+            for (uint32_t i = tid; i < nseps; i += SLIDE_NT) {
+                const uint32_t slot = sep_slot(i);
+                if (!direct(slot)) stash[slide_stash(slot, s)] = sep[i];
+                else if (ok) A[slot] = sep[i];
+            }
+            __syncthreads();   // sep, s_t and s_ok are the next tile's
+            continue;
+        }
+        // The few other tiles (where rows end, or the stash begins): every key's slot
+        // by itself, the loops left rolled so as not to cost the others registers.
+        W w[SLIDE_IT<W, INV>];
+        // of a key of a row: its leaf slot, or ~0u for the separator of row q
+        auto leaf = [&](uint32_t i, uint32_t &q) {
+            q = slide_row<LAYOUT>(c0 + i, s);
+            return c0 + i - q * s.k1 == s.b ? ~0u : s.nint + x0 + i - row0 - q;
+        };
+#pragma unroll 1
+        for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) {
+            const uint32_t i = k * SLIDE_NT + tid, x = x0 + i;
+            if (i >= m) continue;
+            if constexpr (INV) {
+                uint32_t q;
+                if (i < in_rows) {
+                    const uint32_t at = leaf(i, q);
+                    if (at != ~0u) w[k] = A[at];
+                } else if (x < s.tail) {
+                    w[k] = A[s.nint + x - s.nsep];
+                } else {
+                    const uint32_t slot = internal_slot<LAYOUT>(x - tail_i, s, map);
+                    w[k] = direct(slot) ? A[slot] : stash[slide_stash(slot, s)];
+                }
+            } else {
+                w[k] = A[x];
+            }
+        }
+        if constexpr (INV)
+            for (uint32_t i = tid; i < seps; i += SLIDE_NT) {
+                const uint32_t slot = internal_slot<LAYOUT>(row0 + i, s, map);
+                sep[i] = direct(slot) ? A[slot] : stash[slide_stash(slot, s)];
+            }
+        loads_done();
+        __syncthreads();
+        if (tid == 0) s_ok = slide_turn<W, INV>(t, tile, x0, m, s, flags, err, limit);
+        if constexpr (!INV) {   // the stash has no other readers
+#pragma unroll 1
+            for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) {
+                const uint32_t i = k * SLIDE_NT + tid, x = x0 + i;
+                uint32_t q;
+                if (i >= m) continue;
+                if (i < in_rows) {
+                    if (leaf(i, q) == ~0u) sep[q] = w[k];
+                } else if (x >= s.tail) {
+                    const uint32_t slot = internal_slot<LAYOUT>(x - tail_i, s, map);
+                    if (!direct(slot)) stash[slide_stash(slot, s)] = w[k];
+                }
+            }
+        }
+        __syncthreads();
+        // a tile whose wait gave up (the call then reports TL_ETIMEOUT) keeps
+        // its keys to itself
+        const bool ok = s_ok;
+        if constexpr (!INV)
+            for (uint32_t i = tid; i < seps; i += SLIDE_NT) {
+                const uint32_t slot = internal_slot<LAYOUT>(row0 + i, s, map);
+                if (!direct(slot)) stash[slide_stash(slot, s)] = sep[i];
+                else if (ok) A[slot] = sep[i];
+            }
+        if (ok) {
+#pragma unroll 1
+            for (uint32_t k = 0; k < SLIDE_IT<W, INV>; k++) {
+                const uint32_t i = k * SLIDE_NT + tid, x = x0 + i;
+                if (i >= m) continue;
+                uint32_t q, at = 0;
+                if (i < in_rows) at = leaf(i, q);
+                if constexpr (INV) {
+                    A[x] = at == ~0u ? sep[q] : w[k];
+                } else if (i < in_rows) {
+                    if (at != ~0u) A[at] = w[k];
+                } else if (x < s.tail) {
+                    A[s.nint + x - s.nsep] = w[k];
+                } else {
+                    const uint32_t slot = internal_slot<LAYOUT>(x - tail_i, s, map);
+                    if (direct(slot)) A[slot] = w[k];
+                }
+            }
+        }
+        __syncthreads();   // sep, s_t and s_ok are the next tile's
+    }
+}
+
+// dst[0, count) = src[0, count), 16 bytes a lane and load where both have the
+// same place in a 16-byte line
+template <typename W>
+__global__ __launch_bounds__(256) void k_copy_wide(W *__restrict__ dst, const W *__restrict__ src,
+                                                   uint64_t count) {
+    constexpr uint64_t V = 16 / sizeof(W);
+    const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    uint64_t head = count, wide = 0;   // keys before the wide part, its loads
+    if ((((uintptr_t)dst ^ (uintptr_t)src) & 15) == 0) {
+        head = min(count, (uint64_t)((0 - (uintptr_t)dst) & 15) / sizeof(W));
+        wide = (count - head) / V;
+        const uint4 *s = (const uint4 *)(src + head);
+        uint4 *d = (uint4 *)(dst + head);
+        for (uint64_t i = i0; i < wide; i += 4 * step) {
+            uint4 v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (i + k * step < wide) v[k] = s[i + k * step];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (i + k * step < wide) d[i + k * step] = v[k];
+        }
+    }
+    for (uint64_t i = i0; i < head; i += step) dst[i] = src[i];
+    for (uint64_t i = head + wide * V + i0; i < count; i += step) dst[i] = src[i];
+}
+
+template <typename W, int LAYOUT, bool INV>
+static tl_status slide_launch(Ctx *c, W *A, const SlideShape &sh, W *stash, uint32_t *flags,
+                              hipStream_t s) {
+    // Few workgroups a compute unit: those at work stay close together, which
+    // the memory rewards (B-tree b=16 of 2^30 8-byte keys with 1, 2, 4, 8: 4.68,
+    // 4.23, 4.46, 4.47 ms).  The inverse reads small nodes' keys in halves and
+    // needs more loads in flight for it (BST of 5*10^8 4-byte keys with 4, 8:
+    // 1.53, 1.41 ms; b=8 of 2*10^8 8-byte keys with 2, 3, 8: 0.72, 0.70, 0.71).
+    const uint32_t per_cu = !INV ? 2 : sh.b < 4 ? 8 : 3;
+    const dim3 grid(std::min<uint32_t>(sh.tiles, c->num_cus * per_cu));
+    TL_TRY(fill_u32_launch(flags, sh.tiles + 1ull, 0, s));
+    auto copy = [&](uint64_t slot, uint64_t end) -> tl_status {
+        W *a = A + slot, *b = stash + (slot < sh.up ? slot : slot - sh.gap);
+        const uint64_t count = end - slot;
+        const dim3 g((uint32_t)std::min<uint64_t>((count + 1023) / 1024, c->num_cus * 32ull));
+        if (count)
+            hipLaunchKernelGGL(k_copy_wide<W>, g, dim3(256), 0, s, INV ? b : a,
+                               (const W *)(INV ? a : b), count);
+        TL_LAUNCH_CHECK();
+        return TL_OK;
+    };
+    auto copies = [&]() -> tl_status {
+        if (sh.up_end == sh.up) return copy(0, sh.nint);
+        TL_TRY(copy(0, sh.up));
+        return copy(sh.up_end, sh.nint);
+    };
+    if (INV) TL_TRY(copies());
+    hipLaunchKernelGGL((k_level_slide<W, LAYOUT, INV>), grid, dim3(SLIDE_NT), 0, s, A, stash, sh,
+                       flags, c->err_flag, c->wait_ticks);
+    TL_LAUNCH_CHECK();
+    return INV ? TL_OK : copies();
+}
+
+template <typename W, bool INV>
+static tl_status slide_layout(Ctx *c, Layout lay, W *A, const SlideShape &sh, W *stash,
+                              uint32_t *flags, hipStream_t s) {
+    return lay == L_BST ? slide_launch<W, TILE_BST, INV>(c, A, sh, stash, flags, s)
+                        : slide_launch<W, TILE_BTREE, INV>(c, A, sh, stash, flags, s);
+}
+
+// *taken = false (and nothing is enqueued) where the plan has to do it
+template <typename W>
+static tl_status run_slide(Ctx *c, Layout lay, W *A, uint64_t n, uint64_t b, bool inverse,
+                           hipStream_t s, bool *taken) {
+    *taken = false;
+    if ((lay != L_BST && lay != L_BTREE) || n >= (1ull << 32) - 1 ||
+        n <= (lay == L_BTREE ? b : 1))
+        return TL_OK;
+    const SlideShape sh = slide_shape(lay == L_BST ? TILE_BST : TILE_BTREE, n, b,
+                                      inverse ? SLIDE_KEYS<W, true> : SLIDE_KEYS<W, false>);
+    const uint64_t stashed = sh.nint - sh.gap;
+    if (stashed * sizeof(W) > SLIDE_STASH) return TL_OK;
+    W *stash = nullptr;
+    uint32_t *flags = nullptr;
+    // short of memory, the plan makes do with less
+    tl_status st = scratch(c, 0, stashed * sizeof(W), (void **)&stash);
+    if (st == TL_OK) st = scratch(c, 1, (sh.tiles + 1ull) * 4, (void **)&flags);
+    if (st == TL_ENOMEM) return TL_OK;
+    TL_TRY(st);
+    *taken = true;
+    return inverse ? slide_layout<W, true>(c, lay, A, sh, stash, flags, s)
+                   : slide_layout<W, false>(c, lay, A, sh, stash, flags, s);
 }
 
 template <typename T>
@@ -1211,7 +1623,7 @@ static tl_status permute(Layout lay, void *dev_A, uint64_t n, uint64_t b, tl_dty
             return TL_EHIP;
         }
     }
-    if (n <= DIRECT_KEYS && !plan_knobs()) {
+    if (n <= DIRECT_BYTES / W && !plan_knobs()) {
         Timer tm;
         TL_TRY(tm.start(s, ms));
         if (n > (lay == L_BTREE ? b : 1)) {
@@ -1219,6 +1631,17 @@ static tl_status permute(Layout lay, void *dev_A, uint64_t n, uint64_t b, tl_dty
                           : run_direct<uint64_t>(c, lay, (uint64_t *)dev_A, n, b, inverse, s));
         }
         return tm.stop();
+    }
+    if (n > DIRECT_BYTES / W && !plan_knobs()) {
+        Timer tm;
+        TL_TRY(tm.start(s, ms));
+        bool taken;
+        TL_TRY(W == 4 ? run_slide<uint32_t>(c, lay, (uint32_t *)dev_A, n, b, inverse, s, &taken)
+                      : run_slide<uint64_t>(c, lay, (uint64_t *)dev_A, n, b, inverse, s, &taken));
+        if (taken) {
+            TL_TRY(tm.stop());
+            return ms ? check_err_flag(c, s) : TL_OK;
+        }
     }
     Plan pl;
     build_plan(pl, tuning_for(c), lay, n, b, W);

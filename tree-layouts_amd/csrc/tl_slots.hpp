@@ -108,8 +108,29 @@ __device__ inline uint32_t veb_slot(uint32_t x, const SlotShape &s, const SlotMa
     return base + m.small[(1u << d) + x];
 }
 
-// slot of rank x in the layout; m.level[z]: first slot of the level whose keys'
-// internal ranks + 1 are divisible by (b + 1)^z and no more (TILE_BTREE)
+// slot of internal rank x of a BST or B-tree; m.level[z]: first slot of the
+// level whose keys' internal ranks + 1 are divisible by (b + 1)^z and no more
+// (TILE_BTREE)
+template <int LAYOUT>
+__device__ inline uint32_t internal_slot(uint32_t x, const SlotShape &s,
+                                         const SlotMap<LAYOUT> &m) {
+    if constexpr (LAYOUT == TILE_BST) {
+        const uint32_t y = x + 1, z = (uint32_t)__clz((int)__brev(y));
+        return ((y | (1u << s.depth)) >> (z + 1)) - 1;
+    } else {
+        auto div = [&](uint32_t v) { return (uint32_t)__umul64hi(v, s.recip); };
+        const uint32_t k1 = s.b + 1;
+        uint32_t r = x + 1, z = 0, q = div(r);
+        while (r == q * k1) {
+            r = q;
+            q = div(r);
+            z++;
+        }
+        return m.level[z] + r - q - 1;
+    }
+}
+
+// slot of rank x in the layout
 template <int LAYOUT>
 __device__ inline uint32_t slot_of(uint32_t x, const SlotShape &s, const SlotMap<LAYOUT> &m) {
     if constexpr (LAYOUT == TILE_SORTED) {
@@ -123,27 +144,18 @@ __device__ inline uint32_t slot_of(uint32_t x, const SlotShape &s, const SlotMap
         } else {
             x -= s.nsep;
         }
-        const uint32_t y = x + 1, z = (uint32_t)__clz((int)__brev(y));
-        return ((y | (1u << s.depth)) >> (z + 1)) - 1;
+        return internal_slot<LAYOUT>(x, s, m);
     } else {
-        auto div = [&](uint32_t v) { return (uint32_t)__umul64hi(v, s.recip); };
-        const uint32_t k1 = s.b + 1;
         if (x < s.span) {
-            const uint32_t row = div(x);
-            if (x - row * k1 < s.b) return s.nint + x - row;
+            const uint32_t row = (uint32_t)__umul64hi(x, s.recip);
+            if (x - row * (s.b + 1) < s.b) return s.nint + x - row;
             x = row;
         } else if (x < s.span + s.rem) {
             return s.nint + x - s.nsep;
         } else {
             x -= s.span + s.rem - s.nsep;
         }
-        uint32_t r = x + 1, z = 0, q = div(r);
-        while (r == q * k1) {
-            r = q;
-            q = div(r);
-            z++;
-        }
-        return m.level[z] + r - q - 1;
+        return internal_slot<LAYOUT>(x, s, m);
     }
 }
 
