@@ -65,6 +65,20 @@ def test_two_pass_partition_and_skew(layout, b, kind, dev, monkeypatch):
     assert np.array_equal(got, expected(layout, A, Q, kind, b))
 
 
+@pytest.mark.parametrize("n", [300_007, 5_000_011])
+@pytest.mark.parametrize("layout,b", [("bst", 1), ("btree", 16), ("mveb", 0), ("sorted", 0)])
+def test_crowded_range(n, layout, b, dev, monkeypatch):
+    """One and two passes with nearly all queries in one range: more than its
+    workgroup's share, and (two passes) more tiles of one bucket than a share has."""
+    monkeypatch.setenv("TL_QUERY_PATH", "part")
+    rng = np.random.default_rng(13)
+    keys = make_keys("u64", n, rng)
+    A = keys if layout == "sorted" else ol.permute(layout, keys.copy(), b)
+    Q = keys[n // 5 + rng.integers(0, 300, 400_001)]
+    Q[::400] = keys[rng.integers(0, n, Q[::400].size)]
+    assert np.array_equal(answers(layout, b, "u64", A, Q, dev), expected(layout, A, Q, "u64", b))
+
+
 @pytest.mark.parametrize("path", ["tile", "part"])
 @pytest.mark.parametrize("layout,b", [("bst", 1), ("btree", 16), ("btree", 8), ("mveb", 0)])
 def test_repeated_keys(path, layout, b, dev, monkeypatch):

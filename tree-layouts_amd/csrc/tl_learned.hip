@@ -815,7 +815,7 @@ extern "C" tl_status tl_query_btree_learned(const void *dev_A, uint64_t n, uint6
     TL_TRY(tm.start(s, ms));
     unsigned long long *st = (unsigned long long *)dev_stats;
     // A batch that is cheaper to partition needs no start nodes: at 2^30 keys
-    // and 2^27 hits the partitioned root descent takes 5.4 ms, the learned
+    // and 2^27 hits the partitioned root descent takes 4.8 ms, the learned
     // start 9.2 ms (the plain root descent 10.5 ms; the start nodes save a
     // seventh to an eighth of it).  Callers that count fallbacks keep theirs.
     if (!st) {

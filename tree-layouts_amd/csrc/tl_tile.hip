@@ -18,9 +18,9 @@
 // every unsorted descent waits for lines from memory, however its tile is
 // ordered.  Measured (queries of keys that are there, before -> now):
 //   BST 2^20 4-byte keys, 2^20 queries          41 -> 28 us (tile)
-//   B-tree b=16, 2^30 8-byte keys, 2^27         10.5 -> 5.35 ms (partition)
+//   B-tree b=16, 2^30 8-byte keys, 2^27         10.5 -> 4.84 ms (partition)
 //   BST, the same                               28.5 -> 5.3 ms (partition)
-//   mvEB 3*10^8 8-byte keys, 2^26, Zipf(1.1)    5.58 -> 3.30 ms (partition)
+//   mvEB 3*10^8 8-byte keys, 2^26, Zipf(1.1)    5.58 -> 3.08 ms (partition)
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -143,7 +143,7 @@ __device__ inline void tile_btree(const K *__restrict__ A, const TileShape &s, c
 // to that depth): no per-lane position stack.
 template <typename K, int QN>
 __device__ inline void tile_veb(const K *__restrict__ A, const TileShape &s, const VebEntry *tb,
-                                const uint32_t *s_end, const uint32_t *s_tidx, const K (&q)[QN],
+                                const uint32_t *s_end, const uint16_t *s_tidx, const K (&q)[QN],
                                 uint32_t (&res)[QN]) {
     const uint32_t n = s.n;
     bool pend[QN];
@@ -232,7 +232,7 @@ __device__ inline void tile_sorted(const K *__restrict__ A, const TileShape &s, 
 template <typename K, int LAYOUT, int QN>
 __device__ inline void tile_descend(const K *__restrict__ A, const TileShape &s,
                                     const VebEntry *tb, const uint32_t *s_end,
-                                    const uint32_t *s_tidx, const K (&q)[QN],
+                                    const uint16_t *s_tidx, const K (&q)[QN],
                                     uint32_t (&res)[QN]) {
     if constexpr (LAYOUT == TILE_BST)
         tile_bst<K, QN>(A, s, q, res);
@@ -261,7 +261,8 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
     __shared__ K keys[T];                      // the tile in bucket order; then its answers
     __shared__ uint16_t from[T];               // place in the tile of each sorted query
     __shared__ VebEntry tb[LAYOUT == TILE_VEB ? TILE_TABLES : 1];
-    __shared__ uint32_t s_end[64], s_tidx[64];
+    __shared__ uint32_t s_end[64];
+    __shared__ uint16_t s_tidx[64];
     uint32_t *answers = reinterpret_cast<uint32_t *>(keys);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ SlotMap<LAYOUT> map;
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
                 tb[i] = {(uint32_t)s.tables[i].L, (uint32_t)s.tables[i].R, s.tables[i].D};
             if (tid < s.ntables) {
                 s_end[tid] = s.idx ? (uint32_t)s.idx[tid] : s.n;
-                s_tidx[tid] = s.tidx ? s.tidx[tid] : 0u;
+                s_tidx[tid] = s.tidx ? (uint16_t)s.tidx[tid] : (uint16_t)0;
             }
         }
     }
@@ -363,44 +364,47 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
 // ---------------------------------------------------------------------------
 // partitioned lookups: batches of at least a few queries per array line.
 //
-// (2^27 queries of 2^30 8-byte keys move 10 GB in the answering kernel, 2.3 ms,
-// and 24 bytes a query and pass through four kernels: count 0.45 ms, scatter
-// 0.6 ms, return 0.45 ms.)
+// (2^27 queries of 2^30 8-byte keys move 10 GB in the answering kernel, 2.4 ms;
+// the first pass of the queries takes 0.5 ms to count, 0.6 to scatter and 0.55
+// for the way back, the last 0.6 and 0.25.)
 //
 // The array is cut into 2^lg ranges of equal rank count, each small enough
-// for LDS; the queries are put in range order (one counting pass, or two when
-// there are more ranges than a pass has counters), each workgroup then reads a
-// range's keys once, coalesced, and answers the range's queries from LDS, and
-// the answers go back to the order of the queries.  So the array is read once
-// where the descents of unsorted queries miss the caches on every level past
-// the top ones.
+// for LDS.  The queries are put in range order tile by tile (where there are
+// more ranges than a tile has counters, they are partitioned into 2^lg1 buckets
+// first, whole), each workgroup then reads a range's keys once, coalesced, and
+// answers the range's queries of many tiles from LDS, and the answers go back to
+// the order of the queries.  So the array is read once where the descents of
+// unsorted queries miss the caches on every level past the top ones.  A tile
+// keeps its own order to itself: no counts over all tiles, no second read of the
+// queries, contiguous reads on the way back.
 
 constexpr uint32_t RANGE_NT = 512;
-constexpr uint32_t RANGE_CHUNK = 4096;  // queries of one workgroup's turn
 
-// bound[j]: the smallest key of range j
+// bound[j]: the smallest key of range j; the queue is empty
 template <typename W, int LAYOUT>
 __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, TileShape s,
-                                                     uint32_t lg, W *__restrict__ bound) {
+                                                     uint32_t lg, W *__restrict__ bound,
+                                                     uint32_t *queued) {
     __shared__ SlotMap<LAYOUT> map;
     slot_map<LAYOUT>(s, map);
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j == 0) *queued = 0;
     if (j < (1u << lg)) bound[j] = A[slot_of<LAYOUT>(range_first(j, s.n, lg), s, map)];
 }
 
 // Counts of a tile's queries per bucket (counts[t][bucket]); every query's
 // bucket and rank among the tile's queries of it go to pack[].
-template <typename K, bool SECOND, int IT>
+template <typename K, int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_count(
     const K *__restrict__ Q, uint64_t nq, const K *__restrict__ bound, uint32_t lg1, uint32_t lg2,
-    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    uint32_t tiles,
     uint32_t *__restrict__ pack, uint32_t *__restrict__ counts) {
     __shared__ K spl[PART_BINS];
     __shared__ uint32_t cnt[PART_BINS];
-    const uint32_t lg = SECOND ? lg2 : lg1, B = 1u << lg, step = SECOND ? 1u : 1u << lg2;
+    const uint32_t lg = lg1, B = 1u << lg, step = 1u << lg2;
     const uint32_t t = xcd_tile(tiles);
-    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
-    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    if (t >= tiles) return;
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
     K q[IT];
 #pragma unroll
     for (int k = 0; k < IT; k++) {
@@ -410,7 +414,7 @@ __global__ __launch_bounds__(PART_NT) void k_part_count(
     if (threadIdx.x < B) {
         cnt[threadIdx.x] = 0;
         if (threadIdx.x)
-            spl[threadIdx.x] = bound[p.first + (uint64_t)heap_order(threadIdx.x, lg) * step];
+            spl[threadIdx.x] = bound[(uint64_t)heap_order(threadIdx.x, lg) * step];
     }
     __syncthreads();
     uint32_t node[IT];
@@ -437,20 +441,20 @@ __global__ __launch_bounds__(PART_NT) void k_part_count(
 // they were read, single queries filled cache lines so slowly that most were
 // written back several times (5.8 GB for 2^27 8-byte queries, where 1.6 GB
 // are written now).
-template <typename K, bool SECOND, int IT>
+template <typename K, int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_scatter(
     const K *__restrict__ Q, uint64_t nq, uint32_t lg1, uint32_t lg2,
-    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    uint32_t tiles,
     const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
     const uint32_t *__restrict__ pack, K *__restrict__ out) {
     __shared__ K stage[PART_NT * IT];
     __shared__ uint32_t at[PART_BINS], local[PART_BINS];
     __shared__ uint32_t wsum[PART_NT / 64];
     uint32_t *stage_to = reinterpret_cast<uint32_t *>(stage);
-    const uint32_t B = 1u << (SECOND ? lg2 : lg1), tid = threadIdx.x;
+    const uint32_t B = 1u << lg1, tid = threadIdx.x;
     const uint32_t t = xcd_tile(tiles);
-    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
-    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    if (t >= tiles) return;
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
     const uint32_t cnt = (uint32_t)(p.hi - p.lo);
     K q[IT];
     uint32_t pk[IT];
@@ -500,20 +504,19 @@ __global__ __launch_bounds__(PART_NT) void k_part_scatter(
 // The way back: dst[i] = src[place of query i], tile by tile as they were
 // scattered, the runs read into LDS whole (read one by one from there, 2^27
 // answers took 0.72 ms; the vector cache passes on one line a lane).
-// dst may be pack itself.
-template <bool SECOND, int IT, typename AT>
+template <int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_return(
     const uint32_t *__restrict__ src, uint64_t nq, uint32_t lg1, uint32_t lg2,
-    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    uint32_t tiles,
     const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
-    const uint32_t *pack, AT *dst) {
+    const uint32_t *pack, uint64_t *dst) {
     __shared__ uint32_t stage[PART_NT * IT];
     __shared__ uint32_t at[PART_BINS], local[PART_BINS];
     __shared__ uint32_t wsum[PART_NT / 64];
-    const uint32_t B = 1u << (SECOND ? lg2 : lg1), tid = threadIdx.x;
+    const uint32_t B = 1u << lg1, tid = threadIdx.x;
     const uint32_t t = xcd_tile(tiles);
-    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
-    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    if (t >= tiles) return;
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
     const uint32_t cnt = (uint32_t)(p.hi - p.lo);
     uint32_t pk[IT];
 #pragma unroll
@@ -552,13 +555,106 @@ __global__ __launch_bounds__(PART_NT) void k_part_return(
 #pragma unroll
     for (int k = 0; k < IT; k++) {
         const uint64_t i = p.lo + k * PART_NT + tid;
-        if (i < p.hi) dst[i] = (AT)stage[pk[k]];
+        if (i < p.hi) dst[i] = stage[pk[k]];
     }
 }
 
 template <typename K>
 __device__ inline K key_max() {
     return (K)-1 > (K)0 ? (K)-1 : (K)(((K)1 << (8 * sizeof(K) - 2)) - 1 + ((K)1 << (8 * sizeof(K) - 2)));
+}
+
+// The last pass (the only one of lg1 buckets where !SECOND): a tile's queries in
+// range order to the tile's own place, each query's place in the tile to
+// place[], and the places of the ranges' first ones to loc[t][range].
+template <typename K, bool SECOND, int IT>
+__global__ __launch_bounds__(PART_NT) void k_part_tile(
+    const K *__restrict__ Q, uint64_t nq, const K *__restrict__ bound, uint32_t lg1, uint32_t lg2,
+    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    uint16_t *__restrict__ place, uint16_t *__restrict__ loc, K *__restrict__ out) {
+    __shared__ K stage[PART_NT * IT];
+    __shared__ uint32_t cnt[PART_BINS];
+    __shared__ uint32_t wsum[PART_NT / 64];
+    K *spl = stage;   // read before the stage is written
+    const uint32_t lg = SECOND ? lg2 : lg1, B = 1u << lg, tid = threadIdx.x;
+    const uint32_t t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    K q[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        q[k] = i < p.hi ? Q[i] : K{};
+    }
+    if (tid < B) {
+        cnt[tid] = 0;
+        if (tid) spl[tid] = bound[p.first + heap_order(tid, lg)];
+    }
+    __syncthreads();
+    uint32_t node[IT];   // then the range, and the rank among the tile's queries of it
+#pragma unroll
+    for (int k = 0; k < IT; k++) node[k] = 1;
+    for (uint32_t l = 0; l < lg; l++) {
+#pragma unroll
+        for (int k = 0; k < IT; k++) node[k] = 2 * node[k] + (q[k] >= spl[node[k]] ? 1u : 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        if (p.lo + k * PART_NT + tid < p.hi) {
+            const uint32_t bin = node[k] - B;
+            node[k] = bin | (atomicAdd(&cnt[bin], 1u) << PART_LG);
+        }
+    }
+    __syncthreads();
+    uint32_t total;
+    const uint32_t before = block_scan(tid < B ? cnt[tid] : 0u, wsum, &total);
+    if (tid < B) {
+        cnt[tid] = before;
+        loc[(uint64_t)t * B + tid] = (uint16_t)before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        if (i < p.hi) {
+            const uint32_t x = cnt[node[k] & (PART_BINS - 1)] + (node[k] >> PART_LG);
+            place[i] = (uint16_t)x;
+            stage[x] = q[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint32_t x = k * PART_NT + tid;
+        if (x < total) out[p.lo + x] = stage[x];
+    }
+}
+
+// the answers of a tile from its own order to that of its input
+template <bool SECOND, int IT, typename AT>
+__global__ __launch_bounds__(PART_NT) void k_part_back(
+    const uint32_t *__restrict__ found, uint64_t nq, uint32_t lg1, uint32_t lg2,
+    const uint32_t *__restrict__ bstart, const uint32_t *__restrict__ tstart, uint32_t tiles,
+    const uint16_t *__restrict__ place, AT *__restrict__ dst) {
+    __shared__ uint32_t stage[PART_NT * IT];
+    const uint32_t tid = threadIdx.x, t = xcd_tile(tiles);
+    if (t >= (SECOND ? tstart[1u << lg1] : tiles)) return;
+    const PartTile p = part_tile<SECOND>(t, nq, PART_NT * IT, lg1, lg2, bstart, tstart);
+    uint32_t v[IT], x[IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        v[k] = i < p.hi ? found[i] : 0u;
+        x[k] = i < p.hi ? place[i] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < IT; k++) stage[k * PART_NT + tid] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+        const uint64_t i = p.lo + k * PART_NT + tid;
+        if (i < p.hi) dst[i] = (AT)stage[x[k]];
+    }
 }
 
 // slots of a range on one level of a B-tree, where `level`: place y is at
@@ -722,94 +818,200 @@ __device__ inline RangeSlots range_fill(const K *__restrict__ A, const TileShape
     return {false, 0, 0};
 }
 
-// The queries of a range from its keys in LDS.  S holds the queries in range
-// order, range j's at rstart[j] .. rstart[j + 1].  A key that occurs more than
-// once is answered by the descent itself, whose first equal key it has to be.
-template <typename K, int LAYOUT>
-__global__ __launch_bounds__(RANGE_NT) void k_part_answer(
-    const K *__restrict__ A, TileShape s, uint32_t lg, const K *__restrict__ S, uint32_t nq,
-    const uint32_t *__restrict__ rstart, uint32_t chunks, uint32_t *__restrict__ out) {
-    constexpr uint32_t WIN = 64;   // range starts at hand
+// The queries of range j in the tiles [ta, te), at most PART_SPAN of them, from
+// the range's keys in LDS: of those in tile order, [skip, skip + PART_SHARE).
+struct PartShare {
+    uint32_t j, ta, te, skip;
+};
+template <bool SECOND>
+constexpr uint32_t PART_SPAN = SECOND ? 64 : 256;
+constexpr uint32_t PART_SHARE = 8192;
+// consecutive ranges of a workgroup.  After two passes a range has few queries
+// (512 of 2^27 in 2^30 keys), and with one the look-ups that lead to them took a
+// fifth of the time.
+template <bool SECOND>
+constexpr uint32_t PART_RANGES = SECOND ? 8 : 1;
+
+// where the tiles and their queries of each range are
+struct PartLoc {
+    uint32_t lg1, lg2, T, nq, tiles, span;   // span: tiles of a share, at most
+    const uint32_t *bstart, *tstart;         // of two passes
+    const uint16_t *loc;
+};
+
+// The queries of PART_RANGES ranges from their keys in LDS.  S holds the queries,
+// each tile's in range order.  A workgroup takes a range's first share of `span`
+// tiles (SECOND: of the ranges' bucket); whatever is more, where queries crowd,
+// it puts on the queue, whose shares the second launch (REST) takes.  A key that
+// occurs more than once is answered by the descent itself, whose first equal key
+// it has to be.
+// Registers: at most 64 for a vEB, so that four workgroups share a compute unit
+// (3.25 -> 3.08 ms); the others are faster with what they ask for (5.16 -> 4.85).
+template <typename K, int LAYOUT, bool SECOND, bool REST>
+__global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_answer(const K *__restrict__ A, TileShape s,
+                                                             PartLoc pl, uint32_t units,
+                                                             const K *__restrict__ S,
+                                                             uint32_t *queued, PartShare *queue,
+                                                             uint32_t *__restrict__ out) {
+    constexpr uint32_t SPAN = PART_SPAN<SECOND>, RANGES = REST ? 1 : PART_RANGES<SECOND>;
     __shared__ K heap[RANGE_KEYS];
     __shared__ uint32_t sep_slot[LAYOUT == TILE_BTREE ? SEP_SLOTS : 1];
-    __shared__ uint32_t win[WIN + 1];
+    __shared__ uint32_t pre[SPAN], base[SPAN];   // queries before a tile's, the first's place
+    __shared__ uint16_t locs_of[RANGES > 1 ? SPAN : 1][RANGES + 1];
+    // one range's are read before its keys come
+    uint16_t(*locs)[RANGES + 1] =
+        RANGES > 1 ? locs_of : reinterpret_cast<uint16_t(*)[RANGES + 1]>(heap);
+    __shared__ uint32_t wsum[RANGE_NT / 64];
     __shared__ VebEntry tb[LAYOUT == TILE_VEB ? TILE_TABLES : 1];
-    __shared__ uint32_t s_end[64], s_tidx[64];
+    __shared__ uint32_t s_end[64];
+    __shared__ uint16_t s_tidx[64];
     __shared__ SlotMap<LAYOUT> map;
-    const uint32_t tid = threadIdx.x, n = s.n, ranges = 1u << lg;
+    const uint32_t tid = threadIdx.x, n = s.n, lg = pl.lg1 + (SECOND ? pl.lg2 : 0u);
+    const uint32_t B = 1u << (SECOND ? pl.lg2 : pl.lg1);
+    uint32_t unit = REST ? blockIdx.x : xcd_tile(units);
+    const uint32_t shares = REST ? *queued : units;
+    if (unit >= shares) return;
     if constexpr (LAYOUT == TILE_VEB) {
         for (uint32_t i = tid; i < s.table_size; i += RANGE_NT)
             tb[i] = {(uint32_t)s.tables[i].L, (uint32_t)s.tables[i].R, s.tables[i].D};
         if (tid < s.ntables) {
             s_end[tid] = s.idx ? (uint32_t)s.idx[tid] : n;
-            s_tidx[tid] = s.tidx ? s.tidx[tid] : 0u;
+            s_tidx[tid] = s.tidx ? (uint16_t)s.tidx[tid] : (uint16_t)0;
         }
     }
-    const uint32_t chunk = xcd_tile(chunks);
-    if (chunk >= chunks) return;
     slot_map<LAYOUT>(s, map);
-    uint32_t p = chunk * RANGE_CHUNK;
-    const uint32_t p1 = min(nq, p + RANGE_CHUNK);
-    while (p < p1) {
-        // the range of query p, and the starts of the ranges after it
-        uint32_t lo = 0, hi = ranges;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (rstart[mid] <= p) lo = mid;
-            else hi = mid;
+    for (; unit < shares; unit += gridDim.x) {
+        PartShare sh;
+        uint32_t bucket_end = 0, t_first = 0, q_first = 0, q_end = pl.nq;
+        if constexpr (REST) {
+            sh = queue[unit];
+        } else {
+            sh.j = SECOND ? unit * RANGES : unit & (B - 1);
+            sh.skip = 0;
         }
-        const uint32_t j0 = lo;
+        if constexpr (SECOND) {   // the ranges' bucket
+            const uint32_t k = sh.j >> pl.lg2;
+            t_first = pl.tstart[k];
+            bucket_end = pl.tstart[k + 1];
+            q_first = pl.bstart[k];
+            q_end = pl.bstart[k + 1];
+        }
+        if constexpr (!REST) {
+            sh.ta = SECOND ? t_first : (unit >> pl.lg1) * pl.span;
+            sh.te = min(sh.ta + pl.span, SECOND ? bucket_end : pl.tiles);
+        }
+        auto lo_of = [&](uint32_t t) { return q_first + (t - t_first) * pl.T; };
+        // place in tile t of the first query of range r of the bucket
+        auto loc_of = [&](uint32_t t, uint32_t r) -> uint32_t {
+            return r < B ? pl.loc[(uint64_t)t * B + r] : min(pl.T, q_end - lo_of(t));
+        };
+        const uint32_t r_first = sh.j & (B - 1);
+        for (uint32_t i = tid; i < (sh.te - sh.ta) * (RANGES + 1); i += RANGE_NT) {
+            const uint32_t t = i / (RANGES + 1), k = i - t * (RANGES + 1);
+            locs[t][k] = (uint16_t)loc_of(sh.ta + t, r_first + k);
+        }
         __syncthreads();
-        if (tid <= WIN) win[tid] = rstart[min(j0 + tid, ranges)];
-        __syncthreads();
-        for (uint32_t w = 0; w < WIN && p < p1; w++) {
-            const uint32_t qhi = min(p1, win[w + 1]);
-            if (qhi <= p) continue;
-            const uint32_t j = j0 + w;
+        for (uint32_t rr = 0; rr < RANGES; rr++) {
+            const uint32_t j = sh.j + rr;
+            uint32_t total;
+            if constexpr (!REST && SECOND) {
+                for (uint32_t ta = sh.te; ta < bucket_end; ta += pl.span) {
+                    const uint32_t te = min(ta + pl.span, bucket_end);
+                    const uint32_t c = ta + tid < te ? loc_of(ta + tid, r_first + rr + 1) -
+                                                           loc_of(ta + tid, r_first + rr)
+                                                     : 0u;
+                    (void)block_scan(c, wsum, &total);
+                    if (tid == 0)
+                        for (uint32_t skip = 0; skip < total; skip += PART_SHARE)
+                            queue[atomicAdd(queued, 1u)] = {j, ta, te, skip};
+                }
+            }
+            const bool tile = sh.ta + tid < sh.te;
+            const uint32_t before =
+                block_scan(tile ? locs[tid][rr + 1] - locs[tid][rr] : 0u, wsum, &total);
+            if (tid < SPAN) {
+                pre[tid] = before;
+                base[tid] = tile ? lo_of(sh.ta + tid) + locs[tid][rr] : 0u;
+            }
+            if (!REST && tid == 0)
+                for (uint32_t skip = PART_SHARE; skip < total; skip += PART_SHARE)
+                    queue[atomicAdd(queued, 1u)] = {j, sh.ta, sh.te, skip};
+            __syncthreads();
+            const uint32_t end = min(total, sh.skip + PART_SHARE);
+            if (sh.skip >= end) continue;   // the whole workgroup's
+            // where query i of the share is
+            auto place = [&](uint32_t i) {
+                uint32_t t = 0;
+                for (uint32_t h = pl.span >> 1; h > 0; h >>= 1) t += pre[t + h] <= i ? h : 0u;
+                return base[t] + (i - pre[t]);
+            };
             const uint32_t r0 = range_first(j, n, lg), m = range_first(j + 1, n, lg) - r0;
             const uint32_t depth = 32u - (uint32_t)__clz((int)(m - 1));   // 2^depth >= m
-            K q = p + tid < qhi ? S[p + tid] : K{};
-            __syncthreads();   // the last range's queries are answered
+            // two queries a lane and turn: 512 queries in 512 lanes would take a
+            // second turn for the few of half the ranges that have more (a vEB
+            // has no registers for it: 3.1 -> 3.4 ms at 3*10^8 keys)
+            constexpr int QN = LAYOUT == TILE_VEB ? 1 : 2;
+            uint32_t here[QN];
+            K q[QN];
+            auto fetch = [&](uint32_t q0) {
+#pragma unroll
+                for (int k = 0; k < QN; k++) {
+                    const uint32_t i = q0 + k * RANGE_NT + tid;
+                    here[k] = i < end ? place(i) : ~0u;
+                    q[k] = i < end ? S[here[k]] : K{};
+                }
+            };
+            fetch(sh.skip);
             const RangeSlots rs = range_fill<K, LAYOUT>(A, s, map, r0, m, depth, heap, sep_slot);
             __syncthreads();
-            for (uint32_t q0 = p; q0 < qhi; q0 += RANGE_NT) {
-                const uint32_t i = q0 + tid;
-                if (q0 != p) q = i < qhi ? S[i] : K{};
+            for (uint32_t q0 = sh.skip; q0 < end; q0 += QN * RANGE_NT) {
+                if (q0 != sh.skip) fetch(q0);
                 // the keys after the first that are smaller than q
                 // (TILE_SORTED: not larger)
-                uint32_t node = 1;
+                uint32_t node[QN];
+#pragma unroll
+                for (int k = 0; k < QN; k++) node[k] = 1;
                 for (uint32_t l = 0; l < depth; l++) {
-                    const K key = heap[node];
-                    const bool right = LAYOUT == TILE_SORTED ? key <= q : key < q;
-                    node = 2 * node + (right ? 1u : 0u);
-                }
-                const uint32_t below = min(node - (1u << depth), m - 1);
-                uint32_t ans = n;
-                if constexpr (LAYOUT == TILE_SORTED) {
-                    if (heap[0] <= q) ans = r0 + below;
-                } else {
-                    bool again = false;
-                    const uint32_t x = q <= heap[0] ? 0u : below + 1;
-                    if (x < m && heap[heap_at(x, depth)] == q) {
-                        const uint32_t t = rs.c0 + x, row = (t * s.small_mul) >> s.small_shift;
-                        if (LAYOUT == TILE_BTREE && rs.level && row < SEP_SLOTS)
-                            ans = t - row * (s.b + 1) != s.b ? rs.first + x - row : sep_slot[row];
-                        else
-                            ans = slot_of<LAYOUT>(r0 + x, s, map);
-                        if (x == 0 && r0 > 0) again = A[slot_of<LAYOUT>(r0 - 1, s, map)] == q;
-                        if (x + 1 < m) again |= heap[heap_at(x + 1, depth)] == q;
-                    }
-                    if (__any(again)) {
-                        const K qq[1] = {q};
-                        uint32_t res[1];
-                        tile_descend<K, LAYOUT, 1>(A, s, tb, s_end, s_tidx, qq, res);
-                        if (again) ans = res[0];
+#pragma unroll
+                    for (int k = 0; k < QN; k++) {
+                        const K key = heap[node[k]];
+                        const bool right = LAYOUT == TILE_SORTED ? key <= q[k] : key < q[k];
+                        node[k] = 2 * node[k] + (right ? 1u : 0u);
                     }
                 }
-                if (i < qhi) out[i] = ans;
+#pragma unroll
+                for (int k = 0; k < QN; k++) {
+                    const uint32_t below = min(node[k] - (1u << depth), m - 1);
+                    uint32_t ans = n;
+                    if constexpr (LAYOUT == TILE_SORTED) {
+                        if (heap[0] <= q[k]) ans = r0 + below;
+                    } else {
+                        bool again = false;
+                        const uint32_t x = q[k] <= heap[0] ? 0u : below + 1;
+                        if (x < m && here[k] != ~0u && heap[heap_at(x, depth)] == q[k]) {
+                            const uint32_t t = rs.c0 + x, row = (t * s.small_mul) >> s.small_shift;
+                            if (LAYOUT == TILE_BTREE && rs.level && row < SEP_SLOTS)
+                                ans = t - row * (s.b + 1) != s.b ? rs.first + x - row
+                                                                 : sep_slot[row];
+                            else
+                                ans = slot_of<LAYOUT>(r0 + x, s, map);
+                            if (x == 0 && r0 > 0)
+                                again = A[slot_of<LAYOUT>(r0 - 1, s, map)] == q[k];
+                            if (x + 1 < m) again |= heap[heap_at(x + 1, depth)] == q[k];
+                        }
+                        if (__any(again)) {
+                            const K qq[1] = {q[k]};
+                            uint32_t res[1];
+                            tile_descend<K, LAYOUT, 1>(A, s, tb, s_end, s_tidx, qq, res);
+                            if (again) ans = res[0];
+                        }
+                    }
+                    if (here[k] != ~0u) out[here[k]] = ans;
+                }
             }
-            p = qhi;
+            __syncthreads();   // the range's queries are answered
         }
+        __syncthreads();   // the last ranges' locs are read
     }
 }
 
@@ -871,8 +1073,8 @@ tl_status tile_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, 
 
 // where everything of one partitioned batch lies in its workspace
 struct PartPlan {
-    uint32_t lg1, lg2, it, tiles1, tiles2, groups;
-    uint64_t bound, bstart, tstart, rstart, gsum, counts, places, counts2, places2, pack, pack2;
+    uint32_t lg1, lg2, it, tiles1, tiles2, groups, span;
+    uint64_t bound, bstart, tstart, gsum, counts, places, loc, pack, place, found, queued, queue;
     uint64_t second, bytes;
 };
 
@@ -882,11 +1084,20 @@ static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
     while (((n + (1ull << lg) - 1) >> lg) > RANGE_KEYS) lg++;
     p.lg1 = std::min(lg, PART_LG);
     p.lg2 = lg - p.lg1;
+    if (p.lg2 && p.lg2 < 3) {   // a bucket has the ranges of a workgroup at least
+        p.lg1 -= 3 - p.lg2;
+        p.lg2 = 3;
+    }
     p.it = nq >= (1u << 22) ? 16 : 4;
     const uint64_t T = (uint64_t)PART_NT * p.it;
     p.tiles1 = (uint32_t)((nq + T - 1) / T);
     p.tiles2 = p.lg2 ? p.tiles1 + (1u << p.lg1) : 0;
     p.groups = (p.tiles1 + PART_GROUP - 1) / PART_GROUP;
+    // a share is of about as many queries as a range has keys
+    const uint64_t tiles = p.lg2 ? p.tiles2 : p.tiles1, ranges = 1ull << (p.lg2 ? p.lg2 : p.lg1);
+    const uint32_t most = p.lg2 ? PART_SPAN<true> : PART_SPAN<false>;
+    p.span = 1;
+    while (p.span < most && p.span * T < RANGE_KEYS * ranges) p.span *= 2;
     uint64_t at = 0;
     auto take = [&](uint64_t bytes) {
         const uint64_t o = at;
@@ -894,18 +1105,22 @@ static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
         return o;
     };
     p.bound = take((uint64_t)w << lg);
-    p.bstart = take(((1ull << p.lg1) + 1) * 4);
-    p.tstart = take(((1ull << p.lg1) + 1) * 4);
-    p.rstart = p.lg2 ? take(((1ull << lg) + 1) * 4) : p.bstart;
-    p.gsum = take(((uint64_t)p.groups << p.lg1) * 4);
-    p.counts = take(((uint64_t)p.tiles1 << p.lg1) * 4);
-    p.places = take(((uint64_t)p.tiles1 << p.lg1) * 4);
     if (p.lg2) {
-        p.counts2 = take(((uint64_t)p.tiles2 << p.lg2) * 4);
-        p.places2 = take(((uint64_t)p.tiles2 << p.lg2) * 4);
+        p.bstart = take(((1ull << p.lg1) + 1) * 4);
+        p.tstart = take(((1ull << p.lg1) + 1) * 4);
+        p.gsum = take(((uint64_t)p.groups << p.lg1) * 4);
+        p.counts = take(((uint64_t)p.tiles1 << p.lg1) * 4);
+        p.places = take(((uint64_t)p.tiles1 << p.lg1) * 4);
+        p.pack = take(nq * 4);
     }
-    p.pack = take(nq * 4);
-    p.pack2 = take(nq * 4);   // then the answers in the first pass's order
+    p.loc = take(tiles * ranges * 2);
+    p.place = take(nq * 2);
+    p.found = take(nq * 4);   // of two passes: in the first pass's order
+    p.queued = take(4);
+    // shares past their workgroups' own: of crowded ranges, and of buckets past
+    // their first `span` tiles
+    p.queue = take((nq / PART_SHARE + (p.lg2 ? tiles / p.span * ranges : 0) + 1) *
+                   sizeof(PartShare));
     // the queries after the second pass: behind those after the first in the
     // answer array, which has room for both when keys have 4 bytes
     p.second = p.lg2 && w == 8 ? take(nq * 8) : 0;
@@ -920,48 +1135,54 @@ uint64_t part_bytes(const TileArray &a, uint32_t dtype, uint64_t nq) {
     return part_plan(a.n, w, std::min(nq, PART_MAX_QUERIES)).bytes;
 }
 
-template <typename K, bool SECOND, int IT>
+// the first pass of two: q in bucket order to out
+template <typename K, int IT>
 static void part_pass(const PartPlan &p, const K *q, uint64_t nq, char *ws, K *out,
                       hipStream_t s) {
     uint32_t *bstart = (uint32_t *)(ws + p.bstart), *tstart = (uint32_t *)(ws + p.tstart);
-    uint32_t *counts = (uint32_t *)(ws + (SECOND ? p.counts2 : p.counts));
-    uint32_t *places = (uint32_t *)(ws + (SECOND ? p.places2 : p.places));
-    uint32_t *pack = (uint32_t *)(ws + (SECOND ? p.pack2 : p.pack));
-    uint32_t *gsum = (uint32_t *)(ws + p.gsum);
-    const uint32_t tiles = SECOND ? p.tiles2 : p.tiles1, B1 = 1u << p.lg1;
-    const dim3 grid((tiles + 7) / 8 * 8), block(PART_NT);
-    hipLaunchKernelGGL((k_part_count<K, SECOND, IT>), grid, block, 0, s, q, nq,
-                       (const K *)(ws + p.bound), p.lg1, p.lg2, (const uint32_t *)bstart,
-                       (const uint32_t *)tstart, tiles, pack, counts);
-    if (SECOND) {
-        hipLaunchKernelGGL(k_part_places2, dim3(B1), block, 0, s, (const uint32_t *)counts, p.lg1,
-                           p.lg2, (const uint32_t *)bstart, (const uint32_t *)tstart, places,
-                           (uint32_t *)(ws + p.rstart), (uint32_t *)nullptr);
-    } else {
-        hipLaunchKernelGGL(k_part_sums, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
-                           tiles, gsum);
-        hipLaunchKernelGGL(k_part_starts, dim3(1), block, 0, s, gsum, B1, p.groups,
-                           (uint32_t)(PART_NT * IT), bstart, tstart, (uint32_t *)nullptr);
-        hipLaunchKernelGGL(k_part_places, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
-                           tiles, (const uint32_t *)gsum, (const uint32_t *)bstart, places);
-    }
-    hipLaunchKernelGGL((k_part_scatter<K, SECOND, IT>), grid, block, 0, s, q, nq, p.lg1, p.lg2,
-                       (const uint32_t *)bstart, (const uint32_t *)tstart, tiles,
+    uint32_t *counts = (uint32_t *)(ws + p.counts), *places = (uint32_t *)(ws + p.places);
+    uint32_t *pack = (uint32_t *)(ws + p.pack), *gsum = (uint32_t *)(ws + p.gsum);
+    const uint32_t B1 = 1u << p.lg1;
+    const dim3 grid((p.tiles1 + 7) / 8 * 8), block(PART_NT);
+    hipLaunchKernelGGL((k_part_count<K, IT>), grid, block, 0, s, q, nq, (const K *)(ws + p.bound),
+                       p.lg1, p.lg2, p.tiles1, pack, counts);
+    hipLaunchKernelGGL(k_part_sums, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
+                       p.tiles1, gsum);
+    hipLaunchKernelGGL(k_part_starts, dim3(1), block, 0, s, gsum, B1, p.groups,
+                       (uint32_t)(PART_NT * IT), bstart, tstart, (uint32_t *)nullptr);
+    hipLaunchKernelGGL(k_part_places, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
+                       p.tiles1, (const uint32_t *)gsum, (const uint32_t *)bstart, places);
+    hipLaunchKernelGGL((k_part_scatter<K, IT>), grid, block, 0, s, q, nq, p.lg1, p.lg2, p.tiles1,
                        (const uint32_t *)places, (const uint32_t *)counts, (const uint32_t *)pack,
                        out);
 }
 
-// the answers of a pass's output order to its input order
-template <bool SECOND, int IT, typename AT>
-static void part_return(const PartPlan &p, const uint32_t *found, uint64_t nq, char *ws, AT *dst,
-                        hipStream_t s) {
+// the last pass: the queries in, tile by tile, to `tiled`, and their answers to
+// dst in the order of in
+template <typename K, int LAYOUT, bool SECOND, int IT, typename AT>
+static void part_answer(const PartPlan &p, const TileArray &a, const TileShape &sh, const K *in,
+                        uint64_t nq, char *ws, K *tiled, uint32_t *found, AT *dst, hipStream_t s) {
+    const uint32_t *bstart = (const uint32_t *)(ws + p.bstart);
+    const uint32_t *tstart = (const uint32_t *)(ws + p.tstart);
+    uint16_t *place = (uint16_t *)(ws + p.place), *loc = (uint16_t *)(ws + p.loc);
+    uint32_t *queued = (uint32_t *)(ws + p.queued);
+    PartShare *queue = (PartShare *)(ws + p.queue);
     const uint32_t tiles = SECOND ? p.tiles2 : p.tiles1;
-    hipLaunchKernelGGL((k_part_return<SECOND, IT, AT>), dim3((tiles + 7) / 8 * 8), dim3(PART_NT), 0,
-                       s, found, nq, p.lg1, p.lg2, (const uint32_t *)(ws + p.bstart),
-                       (const uint32_t *)(ws + p.tstart), tiles,
-                       (const uint32_t *)(ws + (SECOND ? p.places2 : p.places)),
-                       (const uint32_t *)(ws + (SECOND ? p.counts2 : p.counts)),
-                       (const uint32_t *)(ws + (SECOND ? p.pack2 : p.pack)), dst);
+    const dim3 grid((tiles + 7) / 8 * 8), block(PART_NT);
+    hipLaunchKernelGGL((k_part_tile<K, SECOND, IT>), grid, block, 0, s, in, nq,
+                       (const K *)(ws + p.bound), p.lg1, p.lg2, bstart, tstart, tiles, place, loc,
+                       tiled);
+    const PartLoc pl{p.lg1, p.lg2, (uint32_t)(PART_NT * IT), (uint32_t)nq, tiles, p.span,
+                     bstart, tstart, loc};
+    const uint32_t units = SECOND ? (1u << (p.lg1 + p.lg2)) / PART_RANGES<true>
+                                  : ((tiles + p.span - 1) / p.span) << p.lg1;
+    hipLaunchKernelGGL((k_part_answer<K, LAYOUT, SECOND, false>), dim3((units + 7) / 8 * 8),
+                       dim3(RANGE_NT), 0, s, (const K *)a.A, sh, pl, units, (const K *)tiled,
+                       queued, queue, found);
+    hipLaunchKernelGGL((k_part_answer<K, LAYOUT, SECOND, true>), dim3(1024), dim3(RANGE_NT), 0, s,
+                       (const K *)a.A, sh, pl, units, (const K *)tiled, queued, queue, found);
+    hipLaunchKernelGGL((k_part_back<SECOND, IT, AT>), grid, block, 0, s, (const uint32_t *)found,
+                       nq, p.lg1, p.lg2, bstart, tstart, tiles, (const uint16_t *)place, dst);
 }
 
 template <typename K, int LAYOUT, int IT>
@@ -970,25 +1191,21 @@ static void part_segment(const PartPlan &p, const TileArray &a, const K *q, uint
     using W = typename std::conditional<sizeof(K) == 4, uint32_t, uint64_t>::type;
     const TileShape sh = tile_shape(a);
     const uint32_t lg = p.lg1 + p.lg2;
-    const uint32_t chunks = (uint32_t)((nq + RANGE_CHUNK - 1) / RANGE_CHUNK);
     hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256), dim3(256), 0, s,
-                       (const W *)a.A, sh, lg, (W *)(ws + p.bound));
-    K *first = (K *)ans, *sorted = first;
-    uint32_t *found = (uint32_t *)(ws + p.pack2);
-    part_pass<K, false, IT>(p, q, nq, ws, first, s);
-    if (p.lg2) {
-        sorted = sizeof(K) == 4 ? first + nq : (K *)(ws + p.second);
-        part_pass<K, true, IT>(p, first, nq, ws, sorted, s);
-        found = (uint32_t *)ans;
+                       (const W *)a.A, sh, lg, (W *)(ws + p.bound), (uint32_t *)(ws + p.queued));
+    uint32_t *found = (uint32_t *)(ws + p.found);
+    K *first = (K *)ans;   // the answer array holds queries meanwhile
+    if (!p.lg2) {
+        part_answer<K, LAYOUT, false, IT>(p, a, sh, q, nq, ws, first, found, ans, s);
+        return;
     }
-    hipLaunchKernelGGL((k_part_answer<K, LAYOUT>), dim3((chunks + 7) / 8 * 8), dim3(RANGE_NT), 0,
-                       s, (const K *)a.A, sh, lg, (const K *)sorted, (uint32_t)nq,
-                       (const uint32_t *)(ws + p.rstart), chunks, found);
-    if (p.lg2) {
-        part_return<true, IT>(p, found, nq, ws, (uint32_t *)(ws + p.pack2), s);
-        found = (uint32_t *)(ws + p.pack2);
-    }
-    part_return<false, IT>(p, found, nq, ws, ans, s);
+    part_pass<K, IT>(p, q, nq, ws, first, s);
+    K *tiled = sizeof(K) == 4 ? first + nq : (K *)(ws + p.second);
+    part_answer<K, LAYOUT, true, IT>(p, a, sh, first, nq, ws, tiled, (uint32_t *)ans, found, s);
+    hipLaunchKernelGGL((k_part_return<IT>), dim3((p.tiles1 + 7) / 8 * 8), dim3(PART_NT), 0, s,
+                       (const uint32_t *)found, nq, p.lg1, p.lg2, p.tiles1,
+                       (const uint32_t *)(ws + p.places), (const uint32_t *)(ws + p.counts),
+                       (const uint32_t *)(ws + p.pack), ans);
 }
 
 template <typename K, int LAYOUT>
@@ -1063,46 +1280,57 @@ bool part_can(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
 }
 
 // Time of a batch in picoseconds by each path, from lookups of uniform keys
-// measured on arrays of 2^14 .. 2^28 keys of both widths: a start-up, and per
-// query a figure that grows with the array's bytes (2^16, 2^18 .. 2^32).
+// measured on arrays of 2^12 .. 2^28 keys of both widths, nodes of 1 to 33 keys
+// and 2^19 .. 2^26 queries: a start-up, and per query a figure that grows with
+// the array's bytes (2^16, 2^18 .. 2^32).
 struct PathCost {
     double start;
     uint16_t query[9];
 };
-static double path_ps(const PathCost &c, uint64_t n, uint32_t w, uint64_t nq, double more = 0) {
+static double path_ps(const PathCost &c, uint64_t n, uint32_t w, uint64_t nq) {
     const double l = std::min(16.0, std::max(0.0, log2((double)n * w) - 16)) / 2;
     const int i = std::min(7, (int)l);
-    const double q = c.query[i] + (c.query[i + 1] - c.query[i]) * (l - i);
-    return c.start + (double)nq * std::max(1.0, q + more);
+    return c.start + (double)nq * (c.query[i] + (c.query[i + 1] - c.query[i]) * (l - i));
 }
 
-// the kernels of tl_query.hip, and the tile-sorted descents.  The wide B-tree
-// descent's cost is its lanes': 5 ps more a query for each lane of a node
-// past two.  A partitioned batch reads every range (2.3 ps a key, slots and
-// all) and moves every query 18 ps worth a pass, whatever the layout.
+// the kernels of tl_query.hip but the B-trees' (entry TILE_BTREE is not used)
 static const PathCost COST_OLD[] = {{8e6, {13, 15, 20, 28, 45, 75, 112, 152, 190}},
-                                    {5e6, {18, 22, 22, 26, 27, 32, 44, 57, 70}},
+                                    {0, {0, 0, 0, 0, 0, 0, 0, 0, 0}},
                                     {8e6, {27, 33, 39, 45, 58, 71, 90, 129, 160}},
-                                    {12e6, {13, 22, 31, 40, 122, 197, 248, 290, 330}}};
-static const PathCost COST_GROUP = {5e6, {38, 44, 48, 53, 63, 64, 75, 90, 105}};
+                                    {14e6, {9, 19, 31, 41, 115, 192, 245, 285, 310}}};
+// the tile-sorted descents, 2^20 queries at least: fewer don't fill the device
 static const PathCost COST_TILE[] = {{12e6, {7, 8, 11, 17, 33, 73, 110, 148, 185}},
-                                     {22e6, {15, 18, 22, 32, 45, 76, 124, 180, 240}},
-                                     {38e6, {21, 27, 31, 37, 50, 76, 103, 144, 180}},
-                                     {12e6, {8, 15, 26, 37, 89, 162, 211, 259, 300}}};
+                                     {14e6, {16, 18, 24, 33, 50, 84, 126, 165, 210}},
+                                     {24e6, {21, 25, 27, 38, 50, 74, 103, 144, 180}},
+                                     {8e6, {6, 10, 22, 36, 85, 155, 205, 255, 290}}};
 
+static double tile_ps(const TileArray &a, uint32_t w, uint64_t nq) {
+    return path_ps(COST_TILE[a.layout], a.n, w, std::max<uint64_t>(nq, 1u << 20));
+}
+
+// A B-tree's descent costs its lanes' instructions on every level (wide: 1.3 ps
+// a lane of 8-byte keys, 1.9 of 4-byte keys; else about one), or, where that is
+// more, the lines of the levels past one L2's 4 MB, 19 ps each.
 static double old_ps(const TileArray &a, uint32_t w, uint64_t nq) {
     if (a.layout != TILE_BTREE) return path_ps(COST_OLD[a.layout], a.n, w, nq);
     if (a.b > 64) return 5e6 + (double)nq * 4.0 * a.b;   // one lane scans the nodes
     if (a.b == 1) return path_ps(COST_OLD[TILE_BST], a.n, w, nq);
-    if (wide_ok(a.A, a.b, w))
-        return path_ps(COST_OLD[TILE_BTREE], a.n, w, nq, 5.0 * wide_group(a.b, w) - 10.0);
-    return path_ps(COST_GROUP, a.n, w, nq);
+    uint32_t group = 2;
+    while (group < a.b) group *= 2;
+    const double level =
+        wide_ok(a.A, a.b, w) ? wide_group(a.b, w) * (w == 8 ? 1.3 : 1.9) : group * 0.95;
+    const double per_level = log2((double)a.b + 1);
+    const double lanes = 1 + level * ceil(log2((double)a.n + 1) / per_level);
+    const double lines = 8 + 19 * (log2((double)a.n * w) - 22) / per_level;
+    return 6e6 + (double)nq * std::max(lanes, lines);
 }
 
+// the partitioned batch, whatever the layout: each query's moves, and every
+// range read (with two passes mostly slots and latency)
 static double part_ps(const TileArray &a, uint32_t w, uint64_t nq) {
-    const uint32_t passes = part_plan(a.n, w, std::min(nq, PART_MAX_QUERIES)).lg2 ? 2 : 1;
+    const bool two = part_plan(a.n, w, std::min(nq, PART_MAX_QUERIES)).lg2 != 0;
     const uint64_t segments = (nq + PART_MAX_QUERIES - 1) / PART_MAX_QUERIES;
-    return segments * (50e6 * passes + 2.3 * a.n) + (double)nq * 18 * passes;
+    return segments * (two ? 55e6 + 2.6 * a.n : 30e6 + 1.0 * a.n) + (double)nq * (two ? 25 : 12.5);
 }
 
 Workspace &query_workspace() {
@@ -1123,7 +1351,8 @@ bool part_wanted(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
     const int f = forced_path();
     if (f >= 0) return f == 2;
     const uint32_t w = key_width(dtype);
-    return part_ps(a, w, nq) < other * std::min(old_ps(a, w, nq), path_ps(COST_TILE[a.layout], a.n, w, nq));
+    // (the figures are good to a tenth; near a draw the plain path stays)
+    return part_ps(a, w, nq) < other * std::min(0.9 * old_ps(a, w, nq), 0.95 * tile_ps(a, w, nq));
 }
 
 tl_status part_try(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
@@ -1151,7 +1380,7 @@ tl_status large_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q,
     if (*taken || !tile_can(a, dtype, nq)) return TL_OK;
     const int f = forced_path();
     const uint32_t w = key_width(dtype);
-    if (f == 0 || (f < 0 && path_ps(COST_TILE[a.layout], a.n, w, nq) >= old_ps(a, w, nq)))
+    if (f == 0 || (f < 0 && tile_ps(a, w, nq) >= 0.9 * old_ps(a, w, nq)))
         return TL_OK;
     *taken = true;
     return tile_query(c, a, dtype, q, nq, ans, s);
