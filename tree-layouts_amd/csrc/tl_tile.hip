@@ -1075,7 +1075,7 @@ tl_status tile_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, 
 struct PartPlan {
     uint32_t lg1, lg2, it, tiles1, tiles2, groups, span;
     uint64_t bound, bstart, tstart, gsum, counts, places, loc, pack, place, found, queued, queue;
-    uint64_t second, bytes;
+    uint64_t second, most, bytes;   // most: shares on the queue
 };
 
 static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
@@ -1119,8 +1119,8 @@ static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
     p.queued = take(4);
     // shares past their workgroups' own: of crowded ranges, and of buckets past
     // their first `span` tiles
-    p.queue = take((nq / PART_SHARE + (p.lg2 ? tiles / p.span * ranges : 0) + 1) *
-                   sizeof(PartShare));
+    p.most = nq / PART_SHARE + (p.lg2 ? tiles / p.span * ranges : 0) + 1;
+    p.queue = take(p.most * sizeof(PartShare));
     // the queries after the second pass: behind those after the first in the
     // answer array, which has room for both when keys have 4 bytes
     p.second = p.lg2 && w == 8 ? take(nq * 8) : 0;
@@ -1179,7 +1179,8 @@ static void part_answer(const PartPlan &p, const TileArray &a, const TileShape &
     hipLaunchKernelGGL((k_part_answer<K, LAYOUT, SECOND, false>), dim3((units + 7) / 8 * 8),
                        dim3(RANGE_NT), 0, s, (const K *)a.A, sh, pl, units, (const K *)tiled,
                        queued, queue, found);
-    hipLaunchKernelGGL((k_part_answer<K, LAYOUT, SECOND, true>), dim3(1024), dim3(RANGE_NT), 0, s,
+    hipLaunchKernelGGL((k_part_answer<K, LAYOUT, SECOND, true>),
+                       dim3((uint32_t)std::min<uint64_t>(p.most, 1024)), dim3(RANGE_NT), 0, s,
                        (const K *)a.A, sh, pl, units, (const K *)tiled, queued, queue, found);
     hipLaunchKernelGGL((k_part_back<SECOND, IT, AT>), grid, block, 0, s, (const uint32_t *)found,
                        nq, p.lg1, p.lg2, bstart, tstart, tiles, (const uint16_t *)place, dst);
