@@ -755,9 +755,9 @@ static tl_status run_direct(Ctx *c, Layout lay, W *A, uint64_t n, uint64_t b, bo
 // sweeps from the left.
 // Bound by memory: 2 n keys are moved, and 2 more for each that is stashed (a
 // BST's n/4 to n/2, few of most B-trees); gathering level by level moved 4 to 9
-// for each key.  Plan -> now, forward: BST of 5*10^8 4-byte keys 6.18 -> 1.23 ms
-// (5 TB/s), of 2^30 8-byte keys 7.25 -> 4.87 ms; B-tree b=16 of 2^30 8-byte keys
-// 7.22 -> 4.18 ms (5.5 TB/s); b=8 of 2*10^8 4-byte keys 2.06 -> 0.39 ms, its
+// for each key.  Plan -> now, forward: BST of 5*10^8 4-byte keys 6.18 -> 1.14 ms
+// (5.4 TB/s), of 2^30 8-byte keys 7.25 -> 4.87 ms; B-tree b=16 of 2^30 8-byte keys
+// 7.22 -> 4.06 ms (5.9 TB/s); b=8 of 2*10^8 4-byte keys 2.06 -> 0.39 ms, its
 // inverse 2.10 -> 0.41.
 // Faster than the plan at every size and b measured past DIRECT_BYTES.
 // Tiles of 64 KB: tickets come from one counter at about 66 a us, which bounds
@@ -1062,7 +1062,8 @@ __global__ __launch_bounds__(SLIDE_NT) void k_level_slide(W *__restrict__ A, W *
 }
 
 // dst[0, count) = src[0, count), 16 bytes a lane and load where both have the
-// same place in a 16-byte line
+// same place in a 16-byte line.  A workgroup's four loads a lane are neighbours: a
+// grid apart they took 1.39 ms for 2.95 GB, now 1.26.
 template <typename W>
 __global__ __launch_bounds__(256) void k_copy_wide(W *__restrict__ dst, const W *__restrict__ src,
                                                    uint64_t count) {
@@ -1075,14 +1076,15 @@ __global__ __launch_bounds__(256) void k_copy_wide(W *__restrict__ dst, const W 
         wide = (count - head) / V;
         const uint4 *s = (const uint4 *)(src + head);
         uint4 *d = (uint4 *)(dst + head);
-        for (uint64_t i = i0; i < wide; i += 4 * step) {
+        const uint64_t first = (uint64_t)blockIdx.x * (4 * blockDim.x) + threadIdx.x;
+        for (uint64_t i = first; i < wide; i += 4 * step) {
             uint4 v[4];
 #pragma unroll
             for (int k = 0; k < 4; k++)
-                if (i + k * step < wide) v[k] = s[i + k * step];
+                if (i + k * blockDim.x < wide) v[k] = s[i + k * blockDim.x];
 #pragma unroll
             for (int k = 0; k < 4; k++)
-                if (i + k * step < wide) d[i + k * step] = v[k];
+                if (i + k * blockDim.x < wide) d[i + k * blockDim.x] = v[k];
         }
     }
     for (uint64_t i = i0; i < head; i += step) dst[i] = src[i];
