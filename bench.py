@@ -451,9 +451,21 @@ def time_unpermute(args, A, layout, b, stream):
     return ev0.elapsed_time(ev1) / args.steps
 
 
+def permute_traffic(layout, n, b=1):
+    """HBM bytes of one permute call as the library does it by default at n =
+    2^30 (BST, B-tree b=16: the one-pass slide), or with TL_PERMUTE_PLAN set,
+    from the committed PMC summaries; None for other sizes and layouts"""
+    name = f"btree_b{b}" if layout == "btree" else layout
+    if n != 1 << 30 or name not in ("bst", "btree_b16", "mveb"):
+        return None
+    kind = "permute" if layout == "mveb" or "TL_PERMUTE_PLAN" in os.environ else "slide"
+    t = measured_traffic(f"{name}_n2p30_u64_{kind}_traffic.txt")
+    return None if t is None else round(t)
+
+
 def layout_traffic(layout, n):
-    """HBM bytes per permute call of the BST or mvEB at n = 2^30 from the
-    committed PMC summaries (None for other sizes and layouts)"""
+    """HBM bytes per permute call by plan of the BST or mvEB at n = 2^30 from
+    the committed PMC summaries (None for other sizes and layouts)"""
     if n != 1 << 30 or layout not in ("bst", "mveb"):
         return None
     t = measured_traffic(f"{layout}_n2p30_u64_permute_traffic.txt")
@@ -507,7 +519,7 @@ def other_layouts(args, A, keys, stream, rng, samples=20_000):
         utotal, _ = event_steps(lambda: tl_amd.unpermute(layout, A, kind="u64", timed=False),
                                 steps, stream)
         ums = utotal / steps
-        traffic = layout_traffic(layout, n)
+        traffic = permute_traffic(layout, n)
         out[layout] = {"ms": round(ms, 4), "Gkeys_s": round(n / (ms * 1e-3) / 1e9, 3),
                        "algorithmic_frac": round(2.0 * n * 8 / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                        "traffic": traffic,
@@ -614,7 +626,7 @@ def run_layout(args, dev, layout):
         "checks": {"layout_sample": layout_ok, "answers": ok},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": layout_traffic(layout, n),
+                     "traffic": permute_traffic(layout, n),
                      "kernel": f"whole tl_permute_{layout} call (all its launches)"},
         "cpu_baseline": None,
     }
@@ -837,9 +849,7 @@ def main():
 
     algo_bytes = 2.0 * n * 8
     achieved = algo_bytes / (perm_ms * 1e-3) / 1e9
-    traffic = None
-    if n == 1 << 30 and b == 16:
-        traffic = measured_traffic("btree_b16_n2p30_u64_permute_traffic.txt")
+    traffic = permute_traffic("btree", n, b)
     queries = {"plain_ms": round(q_ms, 4), "plain_Mq_s": round(nq / q_ms / 1e3, 2),
                "plain_timings": timing_stats(nq, q_per, 1e-6),
                "plain_roofline": qroof(q_ms, "plain"),
@@ -882,7 +892,7 @@ def main():
                      "traffic_frac": None if traffic is None
                      else round(traffic / (perm_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "kernel": "one tl_permute_btree call (all its launches); traffic from "
-                               "profiles/btree_b16_n2p30_u64_permute_traffic.txt"},
+                               "profiles/btree_b16_n2p30_u64_slide_traffic.txt"},
         "cpu_baseline": None if cpu is None else {
             "value": round(cpu["permute"]["tp_mean"], 4), "unit": "Gkeys/s",
             "cores": cpu["cores"], "kind": cpu["kind"],
