@@ -3,7 +3,8 @@
 // exactly sized buffers under AddressSanitizer.  Every answer is compared with
 // the CPU oracle's search (the reference's visiting order), with distinct
 // keys and with keys that repeat.  Arguments: layout (bst, btree, mveb, veb,
-// binary), key type (u32, u64, i32, i64), b, queries, then array sizes.
+// binary; veb-as-mveb, mveb-as-veb: a layout and its tables, given to the other
+// one's query), key type (u32, u64, i32, i64), b, queries, then array sizes.
 #include "hip/hip_runtime.h"
 #include "src/tl_tile.hpp"
 #include "tl_oracle.h"
@@ -53,7 +54,7 @@ static uint64_t check(const std::string &lay, uint32_t dtype, uint64_t n, uint64
         else or_permute_btree_u64((uint64_t *)A, n, b, 1);
     } else if (lay != "binary") {
         a.layout = TILE_VEB;
-        a.classic = lay == "veb";
+        a.classic = lay.substr(0, 3) == "veb";
         if (a.classic) {
             if (sizeof(T) == 4) or_permute_classic_u32((uint32_t *)A, n, 1);
             else or_permute_classic_u64((uint64_t *)A, n, 1);
@@ -66,6 +67,7 @@ static uint64_t check(const std::string &lay, uint32_t dtype, uint64_t n, uint64
         a.tables = (const tl_veb_table *)tables.data();
         a.idx = idx;
         a.tidx = tidx;
+        if (lay.find("-as-") != std::string::npos) a.classic = !a.classic;
     }
     uint64_t *got = (uint64_t *)malloc(nq * 8), *want = (uint64_t *)malloc(nq * 8);
     uint64_t bad = 0;
@@ -118,8 +120,8 @@ int main(int argc, char **argv) {
     if (kind == #KIND)                                                                           \
         bad += check<T>(lay, DT, n, b, nq, repeats,                                              \
                         lay == "bst"    ? or_search_bst_##KIND                                   \
-                        : lay == "mveb" ? or_search_mveb_##KIND                                  \
-                        : lay == "veb"  ? or_search_classic_##KIND                               \
+                        : lay[0] == 'm' ? or_search_mveb_##KIND                                  \
+                        : lay[0] == 'v' ? or_search_classic_##KIND                               \
                                         : or_search_binary_##KIND,                               \
                         or_search_btree_##KIND);
             RUN(u32, uint32_t, TL_U32)

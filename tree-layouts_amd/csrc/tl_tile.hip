@@ -380,7 +380,48 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
 
 constexpr uint32_t RANGE_NT = 512;
 
-// bound[j]: the smallest key of range j; the queue is empty
+// whether the caller's vEB table set is the one of this layout (the whole
+// workgroup calls it): of every structure the end and, level by level, the L, R
+// and D that the splits give
+__device__ inline bool veb_tables_match(const TileShape &s) {
+    __shared__ uint32_t differs;
+    if (threadIdx.x == 0) differs = 0;
+    __syncthreads();
+    uint32_t off = 0;
+    bool same = true;
+    for (uint32_t j = 0; j < s.ntables; j++) {
+        uint32_t end = s.n;
+        if (j + 1 < s.ntables) {
+            const VebLevel e = s.chain[j];
+            end = off + (1u << e.rd) - 1 + e.nf * ((1u << e.ld) - 1);
+        }
+        const uint32_t d = 32u - (uint32_t)__clz((int)(s.n - off));
+        const uint32_t at = s.tidx ? s.tidx[j] : 0u;
+        if (off >= end || (s.idx ? s.idx[j] : s.n) != end || (uint64_t)at + d > s.table_size) {
+            same = false;
+            break;
+        }
+        for (uint32_t t = threadIdx.x + 1; t < d; t += blockDim.x) {
+            uint32_t base = 0, levels = d, rd, ld;
+            for (;;) {   // down to the tree whose bottom trees start at level t
+                veb_split(levels, rd, ld, s.classic != 0);
+                if (t == base + rd) break;
+                levels = t < base + rd ? rd : ld;
+                base += t < base + rd ? 0u : rd;
+            }
+            const tl_veb_table e = s.tables[at + t];
+            same = same && e.L == (1ull << ld) - 1 && e.R == (1ull << rd) - 1 && e.D == base;
+        }
+        off = end;
+    }
+    if (!same) differs = 1;
+    __syncthreads();
+    return !differs;
+}
+
+// bound[j]: the smallest key of range j; the queue is empty.  queued[1]: a vEB's
+// table set is another layout's than the call's (the answers then follow the
+// tables, as those of every other path do).
 template <typename W, int LAYOUT>
 __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, TileShape s,
                                                      uint32_t lg, W *__restrict__ bound,
@@ -388,7 +429,14 @@ __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, Ti
     __shared__ SlotMap<LAYOUT> map;
     slot_map<LAYOUT>(s, map);
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j == 0) *queued = 0;
+    if (blockIdx.x == 0) {
+        bool same = true;
+        if constexpr (LAYOUT == TILE_VEB) same = veb_tables_match(s);
+        if (j == 0) {
+            queued[0] = 0;
+            queued[1] = same ? 0u : 1u;
+        }
+    }
     if (j < (1u << lg)) bound[j] = A[slot_of<LAYOUT>(range_first(j, s.n, lg), s, map)];
 }
 
@@ -844,7 +892,9 @@ struct PartLoc {
 // tiles (SECOND: of the ranges' bucket); whatever is more, where queries crowd,
 // it puts on the queue, whose shares the second launch (REST) takes.  A key that
 // occurs more than once is answered by the descent itself, whose first equal key
-// it has to be.
+// it has to be, and so is every query where queued[1] says that the ranks' slots
+// are not those of the caller's vEB tables (a classic table set given to an mvEB
+// query, say): the partition then only orders the queries.
 // Registers: at most 64 for a vEB, so that four workgroups share a compute unit
 // (3.25 -> 3.08 ms); the others are faster with what they ask for (5.16 -> 4.85).
 template <typename K, int LAYOUT, bool SECOND, bool REST>
@@ -871,6 +921,7 @@ __global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_a
     uint32_t unit = REST ? blockIdx.x : xcd_tile(units);
     const uint32_t shares = REST ? *queued : units;
     if (unit >= shares) return;
+    const bool by_tables = LAYOUT == TILE_VEB && queued[1] != 0;
     if constexpr (LAYOUT == TILE_VEB) {
         for (uint32_t i = tid; i < s.table_size; i += RANGE_NT)
             tb[i] = {(uint32_t)s.tables[i].L, (uint32_t)s.tables[i].R, s.tables[i].D};
@@ -986,7 +1037,7 @@ __global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_a
                     if constexpr (LAYOUT == TILE_SORTED) {
                         if (heap[0] <= q[k]) ans = r0 + below;
                     } else {
-                        bool again = false;
+                        bool again = by_tables && here[k] != ~0u;
                         const uint32_t x = q[k] <= heap[0] ? 0u : below + 1;
                         if (x < m && here[k] != ~0u && heap[heap_at(x, depth)] == q[k]) {
                             const uint32_t t = rs.c0 + x, row = (t * s.small_mul) >> s.small_shift;
@@ -996,7 +1047,7 @@ __global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_a
                             else
                                 ans = slot_of<LAYOUT>(r0 + x, s, map);
                             if (x == 0 && r0 > 0)
-                                again = A[slot_of<LAYOUT>(r0 - 1, s, map)] == q[k];
+                                again |= A[slot_of<LAYOUT>(r0 - 1, s, map)] == q[k];
                             if (x + 1 < m) again |= heap[heap_at(x + 1, depth)] == q[k];
                         }
                         if (__any(again)) {
@@ -1116,7 +1167,7 @@ static PartPlan part_plan(uint64_t n, uint32_t w, uint64_t nq) {
     p.loc = take(tiles * ranges * 2);
     p.place = take(nq * 2);
     p.found = take(nq * 4);   // of two passes: in the first pass's order
-    p.queued = take(4);
+    p.queued = take(8);
     // shares past their workgroups' own: of crowded ranges, and of buckets past
     // their first `span` tiles
     p.most = nq / PART_SHARE + (p.lg2 ? tiles / p.span * ranges : 0) + 1;
