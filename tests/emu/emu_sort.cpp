@@ -13,6 +13,8 @@
 #include <unistd.h>
 #include <vector>
 
+int emu_fallbacks, emu_large;   // runs that ended in the radix sort; large buckets
+
 template <typename T>
 static int run(tl_dtype dt, uint64_t n) {
     static const char *names[] = {"wide", "narrow", "heavy", "equal", "sorted", "reverse", "crowds"};
@@ -34,11 +36,12 @@ static int run(tl_dtype dt, uint64_t n) {
         T *a = (T *)malloc(n * sizeof(T));
         std::copy(in.begin(), in.end(), a);
         uint64_t m = 0;
+        emu_fallbacks = emu_large = 0;
         const tl_status st = tl_sort_dedupe(a, n, dt, &m, nullptr, nullptr);
         const bool ok = st == TL_OK && m == want.size() && std::equal(want.begin(), want.end(), a);
-        fprintf(stderr, "[emu-sort] %s dtype %d n=%llu: status %d, %llu of %zu distinct, %s\n",
+        fprintf(stderr, "[emu-sort] %s dtype %d n=%llu: status %d, %llu of %zu distinct, %d fallback, %d large, %s\n",
                 names[d], (int)dt, (unsigned long long)n, (int)st, (unsigned long long)m,
-                want.size(), ok ? "right" : "WRONG");
+                want.size(), emu_fallbacks, emu_large, ok ? "right" : "WRONG");
         bad += !ok;
         free(a);
     }

@@ -3,19 +3,25 @@
 // the sorted, distinct input every layout assumes (the reference's drivers
 // build such input themselves, cpu/src/common.h:33-40).
 //
-// Splitter sort.  The keys are partitioned into buckets of about 1000 by
-// splitters from samples, in one pass (1024 buckets) or two, each a count and
-// a scatter whose tile leaves LDS in bucket order; a bucket is then sorted in
-// LDS by one workgroup and its repeats dropped, and one pass closes the gaps.
-// Whatever the key width and range, every key moves four times (the digits of
-// a radix sort move it once per 8 bits that vary: 100 million 40-bit keys took
-// five passes at 1.0 ms and 6.2 ms in all; now 3.1 ms, as many of 62 bits).  A key equal to a splitter is not partitioned but
-// noted with it, so a key that repeats often costs nothing, however often.
+// Splitter sort.  The keys are partitioned into buckets of 768 to 1536 on
+// average by splitters from samples, in one pass (1024 buckets) or two, each a
+// count and a scatter whose tile leaves LDS in bucket order; a bucket is then
+// sorted in LDS by one workgroup and its repeats dropped, and one pass closes the
+// gaps.  Whatever the key width and range, every key moves four times (the digits
+// of a radix sort move it once per 8 bits that vary: 100 million 40-bit keys took
+// five passes at 1.0 ms and 6.2 ms in all; now 3.1 ms, as many of 62 bits).  A key
+// equal to a splitter is not partitioned but noted with it, so a key that repeats
+// often costs nothing, however often.
 //
-// Bucket sizes are the samples' luck.  Where one does not fit (it never has,
-// by the samples' numbers), nothing has been lost: the partitioned keys and
-// the noted splitters are the input's distinct keys and some repeats, and the
-// radix sort below takes over from them.  It also serves the largest arrays.
+// Bucket sizes are the samples' luck: with m samples to a splitter, a bucket is
+// its average times a Gamma(m) / m of each pass.  For distinct keys in random
+// order 4096 are passed by 0.7 buckets of 2*10^8 keys and by 1.6 of 4*10^8 (32 and
+// 32 samples, an average of 1530), by 0.01 of 10^8 and by fewer below; those few
+// are sorted by larger workgroups.  16384 are passed by fewer than 10^-27.  Inputs
+// made to (or whose repeats lie where no sample does) still can: nothing has been
+// lost then, the partitioned keys and the noted splitters are the input's distinct
+// keys and some repeats, and the radix sort below takes over from them.  It also
+// serves the largest arrays.
 //
 // LSD radix sort, 8-bit digits, stable, ping-ponging between the caller's
 // array and one library-owned buffer of n keys.  Signed keys sort by their
@@ -295,8 +301,10 @@ static tl_status scan_u32(uint32_t *v, uint64_t len, uint32_t *sums, hipStream_t
 // the splitter sort
 
 constexpr uint32_t RANGE_NT = 512, RANGE_IT = 8;
-constexpr uint32_t RANGE_CAP = RANGE_NT * RANGE_IT;   // keys of a bucket, at most
-constexpr uint32_t RANGE_GOAL = 1536;                 // ... on average
+constexpr uint32_t RANGE_CAP = RANGE_NT * RANGE_IT;   // keys of a bucket, mostly
+constexpr uint32_t LARGE_NT = 1024, LARGE_IT = 16;
+constexpr uint32_t LARGE_CAP = LARGE_NT * LARGE_IT;   // ... at most
+constexpr uint32_t RANGE_GOAL = 1536;                 // ... on average, fewer than
 constexpr uint32_t RANGE_BINS = 2048;
 constexpr uint32_t SORT_LG1 = 8;   // log2 of the first of two passes' buckets
 constexpr uint64_t SPLIT_MAX_KEYS = 1ull << 29;       // 2^10 and 2^9 buckets
@@ -564,7 +572,8 @@ __device__ inline U wave_extreme(U v) {
 // presence to kept[j].  One counting pass over 2048 equal parts of the bucket's
 // span leaves a key or two in each, which find their order by comparing.
 // Buckets whose keys crowd are left (kept[j] = CROWDED) to a second launch,
-// which sorts all their digits (and needs the registers for it).
+// which sorts all their digits (and needs the registers for it), and those of more
+// than RANGE_CAP keys (noted in large[]) to a third.
 constexpr uint32_t CROWDED = ~0u;
 template <typename K, bool CROWD_PASS>
 __global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
@@ -572,7 +581,9 @@ __global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
                                                          const uint32_t *__restrict__ rcount,
                                                          const uint32_t *__restrict__ present,
                                                          K *out, uint32_t *__restrict__ kept,
-                                                         uint32_t *__restrict__ overflow) {
+                                                         uint32_t *__restrict__ overflow,
+                                                         uint32_t *__restrict__ nlarge,
+                                                         uint32_t *__restrict__ large) {
     using U = Bits<K>;
     constexpr uint32_t CROWD = 32, NW = RANGE_NT / 64;
     __shared__ U buf[RANGE_CAP];
@@ -585,7 +596,8 @@ __global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
     if (cnt == 0 || cnt > RANGE_CAP) {
         if (tid == 0) {
             kept[j] = present[j];
-            if (cnt) *overflow = 1;
+            if (cnt > LARGE_CAP) *overflow = 1;
+            else if (cnt) large[atomicAdd(nlarge, 1u)] = j;
         }
         return;
     }
@@ -726,6 +738,57 @@ __global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
     if (tid == 0) kept[j] = total + present[j];
 }
 
+// The buckets of more than RANGE_CAP keys, LARGE_CAP at most: all their digits in
+// the LDS of a whole compute unit.  A bucket or two of inputs whose average is
+// near the goal: five of eight sets of 2*10^8 8-byte keys had one, and took 24.3 ms
+// by the radix sort of everything where the others took 6.1; now all take 6.1.
+template <typename K>
+__global__ __launch_bounds__(LARGE_NT) void k_sort_large(const K *__restrict__ S,
+                                                         const uint32_t *__restrict__ rstart,
+                                                         const uint32_t *__restrict__ rcount,
+                                                         const uint32_t *__restrict__ present,
+                                                         K *__restrict__ out,
+                                                         uint32_t *__restrict__ kept,
+                                                         const uint32_t *__restrict__ nlarge,
+                                                         const uint32_t *__restrict__ large) {
+    using U = Bits<K>;
+    constexpr uint32_t NW = LARGE_NT / 64;
+    __shared__ U buf[LARGE_CAP];
+    __shared__ uint32_t hist[NW * 256], wsum[NW], wcount[LARGE_IT * NW];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, m = *nlarge;
+    for (uint32_t l = blockIdx.x; l < m; l += gridDim.x) {
+        const uint32_t j = large[l], lo = rstart[j], cnt = rcount[j];
+        for (uint32_t i = tid; i < cnt; i += LARGE_NT) buf[i] = to_bits<K>(S[lo + i]);
+        __syncthreads();
+        lds_sort<U, LARGE_NT, LARGE_IT>(buf, cnt, hist, wsum);
+        // distinct keys in order: 64 at a time, (k, wave) after (k, wave)
+        uint32_t place[LARGE_IT];
+        uint32_t keep = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < LARGE_IT; k++) {
+            const uint32_t i = k * LARGE_NT + tid;
+            const bool first = i < cnt && (i == 0 || buf[i] != buf[i - 1]);
+            const uint64_t peers = __ballot(first);
+            place[k] = (uint32_t)__popcll(peers & ((1ull << lane) - 1));
+            keep |= first ? 1u << k : 0u;
+            if (lane == 0) wcount[k * NW + w] = (uint32_t)__popcll(peers);
+        }
+        __syncthreads();
+        static_assert(LARGE_IT * NW <= LARGE_NT, "one count a lane");
+        uint32_t total;
+        const uint32_t mine = tid < LARGE_IT * NW ? wcount[tid] : 0u;
+        const uint32_t before = block_scan(mine, wsum, &total);
+        if (tid < LARGE_IT * NW) wcount[tid] = before;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < LARGE_IT; k++)
+            if (keep >> k & 1)
+                out[lo + wcount[k * NW + w] + place[k]] = from_bits<K>(buf[k * LARGE_NT + tid]);
+        if (tid == 0) kept[j] = total + present[j];
+        __syncthreads();   // buf and wcount are the next bucket's
+    }
+}
+
 // the distinct keys of bucket j, behind its splitter where present, to
 // off[j] .. of the result
 template <typename K>
@@ -797,14 +860,20 @@ static void sort_pass(const K *in, K *out, uint64_t n, uint32_t lg1, uint32_t lg
                        (const uint32_t *)places, (const uint32_t *)counts, out);
 }
 
+// most_large: buckets of more than RANGE_CAP keys, at most
 template <typename K>
-static void sort_ranges(const K *S, const uint32_t *rstart, const uint32_t *rcount,
+static void sort_ranges(Ctx *c, const K *S, const uint32_t *rstart, const uint32_t *rcount,
                         const uint32_t *present, K *out, uint32_t *kept, uint32_t *overflow,
-                        uint32_t ranges, hipStream_t s) {
+                        uint32_t *nlarge, uint32_t *large, uint32_t most_large, uint32_t ranges,
+                        hipStream_t s) {
     hipLaunchKernelGGL((k_sort_range<K, false>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
-                       rcount, present, out, kept, overflow);
+                       rcount, present, out, kept, overflow, nlarge, large);
     hipLaunchKernelGGL((k_sort_range<K, true>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
-                       rcount, present, out, kept, overflow);
+                       rcount, present, out, kept, overflow, nlarge, large);
+    const uint32_t grid = std::min<uint32_t>(most_large, c->num_cus);
+    if (grid)
+        hipLaunchKernelGGL(k_sort_large<K>, dim3(grid), dim3(LARGE_NT), 0, s, S, rstart, rcount,
+                           present, out, kept, (const uint32_t *)nlarge, (const uint32_t *)large);
 }
 
 template <typename U>
@@ -819,8 +888,8 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
     }
     uint32_t lg = 1;
     while ((n >> lg) >= RANGE_GOAL) lg++;
-    // few enough splitters a pass for their samples (32 and 64 each): a
-    // bucket's size is then the goal's within a factor of 2.4
+    // few enough splitters a pass for their samples: 16 (2^10 of them) or 32 and
+    // more each in the first, 32 (2^9) or more in the second
     const uint32_t lg1 = lg <= PART_LG ? lg : lg > SORT_LG1 + 9 ? lg - 9 : SORT_LG1;
     const uint32_t lg2 = lg - lg1, ranges = 1u << lg;
     const bool wide = n >= (1u << 22);   // queries per lane of a tile: 16, else 4
@@ -828,25 +897,28 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
     const uint32_t tiles1 = (uint32_t)((n + T - 1) / T), tiles2 = lg2 ? tiles1 + (1u << lg1) : 0;
     const uint32_t groups = (tiles1 + PART_GROUP - 1) / PART_GROUP;
     const uint64_t cells = std::max((uint64_t)tiles1 << lg1, (uint64_t)tiles2 << lg2);
-    // words of scratch slot 5: overflow and a count, bstart, tstart, rstart,
-    // rcount, present, kept and the sums of its scan, gsum, counts, places; then
-    // the splitters
+    // words of scratch slot 5: overflow, a count and the number of large buckets,
+    // bstart, tstart, rstart, rcount, present, kept and the sums of its scan, the
+    // large buckets, gsum, counts, places; then the splitters
     const uint64_t B1 = (1ull << lg1) + 1, sums = ranges / SCAN_CHUNK + 3;
-    uint64_t words = 2 + 2 * B1 + (ranges + 1ull) + 3ull * ranges + sums +
+    const uint32_t most_large = (uint32_t)(n / RANGE_CAP);
+    uint64_t words = 3 + 2 * B1 + (ranges + 1ull) + 3ull * ranges + sums + most_large +
                      ((uint64_t)groups << lg1) + 2 * cells;
     words = (words + 1) & ~1ull;
     uint32_t *m = nullptr;
     TL_TRY(scratch(c, 5, words * 4 + (size_t)ranges * sizeof(K), (void **)&m));
-    uint32_t *overflow = m, *count = m + 1, *bstart = m + 2, *tstart = bstart + B1;
+    uint32_t *overflow = m, *count = m + 1, *nlarge = m + 2;
+    uint32_t *bstart = m + 3, *tstart = bstart + B1;
     uint32_t *rstart = lg2 ? tstart + B1 : bstart, *rcount = tstart + B1 + ranges + 1;
     uint32_t *present = rcount + ranges;
-    uint32_t *kept = present + ranges, *ksum = kept + ranges, *gsum = ksum + sums;
+    uint32_t *kept = present + ranges, *ksum = kept + ranges, *large = ksum + sums;
+    uint32_t *gsum = large + most_large;
     uint32_t *counts = gsum + ((uint64_t)groups << lg1), *places = counts + cells;
     K *bound = (K *)(m + words);
     if (n <= RANGE_CAP) {   // one bucket, sorted where it is
         hipLaunchKernelGGL(k_sort_range_of, dim3(1), dim3(1), 0, s, bstart, (uint32_t)n, rcount,
                            present);
-        sort_ranges<K>(keys, bstart, rcount, present, keys, kept, overflow, 1, s);
+        sort_ranges<K>(c, keys, bstart, rcount, present, keys, kept, overflow, nlarge, large, 0, 1, s);
         TL_LAUNCH_CHECK();
         uint32_t u = 0;
         TL_HIP(hipMemcpyAsync(&u, kept, 4, hipMemcpyDeviceToHost, s));
@@ -856,7 +928,7 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
     }
     K *tmp = nullptr;
     TL_TRY(scratch(c, 4, n * sizeof(K), (void **)&tmp));
-    TL_TRY(fill_u32_launch(m, 2, 0, s));
+    TL_TRY(fill_u32_launch(m, 3, 0, s));
     TL_TRY(fill_u32_launch(present, ranges, 0, s));
     if (lg1 <= 8)
         hipLaunchKernelGGL((k_sort_sample<K, false, 8>), dim3(1), dim3(1024), 0, s,
@@ -885,7 +957,8 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
         std::swap(sorted, other);
     }
 #undef TL_SORT_PASS
-    sort_ranges<K>(sorted, rstart, rcount, present, other, kept, overflow, ranges, s);
+    sort_ranges<K>(c, sorted, rstart, rcount, present, other, kept, overflow, nlarge, large,
+                   most_large, ranges, s);
     TL_LAUNCH_CHECK();
     TL_TRY(scan_u32(kept, ranges, ksum, s));
     const uint32_t *sum = ksum + (ranges + SCAN_CHUNK - 1) / SCAN_CHUNK;
