@@ -714,9 +714,7 @@ __global__ __launch_bounds__(256) void k_direct(W *__restrict__ A, const W *__re
 }
 
 template <typename W, int LAYOUT>
-static tl_status direct_launch(Ctx *c, W *A, const SlotShape &sh, bool inverse, hipStream_t s) {
-    W *stash = nullptr;
-    TL_TRY(scratch(c, 0, (size_t)sh.n * sizeof(W), (void **)&stash));
+static tl_status direct_launch(W *A, W *stash, const SlotShape &sh, bool inverse, hipStream_t s) {
     const uint32_t g = (uint32_t)std::min<uint64_t>((sh.n + 255) / 256, 65535);
     hipLaunchKernelGGL(k_copy_strided<W>, dim3(g), dim3(256), 0, s, stash, 1, (const W *)A, 1,
                        (uint64_t)sh.n);
@@ -733,14 +731,20 @@ static tl_status direct_launch(Ctx *c, W *A, const SlotShape &sh, bool inverse, 
     return TL_OK;
 }
 
+// *taken = false (and nothing is enqueued) where the stash is not to be had: the
+// plan makes do with less
 template <typename W>
 static tl_status run_direct(Ctx *c, Layout lay, W *A, uint64_t n, uint64_t b, bool inverse,
-                            hipStream_t s) {
+                            hipStream_t s, bool *taken) {
+    W *stash = nullptr;
+    const tl_status st = scratch(c, 0, (size_t)n * sizeof(W), (void **)&stash);
+    *taken = st == TL_OK;
+    if (st != TL_OK) return st == TL_ENOMEM ? TL_OK : st;
     const uint32_t tl = lay == L_BST ? TILE_BST : lay == L_BTREE ? TILE_BTREE : TILE_VEB;
     const SlotShape sh = slot_shape(tl, n, b, lay == L_VEB);
-    if (tl == TILE_BST) return direct_launch<W, TILE_BST>(c, A, sh, inverse, s);
-    if (tl == TILE_BTREE) return direct_launch<W, TILE_BTREE>(c, A, sh, inverse, s);
-    return direct_launch<W, TILE_VEB>(c, A, sh, inverse, s);
+    if (tl == TILE_BST) return direct_launch<W, TILE_BST>(A, stash, sh, inverse, s);
+    if (tl == TILE_BTREE) return direct_launch<W, TILE_BTREE>(A, stash, sh, inverse, s);
+    return direct_launch<W, TILE_VEB>(A, stash, sh, inverse, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1625,24 +1629,24 @@ static tl_status permute(Layout lay, void *dev_A, uint64_t n, uint64_t b, tl_dty
             return TL_EHIP;
         }
     }
-    if (n <= DIRECT_BYTES / W && !plan_knobs()) {
-        Timer tm;
-        TL_TRY(tm.start(s, ms));
-        if (n > (lay == L_BTREE ? b : 1)) {
-            TL_TRY(W == 4 ? run_direct<uint32_t>(c, lay, (uint32_t *)dev_A, n, b, inverse, s)
-                          : run_direct<uint64_t>(c, lay, (uint64_t *)dev_A, n, b, inverse, s));
-        }
-        return tm.stop();
-    }
-    if (n > DIRECT_BYTES / W && !plan_knobs()) {
+    const bool moves = n > (lay == L_BTREE ? b : 1);
+    if (moves && !plan_knobs()) {
+        const bool direct = n <= DIRECT_BYTES / W;
         Timer tm;
         TL_TRY(tm.start(s, ms));
         bool taken;
-        TL_TRY(W == 4 ? run_slide<uint32_t>(c, lay, (uint32_t *)dev_A, n, b, inverse, s, &taken)
-                      : run_slide<uint64_t>(c, lay, (uint64_t *)dev_A, n, b, inverse, s, &taken));
+        if (W == 4) {
+            uint32_t *A = (uint32_t *)dev_A;
+            TL_TRY(direct ? run_direct<uint32_t>(c, lay, A, n, b, inverse, s, &taken)
+                          : run_slide<uint32_t>(c, lay, A, n, b, inverse, s, &taken));
+        } else {
+            uint64_t *A = (uint64_t *)dev_A;
+            TL_TRY(direct ? run_direct<uint64_t>(c, lay, A, n, b, inverse, s, &taken)
+                          : run_slide<uint64_t>(c, lay, A, n, b, inverse, s, &taken));
+        }
         if (taken) {
             TL_TRY(tm.stop());
-            return ms ? check_err_flag(c, s) : TL_OK;
+            return ms && !direct ? check_err_flag(c, s) : TL_OK;
         }
     }
     Plan pl;
