@@ -1620,7 +1620,8 @@ static tl_status permute(Layout lay, void *dev_A, uint64_t n, uint64_t b, tl_dty
     Ctx *c;
     TL_TRY(get_ctx(&c));
     hipStream_t s = (hipStream_t)stream;
-    if (n > 1) {
+    const bool moves = n > (lay == L_BTREE ? b : 1);
+    if (moves) {
         // a graph would keep the library's scratch, which may move
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         TL_HIP(hipStreamIsCapturing(s, &cap));
@@ -1629,7 +1630,6 @@ static tl_status permute(Layout lay, void *dev_A, uint64_t n, uint64_t b, tl_dty
             return TL_EHIP;
         }
     }
-    const bool moves = n > (lay == L_BTREE ? b : 1);
     if (moves && !plan_knobs()) {
         const bool direct = n <= DIRECT_BYTES / W;
         Timer tm;
