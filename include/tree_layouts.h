@@ -352,7 +352,11 @@ typedef struct {
 } tl_batch_config;
 
 /* Plans every array (the same plans as the single-array permutations) and
- * uploads the task list; cfg may be NULL. */
+ * uploads the task list; cfg may be NULL.  Until tl_batch_destroy() the handle
+ * holds device memory of its own beside the plans' tables: four stashes of the
+ * largest plan's, and for the lookups that are partitioned at most four
+ * workspaces, each of what the largest batch of its branch needs (at most 18
+ * bytes a query of 2^27, and tables; none where query_queue answers them). */
 tl_status tl_batch_create(const tl_batch_item *items, uint32_t count, const tl_batch_config *cfg,
                           void **handle);
 /* Permutes and queries every array of the batch by the planned path: the

@@ -557,9 +557,10 @@ struct Batch {
     size_t q_ticket_at = 0;
     uint64_t q_chunk = 4096;       // queries per queue ticket
     void *d_queue = nullptr;
-    // workspaces of the partitioned lookups, one per branch
+    // workspaces of the partitioned lookups: branch k's is d_qws[qws_at[k],
+    // qws_at[k + 1]), as large as the largest of its arrays needs
     void *d_qws = nullptr;
-    uint64_t qws_stride = 0;
+    uint64_t qws_at[NSUB + 1] = {};
     tl_batch_config cfg{};
     std::vector<BOp> ops;
     std::vector<BTask> tasks;
@@ -862,6 +863,11 @@ static tl_status build_queues(Batch &B) {
     return TL_OK;
 }
 
+// whether item a's lookups go through the query queues
+static bool by_queue(const Batch &B, uint32_t a) {
+    return B.cfg.query_queue && B.d_queue && B.queued[a];
+}
+
 // item a as its lookups see it (its table set is uploaded)
 static TileArray tile_array(const Batch &B, uint32_t a) {
     const tl_batch_item &it = B.items[a];
@@ -965,19 +971,6 @@ static tl_status build_planned(Batch &B, Ctx *c) {
     TL_HIP(hipMalloc(&B.d_pstash, B.stash_stride * Batch::NSUB));
     TL_HIP(hipMalloc((void **)&B.d_pflags, flag_bytes));
     TL_TRY(build_queues(B));
-    // workspaces for the arrays whose lookups are worth partitioning; short of
-    // memory, the batch does without
-    for (uint32_t a = 0; a < B.items.size(); a++) {
-        const tl_batch_item &it = B.items[a];
-        const TileArray ta = tile_array(B, a);
-        if (it.nq && part_wanted(ta, it.dtype, it.Q, it.nq, it.ans, 1.0))
-            B.qws_stride = std::max(B.qws_stride, part_bytes(ta, it.dtype, it.nq));
-    }
-    B.qws_stride = (B.qws_stride + 255) & ~255ull;
-    if (B.qws_stride && hipMalloc(&B.d_qws, B.qws_stride * Batch::NSUB) != hipSuccess) {
-        (void)hipGetLastError();
-        B.d_qws = nullptr;
-    }
     for (int k = 0; k < Batch::NSUB; k++)
         TL_HIP(hipStreamCreateWithFlags(&B.sub[k], hipStreamNonBlocking));
     for (int f = 0; f < 2; f++) {
@@ -1009,6 +1002,25 @@ static tl_status build_planned(Batch &B, Ctx *c) {
     lpt(lc, B.large_branch);
     lpt(qc, B.query_branch);
     lpt(sc, B.small_branch);
+    // workspaces for the arrays whose lookups are worth partitioning and are no
+    // queue's; short of memory, the batch does without
+    uint64_t need[Batch::NSUB] = {};
+    for (uint32_t a = 0; a < B.items.size(); a++) {
+        const tl_batch_item &it = B.items[a];
+        if (!it.nq || by_queue(B, a)) continue;
+        const TileArray ta = tile_array(B, a);
+        if (part_wanted(ta, it.dtype, it.Q, it.nq, it.ans, 1.0)) {
+            uint64_t &most = need[B.query_branch[a]];
+            most = std::max(most, part_bytes(ta, it.dtype, it.nq));
+        }
+    }
+    for (int k = 0; k < Batch::NSUB; k++)
+        B.qws_at[k + 1] = B.qws_at[k] + ((need[k] + 255) & ~255ull);
+    const uint64_t total = B.qws_at[Batch::NSUB];
+    if (total && hipMalloc(&B.d_qws, total) != hipSuccess) {
+        (void)hipGetLastError();
+        B.d_qws = nullptr;
+    }
     return TL_OK;
 }
 
@@ -1355,8 +1367,8 @@ struct BranchWorkspace {
     BranchWorkspace(const Batch &B, int k) : before(query_workspace()) {
         static char none;   // too small for any batch: no workspace of the library's
         Workspace w;
-        w.mem = B.d_qws ? (char *)B.d_qws + k * B.qws_stride : (void *)&none;
-        w.bytes = B.d_qws ? B.qws_stride : 0;
+        w.mem = B.d_qws ? (char *)B.d_qws + B.qws_at[k] : (void *)&none;
+        w.bytes = B.d_qws ? B.qws_at[k + 1] - B.qws_at[k] : 0;
         query_workspace() = w;
     }
     ~BranchWorkspace() { query_workspace() = before; }
@@ -1382,7 +1394,7 @@ static tl_status run_queries(Batch &B, const unsigned char *base, hipStream_t s)
     }
     for (uint32_t a = 0; a < B.items.size(); a++) {
         const tl_batch_item &it = B.items[a];
-        if (!it.nq || (queues && B.queued[a])) continue;
+        if (!it.nq || by_queue(B, a)) continue;
         hipStream_t q_s = B.sub[B.query_branch[a]];
         const BranchWorkspace ws(B, B.query_branch[a]);
         if (it.layout == 0) {
