@@ -84,7 +84,9 @@ tl_status check_err_flag(Ctx *c, hipStream_t s);
 // calls on several streams and host threads are safe.  Null when every
 // workspace is another thread's at the moment, when the stream is being
 // captured (a graph may not keep library memory) or when memory is short: the
-// caller then does without.
+// caller then does without.  The memory stays for the next calls, until
+// leases_release(): idle workspaces go back to the device when scratch() is short
+// of memory.
 constexpr int LEASES = 2;
 struct Lease {
     void *mem = nullptr;
@@ -95,6 +97,7 @@ struct Lease {
 };
 Lease *lease_take(Ctx *c, size_t bytes, hipStream_t s);
 void lease_give(Lease *l, hipStream_t s);
+void leases_release(Ctx *c);
 
 struct Timer {
     hipEvent_t a = nullptr, b = nullptr;

@@ -71,7 +71,14 @@ tl_status scratch(Ctx *c, int slot, size_t bytes, void **out) {
         }
         size_t want = bytes + bytes / 4;
         void *p = nullptr;
-        if (hipMalloc(&p, want) != hipSuccess) {
+        bool ok = hipMalloc(&p, want) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            leases_release(c);
+            want = bytes;
+            ok = hipMalloc(&p, want) == hipSuccess;
+        }
+        if (!ok) {
             (void)hipGetLastError();
             set_error("hipMalloc of " + std::to_string(want) + " scratch bytes failed");
             return TL_ENOMEM;
@@ -110,44 +117,69 @@ tl_status check_err_flag(Ctx *c, hipStream_t s) {
 static std::mutex g_lease_mu;
 static Lease g_lease[64][LEASES];
 
+// while it lives, another thread's stream capture does not see this thread's
+// allocations and waits
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+static void lease_put(Lease *l) {
+    std::lock_guard<std::mutex> lk(g_lease_mu);
+    l->taken = false;
+}
+
+// a taken lease's memory back to the device, once its last user is done
+static bool lease_free(Lease *l) {
+    if (!l->mem) return true;
+    if (hipEventSynchronize(l->done) != hipSuccess || hipFree(l->mem) != hipSuccess) return false;
+    l->mem = nullptr;
+    l->bytes = 0;
+    return true;
+}
+
 Lease *lease_take(Ctx *c, size_t bytes, hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
         return nullptr;
     }
-    // another thread's capture must not see the calls below
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    std::lock_guard<std::mutex> lk(g_lease_mu);
+    RelaxedCapture relaxed;
     Lease *best = nullptr;
-    for (Lease &l : g_lease[c->device])   // this stream's own first, then a large one
-        if (!l.taken && (!best || (l.mem && l.last == s && best->last != s) ||
-                         (best->last != s && l.bytes > best->bytes)))
-            best = &l;
-    bool ok = best != nullptr;
-    if (ok && !best->done)
-        ok = hipEventCreateWithFlags(&best->done, hipEventDisableTiming) == hipSuccess;
+    {
+        std::lock_guard<std::mutex> lk(g_lease_mu);
+        for (Lease &l : g_lease[c->device])   // this stream's own first, then a large one
+            if (!l.taken && (!best || (l.mem && l.last == s && best->last != s) ||
+                             (best->last != s && l.bytes > best->bytes)))
+                best = &l;
+        if (!best) return nullptr;
+        best->taken = true;
+    }
+    // the lease is this call's alone: what can wait, waits without the lock
+    bool ok = true;
+    if (!best->done) ok = hipEventCreateWithFlags(&best->done, hipEventDisableTiming) == hipSuccess;
     if (ok && best->bytes < bytes) {
-        if (best->mem) {
-            ok = hipEventSynchronize(best->done) == hipSuccess && hipFree(best->mem) == hipSuccess;
-            best->mem = nullptr;
-            best->bytes = 0;
+        ok = lease_free(best);
+        // a quarter more, so that somewhat larger batches need no new one
+        for (size_t want : {bytes + bytes / 4, bytes}) {
+            if (!ok || best->mem) break;
+            if (hipMalloc(&best->mem, want) == hipSuccess) {
+                best->bytes = want;
+            } else {
+                best->mem = nullptr;
+                (void)hipGetLastError();
+            }
         }
-        if (ok && hipMalloc(&best->mem, bytes) != hipSuccess) {
-            best->mem = nullptr;
-            ok = false;
-        }
-        if (ok) best->bytes = bytes;
+        ok = ok && best->mem;
     } else if (ok) {
         ok = hipStreamWaitEvent(s, best->done, 0) == hipSuccess;
     }
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) {
         (void)hipGetLastError();
+        lease_put(best);
         return nullptr;
     }
-    best->taken = true;
     best->last = s;
     return best;
 }
@@ -155,8 +187,20 @@ Lease *lease_take(Ctx *c, size_t bytes, hipStream_t s) {
 void lease_give(Lease *l, hipStream_t s) {
     const bool ok = hipEventRecord(l->done, s) == hipSuccess;
     if (!ok) (void)hipStreamSynchronize(s);   // nothing pending then
-    std::lock_guard<std::mutex> lk(g_lease_mu);
-    l->taken = false;
+    lease_put(l);
+}
+
+void leases_release(Ctx *c) {
+    RelaxedCapture relaxed;
+    for (Lease &l : g_lease[c->device]) {
+        {
+            std::lock_guard<std::mutex> lk(g_lease_mu);
+            if (l.taken) continue;
+            l.taken = true;
+        }
+        if (!lease_free(&l)) (void)hipGetLastError();
+        lease_put(&l);
+    }
 }
 
 tl_status Timer::start(hipStream_t s_, float *ms_) {
