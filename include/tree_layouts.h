@@ -16,11 +16,13 @@
  *
  * Scratch (stash, move flags, plan tables, error word) is per device and
  * owned by the library.  Calls that overlap on one device -- on two streams,
- * or from two host threads -- share it and race: serialise them.  The stash of
- * a BST or B-tree permutation grows to its internal keys, 6.25 GiB at most; when
- * that is more, or is not to be had, the permutation makes do with
- * max(2^24, n/16) keys and takes longer.  Arrays of at most 128 MiB of any
- * layout take a stash of their size.
+ * or from two host threads -- share it and race: serialise them.  It is kept for
+ * the next calls until tl_release_scratch().  The stash of a BST or B-tree
+ * permutation grows to its internal keys (a share of n: 0.38 n for 2^30 keys and
+ * b = 16, half to two thirds of n for a BST), 5.25 GiB at most; when that is more,
+ * is not to be had, or TL_PERMUTE_PLAN is set in the environment, the permutation
+ * makes do with max(2^24, n/16) keys and takes longer.  Arrays of at most 128 MiB
+ * of any layout take a stash of their size.
  *
  * Large query batches are partitioned through workspaces of the library's own
  * (at most two per device, each at most 22 bytes a query of 2^27 and tables);
@@ -67,6 +69,13 @@ const char *tl_version(void);
  * if an in-kernel bounded wait gave up since the last report, else TL_OK.
  * No counterpart in the reference, which has no error path. */
 tl_status tl_sync(void *stream);
+
+/* Gives the current device's scratch and idle workspaces back, after waiting for
+ * the device; the next calls allocate anew.  For programs that share the device's
+ * memory and are done with large permutations, sorts or query batches for now.
+ * Not while another host thread is in a call on the device, queries excepted.  No
+ * counterpart in the reference, which allocates within each call. */
+tl_status tl_release_scratch(void);
 
 /* Diagnostic: runs one workgroup whose bounded wait can never be satisfied,
  * bounded at wait_ms (1..60000), and returns what tl_sync returns afterwards

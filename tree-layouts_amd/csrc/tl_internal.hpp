@@ -86,7 +86,7 @@ tl_status check_err_flag(Ctx *c, hipStream_t s);
 // captured (a graph may not keep library memory) or when memory is short: the
 // caller then does without.  The memory stays for the next calls, until
 // leases_release(): idle workspaces go back to the device when scratch() is short
-// of memory.
+// of memory or the program asks (tl_release_scratch).
 constexpr int LEASES = 2;
 struct Lease {
     void *mem = nullptr;

@@ -69,7 +69,9 @@ tl_status scratch(Ctx *c, int slot, size_t bytes, void **out) {
             c->scratch[slot] = nullptr;
             c->scratch_bytes[slot] = 0;
         }
-        size_t want = bytes + bytes / 4;
+        // room for somewhat larger calls, but of a stash of gigabytes (5 GiB at
+        // most) not a quarter
+        size_t want = bytes + std::min(bytes / 4, (size_t)256 << 20);
         void *p = nullptr;
         bool ok = hipMalloc(&p, want) == hipSuccess;
         if (!ok) {
@@ -239,5 +241,17 @@ extern "C" tl_status tl_sync(void *stream) {
     tl::Ctx *c;
     TL_TRY(tl::get_ctx(&c));
     return tl::check_err_flag(c, (hipStream_t)stream);
+}
+extern "C" tl_status tl_release_scratch(void) {
+    tl::Ctx *c;
+    TL_TRY(tl::get_ctx(&c));
+    TL_HIP(hipDeviceSynchronize());
+    tl::leases_release(c);
+    for (int k = 0; k < 6; k++) {
+        if (c->scratch[k]) TL_HIP(hipFree(c->scratch[k]));
+        c->scratch[k] = nullptr;
+        c->scratch_bytes[k] = 0;
+    }
+    return TL_OK;
 }
 extern "C" const char *tl_version(void) { return "tree-layouts-mi355x 0.1 (gfx950)"; }

@@ -118,6 +118,7 @@ _SIGS = {
                        ctypes.c_uint64, ctypes.c_void_p, ctypes.c_uint64,
                        ctypes.POINTER(ctypes.c_uint64)],
     "tl_sync": [ctypes.c_void_p],
+    "tl_release_scratch": [],
     "tl_sort_dedupe": [ctypes.c_void_p, ctypes.c_uint64, ctypes.c_int,
                        ctypes.POINTER(ctypes.c_uint64), ctypes.c_void_p,
                        ctypes.POINTER(ctypes.c_float)],
@@ -257,6 +258,11 @@ def sync(stream=None):
     """Wait for the stream and raise TLError(TL_ETIMEOUT) if an in-kernel
     bounded wait of an untimed call gave up since the last report."""
     _check(lib().tl_sync(_stream(stream)))
+
+
+def release_scratch():
+    """Give the current device's library scratch and idle workspaces back."""
+    _check(lib().tl_release_scratch())
 
 
 def selftest_timeout(wait_ms, stream=None):
