@@ -15,6 +15,7 @@ Prints one JSON line (see the keys below); --gpus N > 1 is rejected because
 this build runs on one GPU.
 """
 import argparse
+import contextlib
 import json
 import os
 import sys
@@ -78,6 +79,20 @@ def event_steps(fn, steps, stream):
     torch.cuda.synchronize()
     per = [evs[i].elapsed_time(evs[i + 1]) for i in range(steps)]
     return evs[0].elapsed_time(evs[-1]), per
+
+
+@contextlib.contextmanager
+def query_path(path):
+    """Large batches by that path (the library reads the variable on each call)"""
+    before = os.environ.get("TL_QUERY_PATH")
+    os.environ["TL_QUERY_PATH"] = path
+    try:
+        yield
+    finally:
+        if before is None:
+            del os.environ["TL_QUERY_PATH"]
+        else:
+            os.environ["TL_QUERY_PATH"] = before
 
 
 def btree_query_bytes(n, b, w, cache_bytes=256 << 20):
@@ -796,30 +811,48 @@ def main():
     del bans
     log(f"[bench] binary search {bs_ms:.3f} ms ({nq / bs_ms / 1e3:.1f} Mq/s) ok={bs_ok}")
 
-    # ---- learned start node: the configuration's model (2^16 leaves) is the
-    # headline; a larger leaf count is reported beside it
-    learned, learned_big = None, None
+    # ---- learned start node against the root: descents of both kinds, since a
+    # batch of this size is otherwise partitioned, whichever entry point it comes
+    # by.  The configuration's model (2^16 leaves) is the headline; a larger leaf
+    # count is reported beside it, and the learned entry point as it is called
+    learned, learned_big, d_ms = None, None, None
     if not args.skip_learned:
-        learned = tl_amd.bench_learned(A, keys, Q, ans, b, args.steps, args.warmup, n,
-                                       num_leaves=1 << args.log2leaves)
-        learned["vs_plain"] = round(q_ms / learned["ms"], 4)
-        log(f"[bench] learned (2^{args.log2leaves} leaves) {learned}")
-        if args.log2leaves_big and args.log2leaves_big != args.log2leaves:
-            learned_big = tl_amd.bench_learned(A, keys, Q, ans, b, args.steps, args.warmup, n,
-                                               num_leaves=1 << args.log2leaves_big)
-            learned_big["vs_plain"] = round(q_ms / learned_big["ms"], 4)
-            log(f"[bench] learned (2^{args.log2leaves_big} leaves) {learned_big}")
+        dans = torch.empty_like(ans)
+        with query_path("plain"):
+            for _ in range(max(1, args.warmup)):
+                tl_amd.query_btree(A, b, Q, dans, kind="u64", timed=False)
+            d_total, _ = event_steps(
+                lambda: tl_amd.query_btree(A, b, Q, dans, kind="u64", timed=False), args.steps,
+                stream)
+            d_ms = d_total / args.steps
+            plain_ok = plain_ok and bool(torch.equal(dans, ans))
+            log(f"[bench] root descents {d_ms:.3f} ms ({nq / d_ms / 1e3:.1f} Mq/s)")
+            learned = tl_amd.bench_learned(A, keys, Q, ans, b, args.steps, args.warmup, n,
+                                           num_leaves=1 << args.log2leaves)
+            learned["vs_plain"] = round(d_ms / learned["ms"], 4)
+            log(f"[bench] learned (2^{args.log2leaves} leaves) {learned}")
+            if args.log2leaves_big and args.log2leaves_big != args.log2leaves:
+                learned_big = tl_amd.bench_learned(A, keys, Q, ans, b, args.steps, args.warmup, n,
+                                                   num_leaves=1 << args.log2leaves_big)
+                learned_big["vs_plain"] = round(d_ms / learned_big["ms"], 4)
+                log(f"[bench] learned (2^{args.log2leaves_big} leaves) {learned_big}")
+        call = tl_amd.bench_learned(A, keys, Q, ans, b, args.steps, args.warmup, n,
+                                    num_leaves=1 << args.log2leaves)
+        learned["call_ms"], learned["call_answers_equal"] = call["ms"], call["answers_equal_plain"]
+        del dans
+        log(f"[bench] learned entry point as called {call['ms']:.3f} ms")
 
     # query roofline: algorithmic bytes of the DRAM-resident levels
     q_all_b, q_dram_b = btree_query_bytes(n, b, 8)
 
     # measured traffic per call (FETCH_SIZE + WRITE_SIZE, committed PMC summary;
     # L2 misses, which include lines the Infinity Cache serves) at this size
-    q_traffic = None
+    q_traffic, d_traffic = None, None
     if n == 1 << 30 and b == 16 and nq == 1 << 27:
         q_traffic = measured_traffic_entry("btree_b16_n2p30_u64_query_traffic.txt")
+        d_traffic = measured_traffic_entry("btree_b16_n2p30_u64_descent_traffic.txt")
 
-    def qroof(ms, tag=None):
+    def qroof(ms, tag=None, q_traffic=q_traffic):
         ach = nq * q_dram_b / (ms * 1e-3) / 1e9
         out = {"bound": "hbm", "bytes_per_query": round(q_dram_b, 1),
                "bytes_per_query_all_levels": round(q_all_b, 1), "achieved": round(ach, 1),
@@ -857,8 +890,10 @@ def main():
                "binary_search": {"ms": round(bs_ms, 4), "Mq_s": round(nq / bs_ms / 1e3, 2),
                                  "answers_ok": bs_ok, "roofline": qroof(bs_ms, "binary")}}
     if learned is not None:
+        queries["descent_ms"] = round(d_ms, 4)
+        queries["descent_roofline"] = qroof(d_ms, "plain", d_traffic)
         queries["learned_roofline"] = qroof(
-            learned["ms"], "learned16" if args.log2leaves == 16 else None)
+            learned["ms"], "learned16" if args.log2leaves == 16 else None, d_traffic)
     if learned_big is not None:
         queries["learned_more_leaves"] = learned_big
     out = {
