@@ -381,27 +381,29 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
 constexpr uint32_t RANGE_NT = 512;
 
 // whether the caller's vEB table set is the one of this layout (the whole
-// workgroup calls it): of every structure the end and, level by level, the L, R
-// and D that the splits give
+// workgroup calls it): of every structure, a wave each, the end and, level by
+// level, the L, R and D that the splits give
 __device__ inline bool veb_tables_match(const TileShape &s) {
     __shared__ uint32_t differs;
     if (threadIdx.x == 0) differs = 0;
     __syncthreads();
-    uint32_t off = 0;
     bool same = true;
-    for (uint32_t j = 0; j < s.ntables; j++) {
-        uint32_t end = s.n;
-        if (j + 1 < s.ntables) {
-            const VebLevel e = s.chain[j];
-            end = off + (1u << e.rd) - 1 + e.nf * ((1u << e.ld) - 1);
-        }
+    auto keys_of = [&](uint32_t j) {   // of structure j, up to the next
+        const VebLevel e = s.chain[j];
+        return (1u << e.rd) - 1 + e.nf * ((1u << e.ld) - 1);
+    };
+    uint32_t off = 0, i = 0;
+    for (uint32_t j = threadIdx.x >> 6; j < s.ntables; j += blockDim.x >> 6) {
+        for (; i < j; i++) off += keys_of(i);
+        const uint32_t end = j + 1 < s.ntables ? off + keys_of(j) : s.n;
         const uint32_t d = 32u - (uint32_t)__clz((int)(s.n - off));
         const uint32_t at = s.tidx ? s.tidx[j] : 0u;
         if (off >= end || (s.idx ? s.idx[j] : s.n) != end || (uint64_t)at + d > s.table_size) {
             same = false;
             break;
         }
-        for (uint32_t t = threadIdx.x + 1; t < d; t += blockDim.x) {
+        const uint32_t t = threadIdx.x & 63;
+        if (t >= 1 && t < d) {
             uint32_t base = 0, levels = d, rd, ld;
             for (;;) {   // down to the tree whose bottom trees start at level t
                 veb_split(levels, rd, ld, s.classic != 0);
@@ -412,7 +414,6 @@ __device__ inline bool veb_tables_match(const TileShape &s) {
             const tl_veb_table e = s.tables[at + t];
             same = same && e.L == (1ull << ld) - 1 && e.R == (1ull << rd) - 1 && e.D == base;
         }
-        off = end;
     }
     if (!same) differs = 1;
     __syncthreads();
@@ -421,22 +422,23 @@ __device__ inline bool veb_tables_match(const TileShape &s) {
 
 // bound[j]: the smallest key of range j; the queue is empty.  queued[1]: a vEB's
 // table set is another layout's than the call's (the answers then follow the
-// tables, as those of every other path do).
+// tables, as those of every other path do); the last workgroup finds that out.
 template <typename W, int LAYOUT>
 __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, TileShape s,
                                                      uint32_t lg, W *__restrict__ bound,
                                                      uint32_t *queued) {
     __shared__ SlotMap<LAYOUT> map;
-    slot_map<LAYOUT>(s, map);
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.x == 0) {
+    if (blockIdx.x + 1 == gridDim.x) {
         bool same = true;
         if constexpr (LAYOUT == TILE_VEB) same = veb_tables_match(s);
-        if (j == 0) {
+        if (threadIdx.x == 0) {
             queued[0] = 0;
             queued[1] = same ? 0u : 1u;
         }
+        return;
     }
+    slot_map<LAYOUT>(s, map);
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j < (1u << lg)) bound[j] = A[slot_of<LAYOUT>(range_first(j, s.n, lg), s, map)];
 }
 
@@ -1243,7 +1245,7 @@ static void part_segment(const PartPlan &p, const TileArray &a, const K *q, uint
     using W = typename std::conditional<sizeof(K) == 4, uint32_t, uint64_t>::type;
     const TileShape sh = tile_shape(a);
     const uint32_t lg = p.lg1 + p.lg2;
-    hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256), dim3(256), 0, s,
+    hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256 + 1), dim3(256), 0, s,
                        (const W *)a.A, sh, lg, (W *)(ws + p.bound), (uint32_t *)(ws + p.queued));
     uint32_t *found = (uint32_t *)(ws + p.found);
     K *first = (K *)ans;   // the answer array holds queries meanwhile
