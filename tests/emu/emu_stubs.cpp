@@ -21,10 +21,12 @@ tl_status get_ctx(Ctx **out) {
     *out = &g;
     return TL_OK;
 }
-// $EMU_SCRATCH_MAX: bytes of a slot beyond which memory is short
+// $EMU_SCRATCH_MAX: bytes of a slot beyond which memory is short ($EMU_SCRATCH_SLOT:
+// of that slot alone)
 tl_status scratch(Ctx *c, int slot, size_t bytes, void **out) {
     const char *e = getenv("EMU_SCRATCH_MAX");
-    if (e && bytes > strtoull(e, nullptr, 10)) return TL_ENOMEM;
+    const char *of = getenv("EMU_SCRATCH_SLOT");
+    if (e && (!of || atoi(of) == slot) && bytes > strtoull(e, nullptr, 10)) return TL_ENOMEM;
     if (c->scratch_bytes[slot] < bytes) {
         free(c->scratch[slot]);
         c->scratch[slot] = malloc(bytes);

@@ -20,3 +20,14 @@ def test_short_scratch(program, layout, width, n, scratch):
                        capture_output=True, text=True, timeout=900, env=env)
     assert r.returncode == 0, r.stderr[-4000:]
     assert r.stderr.count("0 wrong, inverse 0 wrong") == 1, r.stderr[-4000:]
+
+
+def test_short_splitter_tables():
+    """The sort where the splitters' tables are not to be had, but the radix sort's."""
+    subprocess.run(["make", "-C", EMU, "-j4", "_build/emu_sort2"], check=True, capture_output=True)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0", EMU_SCRATCH_SLOT="5",
+               EMU_SCRATCH_MAX="4000")
+    r = subprocess.run([os.path.join(EMU, "_build", "emu_sort2"), "u64", "5000"],
+                       capture_output=True, text=True, timeout=900, env=env)
+    assert r.returncode == 0, r.stderr[-4000:]
+    assert r.stderr.count(", right") == 7, r.stderr[-4000:]

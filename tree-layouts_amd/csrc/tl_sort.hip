@@ -1075,7 +1075,7 @@ extern "C" tl_status tl_sort_dedupe(void *dev_keys, uint64_t n, tl_dtype dtype, 
     hipStream_t s = (hipStream_t)stream;
     Timer tm;
     TL_TRY(tm.start(s, ms));
-    tl_status st;
+    tl_status st = TL_ENOMEM;
     if (n <= SPLIT_MAX_KEYS && !(getenv("TL_SORT_RADIX") && atoi(getenv("TL_SORT_RADIX")) == 1)) {
         switch (dtype) {
         case TL_U32: st = split_sort<uint32_t>(c, (uint32_t *)dev_keys, n, n_out, s); break;
@@ -1083,10 +1083,12 @@ extern "C" tl_status tl_sort_dedupe(void *dev_keys, uint64_t n, tl_dtype dtype, 
         case TL_I32: st = split_sort<int32_t>(c, (int32_t *)dev_keys, n, n_out, s); break;
         default: st = split_sort<int64_t>(c, (int64_t *)dev_keys, n, n_out, s); break;
         }
-    } else if (W == 4) {
+    }
+    // the radix sort's tables are a quarter of the splitters' at 2^29 keys
+    if (st == TL_ENOMEM && W == 4) {
         const uint32_t flip = dtype == TL_I32 ? 0x80000000u : 0u;
         st = sort_dedupe_t<uint32_t>(c, (uint32_t *)dev_keys, n, flip, n_out, s);
-    } else {
+    } else if (st == TL_ENOMEM) {
         const uint64_t flip = dtype == TL_I64 ? 0x8000000000000000ull : 0ull;
         st = sort_dedupe_t<uint64_t>(c, (uint64_t *)dev_keys, n, flip, n_out, s);
     }
