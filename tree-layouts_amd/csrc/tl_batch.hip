@@ -583,7 +583,8 @@ struct Batch {
         if (graph) (void)hipGraphDestroy(graph);
         for (void *p : {(void *)d_ops, (void *)d_tasks, (void *)d_blob, (void *)d_done,
                         (void *)d_ticket, (void *)d_flags, (void *)d_err, d_stash, d_pdata,
-                        d_pstash, (void *)d_pflags, d_wdata, d_wstash, (void *)d_wctr, d_queue, d_qws})
+                        d_pstash, (void *)d_pflags, d_wdata, d_wstash, (void *)d_wctr, d_queue,
+                        d_qws})
             if (p) (void)hipFree(p);
         for (int k = 0; k < NSUB; k++)
             if (sub[k]) (void)hipStreamDestroy(sub[k]);

@@ -757,8 +757,11 @@ static tl_status run_direct(Ctx *c, Layout lay, W *A, uint64_t n, uint64_t b, bo
 // tile stores once the tiles it overwrites, all right of it, have been read,
 // as in chained moves.  The inverse copies the stash's slots there first and
 // sweeps from the left.
-// Bound by memory: 2 n keys are moved, and 2 more for each that is stashed (a
-// BST's n/4 to n/2, few of most B-trees); gathering level by level moved 4 to 9
+// Bound by memory: 2 n keys are moved, and 2 more for each that is stashed: all
+// internal keys, but for the part of the level above the leaves that goes
+// straight.  That is n/2 of a BST with one leaf or all of them, 2 n/3 where the
+// leaves are as many as the keys above that level, and of a B-tree from n / (b + 1)
+// to nearly all (0.38 n at b = 16 and 2^30).  Gathering level by level moved 4 to 9
 // for each key.  Plan -> now, forward: BST of 5*10^8 4-byte keys 6.18 -> 1.14 ms
 // (5.4 TB/s), of 2^30 8-byte keys 7.25 -> 4.87 ms; B-tree b=16 of 2^30 8-byte keys
 // 7.22 -> 4.06 ms (5.9 TB/s); b=8 of 2*10^8 4-byte keys 2.06 -> 0.39 ms, its
@@ -773,7 +776,13 @@ template <typename W, bool INV>
 constexpr uint32_t SLIDE_IT = SLIDE_LANE / (INV ? 8 : sizeof(W));
 template <typename W, bool INV>
 constexpr uint32_t SLIDE_KEYS = SLIDE_NT * SLIDE_IT<W, INV>;
-constexpr uint64_t SLIDE_STASH = 5ull << 30;   // bytes, at most
+// Bytes, at most: a stash is kept for the next call, so it is bounded by what a
+// program that shares the 288 GB can spare (a sixtieth) and not by n.  It serves
+// BSTs up to 1.2 * 10^9 8-byte keys and B-trees of 16 keys a node at every size the
+// slide takes; past it, and where nearly every key is internal (18 keys a node, just
+// over 19^7 of them), the plan takes over: BST of 2^30 keys 4.7 ms, by the plan
+// 7.25; B-tree 4.05, by the plan 7.22.
+constexpr uint64_t SLIDE_STASH = 5ull << 30;
 
 struct SlideShape : SlotShape {
     uint32_t tiles, k1, mul;   // t / k1 = t * mul >> 32 for t < 2^16, k1 < 2^13
@@ -903,7 +912,8 @@ __global__ __launch_bounds__(SLIDE_NT) void k_level_slide(W *__restrict__ A, W *
         // key's slot took three times the vector instructions that the memory
         // leaves time for with 4-byte keys.
         const uint32_t up0 = x0 - tail_i, up_row0 = (uint32_t)__umul64hi(up0, s.recip);
-        const bool leaves = in_rows == SLIDE_KEYS<W, INV>, ups = x0 >= s.tail && m == SLIDE_KEYS<W, INV>;
+        const bool leaves = in_rows == SLIDE_KEYS<W, INV>;
+        const bool ups = x0 >= s.tail && m == SLIDE_KEYS<W, INV>;
         const uint32_t up_slot = s.up + up0 - up_row0;   // the first key's, and the last's at most
         const bool up_in = up_slot + SLIDE_KEYS<W, INV> <= s.up_end, up_out = up_slot >= s.up_end;
         if (leaves || (ups && (up_in || up_out))) {
@@ -935,7 +945,8 @@ __global__ __launch_bounds__(SLIDE_NT) void k_level_slide(W *__restrict__ A, W *
             };
             // slot of the separator of row q
             auto sep_slot = [&](uint32_t q) {
-                return internal_slot<LAYOUT>(leaves ? row0 + q : (up_row0 + q) * s.k1 + s.b, s, map);
+                const uint32_t i = leaves ? row0 + q : (up_row0 + q) * s.k1 + s.b;
+                return internal_slot<LAYOUT>(i, s, map);
             };
             W *mine = A + x0 + tid;
             if constexpr (INV) {

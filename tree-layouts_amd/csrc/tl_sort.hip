@@ -850,7 +850,8 @@ static void sort_pass(const K *in, K *out, uint64_t n, uint32_t lg1, uint32_t lg
         hipLaunchKernelGGL(k_part_sums, dim3(groups), block, 0, s, (const uint32_t *)counts,
                            1u << lg1, tiles, gsum);
         hipLaunchKernelGGL(k_part_starts, dim3(1), block, 0, s, gsum, 1u << lg1, groups,
-                           (uint32_t)(PART_NT * IT), bstart, tstart, lg2 ? (uint32_t *)nullptr : rcount);
+                           (uint32_t)(PART_NT * IT), bstart, tstart,
+                           lg2 ? (uint32_t *)nullptr : rcount);
         hipLaunchKernelGGL(k_part_places, dim3(groups), block, 0, s, (const uint32_t *)counts,
                            1u << lg1, tiles, (const uint32_t *)gsum, (const uint32_t *)bstart,
                            places);
@@ -918,7 +919,8 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
     if (n <= RANGE_CAP) {   // one bucket, sorted where it is
         hipLaunchKernelGGL(k_sort_range_of, dim3(1), dim3(1), 0, s, bstart, (uint32_t)n, rcount,
                            present);
-        sort_ranges<K>(c, keys, bstart, rcount, present, keys, kept, overflow, nlarge, large, 0, 1, s);
+        sort_ranges<K>(c, keys, bstart, rcount, present, keys, kept, overflow, nlarge, large, 0, 1,
+                       s);
         TL_LAUNCH_CHECK();
         uint32_t u = 0;
         TL_HIP(hipMemcpyAsync(&u, kept, 4, hipMemcpyDeviceToHost, s));

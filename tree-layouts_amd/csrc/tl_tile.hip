@@ -250,10 +250,11 @@ constexpr int TILE_QN = 4;     // descents of a lane in flight
 // IT queries per lane, tiles of NT * IT.  Workgroups go round robin to the 8
 // XCDs; each XCD takes one run of consecutive tiles (neighbouring tiles of a
 // batch in key order share their cache lines in one L2).
-template <typename K, int LAYOUT, int IT, typename AT>
+template <typename K, int LAYOUT, int IT>
 __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A, TileShape s,
                                                         const K *__restrict__ Q, uint64_t nq,
-                                                        AT *__restrict__ ans, uint32_t tiles) {
+                                                        uint64_t *__restrict__ ans,
+                                                        uint32_t tiles) {
     constexpr uint32_t T = TILE_NT * IT;
     __shared__ K spl[TILE_BINS];               // heap order, node 1 the root
     __shared__ uint32_t bins[TILE_BINS];
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(TILE_NT) void k_query_tile(const K *__restrict__ A,
                 if ((wave * IT + k0 + k) * 64 + lane < cnt) answers[src[k0 + k]] = res[k];
         }
         __syncthreads();
-        for (uint32_t i = tid; i < cnt; i += TILE_NT) ans[base + i] = (AT)answers[i];
+        for (uint32_t i = tid; i < cnt; i += TILE_NT) ans[base + i] = answers[i];
         __syncthreads();
     }
 }
@@ -447,14 +448,13 @@ __global__ __launch_bounds__(256) void k_part_bounds(const W *__restrict__ A, Ti
 template <typename K, int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_count(
     const K *__restrict__ Q, uint64_t nq, const K *__restrict__ bound, uint32_t lg1, uint32_t lg2,
-    uint32_t tiles,
-    uint32_t *__restrict__ pack, uint32_t *__restrict__ counts) {
+    uint32_t tiles, uint32_t *__restrict__ pack, uint32_t *__restrict__ counts) {
     __shared__ K spl[PART_BINS];
     __shared__ uint32_t cnt[PART_BINS];
     const uint32_t lg = lg1, B = 1u << lg, step = 1u << lg2;
     const uint32_t t = xcd_tile(tiles);
     if (t >= tiles) return;
-    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, 0, 0, nullptr, nullptr);
     K q[IT];
 #pragma unroll
     for (int k = 0; k < IT; k++) {
@@ -486,15 +486,14 @@ __global__ __launch_bounds__(PART_NT) void k_part_count(
     if (threadIdx.x < B) counts[(uint64_t)t * B + threadIdx.x] = cnt[threadIdx.x];
 }
 
-// Every query to its place.  The tile is put in bucket order in LDS first (the places, then the queries, through one
-// buffer), so that a bucket's queries leave as one run: written from where
-// they were read, single queries filled cache lines so slowly that most were
-// written back several times (5.8 GB for 2^27 8-byte queries, where 1.6 GB
+// Every query to its place.  The tile is put in bucket order in LDS first (the
+// places, then the queries, through one buffer), so that a bucket's queries leave
+// as one run: written from where they were read, single queries filled cache
+// lines so slowly that most were written back several times (5.8 GB for 2^27 8-byte queries, where 1.6 GB
 // are written now).
 template <typename K, int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_scatter(
-    const K *__restrict__ Q, uint64_t nq, uint32_t lg1, uint32_t lg2,
-    uint32_t tiles,
+    const K *__restrict__ Q, uint64_t nq, uint32_t lg1, uint32_t tiles,
     const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
     const uint32_t *__restrict__ pack, K *__restrict__ out) {
     __shared__ K stage[PART_NT * IT];
@@ -504,7 +503,7 @@ __global__ __launch_bounds__(PART_NT) void k_part_scatter(
     const uint32_t B = 1u << lg1, tid = threadIdx.x;
     const uint32_t t = xcd_tile(tiles);
     if (t >= tiles) return;
-    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, 0, 0, nullptr, nullptr);
     const uint32_t cnt = (uint32_t)(p.hi - p.lo);
     K q[IT];
     uint32_t pk[IT];
@@ -556,8 +555,7 @@ __global__ __launch_bounds__(PART_NT) void k_part_scatter(
 // answers took 0.72 ms; the vector cache passes on one line a lane).
 template <int IT>
 __global__ __launch_bounds__(PART_NT) void k_part_return(
-    const uint32_t *__restrict__ src, uint64_t nq, uint32_t lg1, uint32_t lg2,
-    uint32_t tiles,
+    const uint32_t *__restrict__ src, uint64_t nq, uint32_t lg1, uint32_t tiles,
     const uint32_t *__restrict__ places, const uint32_t *__restrict__ counts,
     const uint32_t *pack, uint64_t *dst) {
     __shared__ uint32_t stage[PART_NT * IT];
@@ -566,7 +564,7 @@ __global__ __launch_bounds__(PART_NT) void k_part_return(
     const uint32_t B = 1u << lg1, tid = threadIdx.x;
     const uint32_t t = xcd_tile(tiles);
     if (t >= tiles) return;
-    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, lg1, lg2, nullptr, nullptr);
+    const PartTile p = part_tile<false>(t, nq, PART_NT * IT, 0, 0, nullptr, nullptr);
     const uint32_t cnt = (uint32_t)(p.hi - p.lo);
     uint32_t pk[IT];
 #pragma unroll
@@ -611,7 +609,8 @@ __global__ __launch_bounds__(PART_NT) void k_part_return(
 
 template <typename K>
 __device__ inline K key_max() {
-    return (K)-1 > (K)0 ? (K)-1 : (K)(((K)1 << (8 * sizeof(K) - 2)) - 1 + ((K)1 << (8 * sizeof(K) - 2)));
+    const K half = (K)1 << (8 * sizeof(K) - 2);
+    return (K)-1 > (K)0 ? (K)-1 : (K)(half - 1 + half);
 }
 
 // The last pass (the only one of lg1 buckets where !SECOND): a tile's queries in
@@ -900,11 +899,9 @@ struct PartLoc {
 // Registers: at most 64 for a vEB, so that four workgroups share a compute unit
 // (3.25 -> 3.08 ms); the others are faster with what they ask for (5.16 -> 4.85).
 template <typename K, int LAYOUT, bool SECOND, bool REST>
-__global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_answer(const K *__restrict__ A, TileShape s,
-                                                             PartLoc pl, uint32_t units,
-                                                             const K *__restrict__ S,
-                                                             uint32_t *queued, PartShare *queue,
-                                                             uint32_t *__restrict__ out) {
+__global__ __launch_bounds__(RANGE_NT, LAYOUT == TILE_VEB ? 8 : 1) void k_part_answer(
+    const K *__restrict__ A, TileShape s, PartLoc pl, uint32_t units, const K *__restrict__ S,
+    uint32_t *queued, PartShare *queue, uint32_t *__restrict__ out) {
     constexpr uint32_t SPAN = PART_SPAN<SECOND>, RANGES = REST ? 1 : PART_RANGES<SECOND>;
     __shared__ K heap[RANGE_KEYS];
     __shared__ uint32_t sep_slot[LAYOUT == TILE_BTREE ? SEP_SLOTS : 1];
@@ -1088,35 +1085,35 @@ static TileShape tile_shape(const TileArray &a) {
     return s;
 }
 
-template <typename K, int LAYOUT, int IT, typename AT>
-static void tile_launch(Ctx *c, const TileArray &a, const void *q, uint64_t nq, AT *ans,
+template <typename K, int LAYOUT, int IT>
+static void tile_launch(Ctx *c, const TileArray &a, const void *q, uint64_t nq, uint64_t *ans,
                         hipStream_t s) {
     constexpr uint32_t T = TILE_NT * IT;
     const uint32_t tiles = (uint32_t)((nq + T - 1) / T);
     const uint32_t per_cu = 4;
     const uint32_t grid = std::min<uint32_t>((tiles + 7) / 8, c->num_cus * per_cu / 8) * 8;
-    hipLaunchKernelGGL((k_query_tile<K, LAYOUT, IT, AT>), dim3(grid), dim3(TILE_NT), 0, s,
+    hipLaunchKernelGGL((k_query_tile<K, LAYOUT, IT>), dim3(grid), dim3(TILE_NT), 0, s,
                        (const K *)a.A, tile_shape(a), (const K *)q, nq, ans, tiles);
 }
 
-template <typename K, int IT, typename AT>
-static void tile_layout(Ctx *c, const TileArray &a, const void *q, uint64_t nq, AT *ans,
+template <typename K, int IT>
+static void tile_layout(Ctx *c, const TileArray &a, const void *q, uint64_t nq, uint64_t *ans,
                         hipStream_t s) {
     switch (a.layout) {
-    case TILE_BST: tile_launch<K, TILE_BST, IT, AT>(c, a, q, nq, ans, s); break;
-    case TILE_BTREE: tile_launch<K, TILE_BTREE, IT, AT>(c, a, q, nq, ans, s); break;
-    case TILE_VEB: tile_launch<K, TILE_VEB, IT, AT>(c, a, q, nq, ans, s); break;
-    default: tile_launch<K, TILE_SORTED, IT, AT>(c, a, q, nq, ans, s); break;
+    case TILE_BST: tile_launch<K, TILE_BST, IT>(c, a, q, nq, ans, s); break;
+    case TILE_BTREE: tile_launch<K, TILE_BTREE, IT>(c, a, q, nq, ans, s); break;
+    case TILE_VEB: tile_launch<K, TILE_VEB, IT>(c, a, q, nq, ans, s); break;
+    default: tile_launch<K, TILE_SORTED, IT>(c, a, q, nq, ans, s); break;
     }
 }
 
 tl_status tile_query(Ctx *c, const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
                      uint64_t *ans, hipStream_t s) {
     switch (dtype) {
-    case TL_U32: tile_layout<uint32_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
-    case TL_U64: tile_layout<uint64_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
-    case TL_I32: tile_layout<int32_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
-    default: tile_layout<int64_t, 8, uint64_t>(c, a, q, nq, ans, s); break;
+    case TL_U32: tile_layout<uint32_t, 8>(c, a, q, nq, ans, s); break;
+    case TL_U64: tile_layout<uint64_t, 8>(c, a, q, nq, ans, s); break;
+    case TL_I32: tile_layout<int32_t, 8>(c, a, q, nq, ans, s); break;
+    default: tile_layout<int64_t, 8>(c, a, q, nq, ans, s); break;
     }
     TL_LAUNCH_CHECK();
     return TL_OK;
@@ -1205,7 +1202,7 @@ static void part_pass(const PartPlan &p, const K *q, uint64_t nq, char *ws, K *o
                        (uint32_t)(PART_NT * IT), bstart, tstart, (uint32_t *)nullptr);
     hipLaunchKernelGGL(k_part_places, dim3(p.groups), block, 0, s, (const uint32_t *)counts, B1,
                        p.tiles1, (const uint32_t *)gsum, (const uint32_t *)bstart, places);
-    hipLaunchKernelGGL((k_part_scatter<K, IT>), grid, block, 0, s, q, nq, p.lg1, p.lg2, p.tiles1,
+    hipLaunchKernelGGL((k_part_scatter<K, IT>), grid, block, 0, s, q, nq, p.lg1, p.tiles1,
                        (const uint32_t *)places, (const uint32_t *)counts, (const uint32_t *)pack,
                        out);
 }
@@ -1245,8 +1242,9 @@ static void part_segment(const PartPlan &p, const TileArray &a, const K *q, uint
     using W = typename std::conditional<sizeof(K) == 4, uint32_t, uint64_t>::type;
     const TileShape sh = tile_shape(a);
     const uint32_t lg = p.lg1 + p.lg2;
-    hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256 + 1), dim3(256), 0, s,
-                       (const W *)a.A, sh, lg, (W *)(ws + p.bound), (uint32_t *)(ws + p.queued));
+    hipLaunchKernelGGL((k_part_bounds<W, LAYOUT>), dim3(((1u << lg) + 255) / 256 + 1), dim3(256),
+                       0, s, (const W *)a.A, sh, lg, (W *)(ws + p.bound),
+                       (uint32_t *)(ws + p.queued));
     uint32_t *found = (uint32_t *)(ws + p.found);
     K *first = (K *)ans;   // the answer array holds queries meanwhile
     if (!p.lg2) {
@@ -1257,7 +1255,7 @@ static void part_segment(const PartPlan &p, const TileArray &a, const K *q, uint
     K *tiled = sizeof(K) == 4 ? first + nq : (K *)(ws + p.second);
     part_answer<K, LAYOUT, true, IT>(p, a, sh, first, nq, ws, tiled, (uint32_t *)ans, found, s);
     hipLaunchKernelGGL((k_part_return<IT>), dim3((p.tiles1 + 7) / 8 * 8), dim3(PART_NT), 0, s,
-                       (const uint32_t *)found, nq, p.lg1, p.lg2, p.tiles1,
+                       (const uint32_t *)found, nq, p.lg1, p.tiles1,
                        (const uint32_t *)(ws + p.places), (const uint32_t *)(ws + p.counts),
                        (const uint32_t *)(ws + p.pack), ans);
 }
