@@ -24,6 +24,7 @@
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <type_traits>
@@ -1390,11 +1391,20 @@ Workspace &query_workspace() {
     return w;
 }
 
-// $TL_QUERY_PATH: plain, tile or part picks that path wherever it can run
+// $TL_QUERY_PATH: plain, tile or part picks that path wherever it can run.  Without
+// it, a variable that shapes the plain descents keeps those for batches of any size.
 static int forced_path() {
+    static const char *const knobs[] = {"TL_BTREE_WIDE=", "TL_BTREE_IDX64=", "TL_BTREE_QPG=",
+                                        "TL_LEARNED_FUSED=", "TL_VEB_QPL=", "TL_VEB_TOP="};
     const char *e = getenv("TL_QUERY_PATH");
-    if (!e) return -1;
-    return !strcmp(e, "plain") ? 0 : !strcmp(e, "tile") ? 1 : !strcmp(e, "part") ? 2 : -1;
+    if (e && !strcmp(e, "plain")) return 0;
+    if (e && !strcmp(e, "tile")) return 1;
+    if (e && !strcmp(e, "part")) return 2;
+    for (char **v = environ; *v; v++)
+        if (!strncmp(*v, "TL_", 3))
+            for (const char *k : knobs)
+                if (!strncmp(*v, k, strlen(k))) return 0;
+    return -1;
 }
 
 bool part_wanted(const TileArray &a, uint32_t dtype, const void *q, uint64_t nq,
