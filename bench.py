@@ -344,18 +344,8 @@ def config5_arrays(dev, count=4096, queries=True):
                        "ans": ans})
         pristine.append(keys)
         perm_bytes += 2.0 * n * w
-        if lay == "btree":
-            depth = 1
-            cap = 8
-            while cap < n:
-                cap = cap * 9 + 8
-                depth += 1
-            node = 8 * w
-        else:
-            depth = int(np.floor(np.log2(n))) + 1
-            node = w
         if queries:
-            query_bytes += 4.0 * n * (w + 8 + depth * node)
+            query_bytes += lookup_bytes(n, 4 * n, w)
     return arrays, pristine, perm_bytes, query_bytes
 
 
