@@ -272,7 +272,9 @@ tl_status tl_learned_predict(const void *dev_model, const void *dev_keys, uint64
 /* tl_query_btree with the descent started at the deepest node whose subtree
  * holds the model's rank window; queries the window does not settle are
  * answered by the plain root descent.  dev_stats (optional, one uint64,
- * accumulated) counts those fallbacks.  2 <= b <= 64. */
+ * accumulated) counts those fallbacks; without it, a large batch that is cheaper
+ * to partition is answered that way, as tl_query_btree would, and the model is
+ * not read (TL_QUERY_PATH=plain in the environment keeps it).  2 <= b <= 64. */
 tl_status tl_query_btree_learned(const void *dev_A, uint64_t n, uint64_t b, tl_dtype dtype,
                                  const void *dev_model, const void *dev_q, uint64_t nq,
                                  uint64_t *dev_ans, uint64_t *dev_stats, void *stream, float *ms);
