@@ -25,7 +25,7 @@
  * of any layout take a stash of their size.
  *
  * Large query batches are partitioned through workspaces of the library's own
- * (at most two per device, each at most 22 bytes a query of 2^27 and tables);
+ * (at most two per device, each at most 23 bytes a query of 2^27 and tables);
  * queries may overlap with other queries on any stream or host thread.  A
  * query enqueued on a stream that is being captured uses none.
  *
