@@ -739,9 +739,9 @@ __global__ __launch_bounds__(RANGE_NT) void k_sort_range(const K *S,
 }
 
 // The buckets of more than RANGE_CAP keys, LARGE_CAP at most: all their digits in
-// the LDS of a whole compute unit.  A bucket or two of inputs whose average is
+// the LDS of a whole compute unit.  Launched once the host knows that there are any.  A bucket or two of inputs whose average is
 // near the goal: five of eight sets of 2*10^8 8-byte keys had one, and took 24.3 ms
-// by the radix sort of everything where the others took 6.1; now all take 6.1.
+// by the radix sort of everything where the others took 6.1; now 6.2 against 6.05.
 template <typename K>
 __global__ __launch_bounds__(LARGE_NT) void k_sort_large(const K *__restrict__ S,
                                                          const uint32_t *__restrict__ rstart,
@@ -789,8 +789,16 @@ __global__ __launch_bounds__(LARGE_NT) void k_sort_large(const K *__restrict__ S
     }
 }
 
+// counts[j]: what became off[j] when it was scanned
+__global__ __launch_bounds__(256) void k_sort_counts(const uint32_t *__restrict__ off,
+                                                     uint32_t ranges, const uint32_t *sum,
+                                                     uint32_t *__restrict__ counts) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < ranges) counts[j] = (j + 1 < ranges ? off[j + 1] : *sum) - off[j];
+}
+
 // the distinct keys of bucket j, behind its splitter where present, to
-// off[j] .. of the result
+// off[j] .. of the result, unless buckets are yet to be sorted
 template <typename K>
 __global__ __launch_bounds__(256) void k_sort_close(const K *__restrict__ T,
                                                     const uint32_t *__restrict__ rstart,
@@ -799,8 +807,9 @@ __global__ __launch_bounds__(256) void k_sort_close(const K *__restrict__ T,
                                                     const uint32_t *__restrict__ off,
                                                     uint32_t ranges, const uint32_t *sum,
                                                     const uint32_t *__restrict__ overflow,
+                                                    const uint32_t *__restrict__ nlarge,
                                                     K *__restrict__ keys) {
-    if (*overflow) return;
+    if (*overflow || (nlarge && *nlarge)) return;
     const uint32_t j = blockIdx.x, o = off[j], lo = rstart[j], pre = present[j];
     const uint32_t c = (j + 1 < ranges ? off[j + 1] : *sum) - o - pre;
     if (pre && threadIdx.x == 0) keys[o] = bound[j];
@@ -861,20 +870,14 @@ static void sort_pass(const K *in, K *out, uint64_t n, uint32_t lg1, uint32_t lg
                        (const uint32_t *)places, (const uint32_t *)counts, out);
 }
 
-// most_large: buckets of more than RANGE_CAP keys, at most
 template <typename K>
-static void sort_ranges(Ctx *c, const K *S, const uint32_t *rstart, const uint32_t *rcount,
+static void sort_ranges(const K *S, const uint32_t *rstart, const uint32_t *rcount,
                         const uint32_t *present, K *out, uint32_t *kept, uint32_t *overflow,
-                        uint32_t *nlarge, uint32_t *large, uint32_t most_large, uint32_t ranges,
-                        hipStream_t s) {
+                        uint32_t *nlarge, uint32_t *large, uint32_t ranges, hipStream_t s) {
     hipLaunchKernelGGL((k_sort_range<K, false>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
                        rcount, present, out, kept, overflow, nlarge, large);
     hipLaunchKernelGGL((k_sort_range<K, true>), dim3(ranges), dim3(RANGE_NT), 0, s, S, rstart,
                        rcount, present, out, kept, overflow, nlarge, large);
-    const uint32_t grid = std::min<uint32_t>(most_large, c->num_cus);
-    if (grid)
-        hipLaunchKernelGGL(k_sort_large<K>, dim3(grid), dim3(LARGE_NT), 0, s, S, rstart, rcount,
-                           present, out, kept, (const uint32_t *)nlarge, (const uint32_t *)large);
 }
 
 template <typename U>
@@ -898,29 +901,32 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
     const uint32_t tiles1 = (uint32_t)((n + T - 1) / T), tiles2 = lg2 ? tiles1 + (1u << lg1) : 0;
     const uint32_t groups = (tiles1 + PART_GROUP - 1) / PART_GROUP;
     const uint64_t cells = std::max((uint64_t)tiles1 << lg1, (uint64_t)tiles2 << lg2);
-    // words of scratch slot 5: overflow, a count and the number of large buckets,
-    // bstart, tstart, rstart, rcount, present, kept and the sums of its scan, the
-    // large buckets, gsum, counts, places; then the splitters
+    // scratch slot 5, each from a cache line on: overflow, a count and the number of
+    // large buckets; bstart, tstart, rstart, rcount, present, kept and the sums of its
+    // scan, the large buckets, gsum, counts, places; then the splitters
     const uint64_t B1 = (1ull << lg1) + 1, sums = ranges / SCAN_CHUNK + 3;
     const uint32_t most_large = (uint32_t)(n / RANGE_CAP);
-    uint64_t words = 3 + 2 * B1 + (ranges + 1ull) + 3ull * ranges + sums + most_large +
-                     ((uint64_t)groups << lg1) + 2 * cells;
-    words = (words + 1) & ~1ull;
+    uint64_t words = 64;
+    auto take = [&](uint64_t count) {
+        const uint64_t at = words;
+        words += (count + 63) & ~63ull;
+        return at;
+    };
+    const uint64_t at_b = take(B1), at_t = take(B1), at_r = take(ranges + 1ull);
+    const uint64_t at_rc = take(ranges), at_p = take(ranges), at_k = take(ranges);
+    const uint64_t at_ks = take(sums), at_l = take(most_large);
+    const uint64_t at_g = take((uint64_t)groups << lg1), at_c = take(cells), at_pl = take(cells);
     uint32_t *m = nullptr;
     TL_TRY(scratch(c, 5, words * 4 + (size_t)ranges * sizeof(K), (void **)&m));
     uint32_t *overflow = m, *count = m + 1, *nlarge = m + 2;
-    uint32_t *bstart = m + 3, *tstart = bstart + B1;
-    uint32_t *rstart = lg2 ? tstart + B1 : bstart, *rcount = tstart + B1 + ranges + 1;
-    uint32_t *present = rcount + ranges;
-    uint32_t *kept = present + ranges, *ksum = kept + ranges, *large = ksum + sums;
-    uint32_t *gsum = large + most_large;
-    uint32_t *counts = gsum + ((uint64_t)groups << lg1), *places = counts + cells;
+    uint32_t *bstart = m + at_b, *tstart = m + at_t, *rstart = lg2 ? m + at_r : bstart;
+    uint32_t *rcount = m + at_rc, *present = m + at_p, *kept = m + at_k, *ksum = m + at_ks;
+    uint32_t *large = m + at_l, *gsum = m + at_g, *counts = m + at_c, *places = m + at_pl;
     K *bound = (K *)(m + words);
     if (n <= RANGE_CAP) {   // one bucket, sorted where it is
         hipLaunchKernelGGL(k_sort_range_of, dim3(1), dim3(1), 0, s, bstart, (uint32_t)n, rcount,
                            present);
-        sort_ranges<K>(c, keys, bstart, rcount, present, keys, kept, overflow, nlarge, large, 0, 1,
-                       s);
+        sort_ranges<K>(keys, bstart, rcount, present, keys, kept, overflow, nlarge, large, 1, s);
         TL_LAUNCH_CHECK();
         uint32_t u = 0;
         TL_HIP(hipMemcpyAsync(&u, kept, 4, hipMemcpyDeviceToHost, s));
@@ -959,21 +965,41 @@ static tl_status split_sort(Ctx *c, K *keys, uint64_t n, uint64_t *n_out, hipStr
         std::swap(sorted, other);
     }
 #undef TL_SORT_PASS
-    sort_ranges<K>(c, sorted, rstart, rcount, present, other, kept, overflow, nlarge, large,
-                   most_large, ranges, s);
+    sort_ranges<K>(sorted, rstart, rcount, present, other, kept, overflow, nlarge, large, ranges,
+                   s);
     TL_LAUNCH_CHECK();
-    TL_TRY(scan_u32(kept, ranges, ksum, s));
     const uint32_t *sum = ksum + (ranges + SCAN_CHUNK - 1) / SCAN_CHUNK;
     // close the gaps into the buffer that held the partitioned keys
-    hipLaunchKernelGGL(k_sort_close<K>, dim3(ranges), dim3(256), 0, s, (const K *)other,
-                       (const uint32_t *)rstart, (const uint32_t *)present, (const K *)bound,
-                       (const uint32_t *)kept, ranges, sum, (const uint32_t *)overflow, sorted);
-    TL_LAUNCH_CHECK();
-    uint32_t h[3];   // overflow; keys partitioned (and the second pass's gaps); distinct keys
-    TL_HIP(hipMemcpyAsync(&h[0], overflow, 4, hipMemcpyDeviceToHost, s));
+    auto close = [&](uint32_t *off, const uint32_t *unsorted) -> tl_status {
+        TL_TRY(scan_u32(off, ranges, ksum, s));
+        hipLaunchKernelGGL(k_sort_close<K>, dim3(ranges), dim3(256), 0, s, (const K *)other,
+                           (const uint32_t *)rstart, (const uint32_t *)present, (const K *)bound,
+                           (const uint32_t *)off, ranges, sum, (const uint32_t *)overflow,
+                           unsorted, sorted);
+        TL_LAUNCH_CHECK();
+        return TL_OK;
+    };
+    TL_TRY(close(kept, nlarge));
+    // overflow, a count, large buckets; keys partitioned (and the second pass's
+    // gaps); distinct keys
+    uint32_t w[3], h[3];
+    TL_HIP(hipMemcpyAsync(w, overflow, 12, hipMemcpyDeviceToHost, s));
     TL_HIP(hipMemcpyAsync(&h[1], bstart + (1u << lg1), 4, hipMemcpyDeviceToHost, s));
     TL_HIP(hipMemcpyAsync(&h[2], sum, 4, hipMemcpyDeviceToHost, s));
     TL_HIP(hipStreamSynchronize(s));
+    h[0] = w[0];
+    if (!h[0] && w[2]) {
+        hipLaunchKernelGGL(k_sort_counts, dim3((ranges + 255) / 256), dim3(256), 0, s,
+                           (const uint32_t *)kept, ranges, sum, counts);
+        hipLaunchKernelGGL(k_sort_large<K>, dim3(std::min<uint32_t>(w[2], c->num_cus)),
+                           dim3(LARGE_NT), 0, s, (const K *)sorted, (const uint32_t *)rstart,
+                           (const uint32_t *)rcount, (const uint32_t *)present, other, counts,
+                           (const uint32_t *)nlarge, (const uint32_t *)large);
+        TL_LAUNCH_CHECK();
+        TL_TRY(close(counts, nullptr));
+        TL_HIP(hipMemcpyAsync(&h[2], sum, 4, hipMemcpyDeviceToHost, s));
+        TL_HIP(hipStreamSynchronize(s));
+    }
     const uint64_t have = h[0] ? h[1] : h[2];
     if (sorted != keys && have)
         TL_HIP(hipMemcpyAsync(keys, sorted, have * sizeof(K), hipMemcpyDeviceToDevice, s));
