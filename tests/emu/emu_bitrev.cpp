@@ -2,7 +2,7 @@
 // bit-reversal tiles of tl_kernels.hpp in all their forms (plain; phase one
 // absorbing row ends; the levels shifted in place / unfolded) and the level
 // heads copy, built for the host over the HIP shim and run one workgroup at a
-// time with every lane a thread, on exactly sized host buffers under
+// time with every lane a fiber, on exactly sized host buffers under
 // AddressSanitizer.
 //
 // The forward sequence (phase one in place, the level heads and the leaf to

@@ -1,7 +1,7 @@
 // Serial CPU emulation of the uneven batch's single persistent launch (k_batch):
 // the product's tl_batch.hip, compiled for the host over a shim of the HIP
 // surface (tests/emu/hip/hip_runtime.h), runs its kernels one workgroup at a
-// time with every lane a thread, on host memory, under AddressSanitizer.  This
+// time with every lane a fiber, on host memory, under AddressSanitizer.  This
 // driver builds a mixed batch, runs the persistent launch through
 // tl_batch_run, and checks every array against the oracle.
 #include "hip/hip_runtime.h"

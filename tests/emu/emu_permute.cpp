@@ -1,6 +1,6 @@
 // CPU emulation of the single-array permutations: the product's
 // tl_permute.hip, compiled for the host over the HIP shim, runs every plan
-// launch one workgroup at a time with every lane a thread, on exactly sized
+// launch one workgroup at a time with every lane a fiber, on exactly sized
 // host buffers under AddressSanitizer.  Chained moves take their tickets in
 // order (one workgroup runs to the end before the next starts), so every
 // wait is already satisfied when it is reached.  Each case permutes 0..n-1,

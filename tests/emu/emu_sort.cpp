@@ -1,5 +1,5 @@
 // CPU emulation of the sort: tl_sort.hip built for the host over the HIP shim,
-// one workgroup at a time with every lane a thread, under AddressSanitizer.
+// one workgroup at a time with every lane a fiber, under AddressSanitizer.
 // Every result is compared with std::sort and std::unique, over inputs that
 // reach its paths: wide and narrow ranges, keys that repeat often, one key
 // alone, keys in order and in reverse, and crowds with outliers.  Arguments: key

@@ -1,5 +1,5 @@
 // CPU emulation of the tile-sorted lookups: tl_tile.hip built for the host
-// over the HIP shim, one workgroup at a time with every lane a thread, on
+// over the HIP shim, one workgroup at a time with every lane a fiber, on
 // exactly sized buffers under AddressSanitizer.  Every answer is compared with
 // the CPU oracle's search (the reference's visiting order), with distinct
 // keys and with keys that repeat.  Arguments: layout (bst, btree, mveb, veb,

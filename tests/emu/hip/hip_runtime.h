@@ -1,5 +1,5 @@
 // Host shim of the HIP device and runtime surface that tl_batch.hip uses, for a
-// serial CPU emulation of its kernels (lanes = threads, one workgroup at a time).
+// serial CPU emulation of its kernels (lanes = fibers, one workgroup at a time).
 #pragma once
 #include <stdint.h>
 #include <stddef.h>
@@ -118,7 +118,7 @@ inline hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorU
 inline hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 inline hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 
-// kernel launch: every workgroup in turn, its lanes as threads
+// kernel launch: every workgroup in turn, its lanes as fibers
 #include <functional>
 void emu_run_block(dim3 grid, dim3 block, dim3 bid, size_t smem, const std::function<void()> &body);
 template <class... P, class... A>
